@@ -29,7 +29,8 @@ METRIC = "MLUPS & %HBM peak: FP64 vs FP32/FP16-store at stated error; adjoint/fw
 
 
 # sources of the step kernel: a traffic figure measured on other sources is stale
-STEP_KERNEL_SOURCES = ("step_fused.hip", "fused_common.h", "device_common.h", "dugks_internal.h", "lattice.h")
+STEP_KERNEL_SOURCES = ("step_fused.hip", "step_kernel.h", "step_common.h",
+                       "fused_common.h", "device_common.h", "dugks_internal.h", "lattice.h")
 
 
 def step_kernel_hash():

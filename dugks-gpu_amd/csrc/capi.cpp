@@ -294,9 +294,7 @@ hipError_t build_params(Ctx& c) {
   P.famb_dev = c.famb_dev;
   c.red_len = reduction_scratch_doubles() + 64;
   if ((e = c.alloc((void**)&c.red, c.red_len * sizeof(double))) != hipSuccess) return e;
-  // per-block flow sums of the fused kernel: at most (nx/32)(ny/8) blocks
-  // per z-chunk, z-chunks of at least 1 plane
-  c.flow_partial_len = (size_t)(s.n[0] / 32 + 1) * (s.n[1] / 8 + 1) * (s.n[2] + 1);
+  c.flow_partial_len = (size_t)step_fused_blocks(s, c.precision);
   if ((e = c.alloc((void**)&c.flow_partial, c.flow_partial_len * sizeof(double))) != hipSuccess) return e;
   return hipSuccess;
 }

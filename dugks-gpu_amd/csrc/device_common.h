@@ -131,13 +131,6 @@ struct StateBuf<NeqHalf> {
   __amdgpu_buffer_rsrc_t r;
   __device__ __forceinline__ StateBuf(const NeqHalf* p, unsigned bytes)
       : r(__builtin_amdgcn_make_buffer_rsrc(const_cast<NeqHalf*>(p), 0, (int)bytes, 0x00020000)) {}
-  __device__ __forceinline__ __half raw(unsigned vb, unsigned sb) const {
-    return __ushort_as_half(__builtin_amdgcn_raw_buffer_load_b16(r, (int)vb, (int)sb, 0));
-  }
-  // the 16 bits zero-extended to 32 (see RawCell)
-  __device__ __forceinline__ unsigned raw32(unsigned vb, unsigned sb) const {
-    return (unsigned)__builtin_amdgcn_raw_buffer_load_b16(r, (int)vb, (int)sb, 0);
-  }
   __device__ __forceinline__ void put(__half v, unsigned vb, unsigned sb) const {
     __builtin_amdgcn_raw_buffer_store_b16(__half_as_ushort(v), r, (int)vb, (int)sb, 0);
   }
@@ -480,21 +473,6 @@ struct NeqEq {
   }
 };
 
-// Centre stage in shifted populations: hb_i = f-bar+_i - w_i from h_i, the
-// cell's drho = rho - 1 and momentum velocity u0 (with FP16 non-equilibrium
-// storage the stored ones, which the decoded populations match to the FP16
-// rounding of their non-equilibrium parts).
-template <class Real>
-__device__ __forceinline__ void centre_fbar_shift(const Real (&h)[Q], Real drho, const Real (&u0)[3],
-                                                  const Real F[3], Real hdt, Real bw0, Real bw2, Real (&hb)[Q]) {
-  const EqShift<Real> eq(ExactProducts{}, drho, u0[0] + hdt * F[0], u0[1] + hdt * F[1], u0[2] + hdt * F[2], F, bw2,
-                         bw0);
-  static_for<Q>([&](auto I) {
-    constexpr int ip = decltype(I)::value;
-    hb[ip] = eq.template relax<ip>(-bw2, h[ip], cdot<ip>(F[0], F[1], F[2]));
-  });
-}
-
 // Centre-stage f-bar+ of one cell (calc_fb1 of the reference, src/dugks.cu:1131-1196):
 //   rho = sum f, u = j/rho + h F, feq_i(rho, u),
 //   fb_i = bw1 f_i + (bw2 + bw0 (c_i - u).F / RT) feq_i.
@@ -558,8 +536,7 @@ __device__ __forceinline__ void cell_moments(const Real (&ff)[Q], Real& rho, Rea
   });
 }
 
-// rho and the momentum velocity u0 = j / rho of one cell; with `shifted`
-// the populations are h = f - w and rho_out is sum h = rho - 1.  FP32
+// rho and the momentum velocity u0 = j / rho of one cell.  FP32
 // populations are summed in FP64 and the results rounded to FP32 once: the
 // rounding of FP32 sums (about 1e-8 of j, a quarter of the velocity a
 // typical body force adds per step) repeats from step to step in a slowly
@@ -567,7 +544,7 @@ __device__ __forceinline__ void cell_moments(const Real (&ff)[Q], Real& rho, Rea
 // Re_tau = 180 channel moves the rms-velocity profiles by 1e-3 of their
 // size (FP64 sums: 2e-4).
 template <class Real>
-__device__ __forceinline__ void cell_rho_u(const Real (&ff)[Q], Real& rho_out, Real (&u0)[3], bool shifted = false) {
+__device__ __forceinline__ void cell_rho_u(const Real (&ff)[Q], Real& rho_out, Real (&u0)[3]) {
   if constexpr (sizeof(Real) == 4) {
     double r, j[3];
     static_for<Q>([&](auto I) {
@@ -579,17 +556,16 @@ __device__ __forceinline__ void cell_rho_u(const Real (&ff)[Q], Real& rho_out, R
       if constexpr (ip == 5) j[2] = v; else if constexpr (CZ[ip] != 0) j[2] += CZ[ip] > 0 ? v : -v;
     });
     rho_out = (Real)r;
-    const double rho = shifted ? 1.0 + r : r;
     // 1/rho: the hardware reciprocal and one Newton step (error ~1e-14)
-    double x = __builtin_amdgcn_rcp(rho);
-    x = __builtin_fma(x, __builtin_fma(-rho, x, 1.0), x);
+    double x = __builtin_amdgcn_rcp(r);
+    x = __builtin_fma(x, __builtin_fma(-r, x, 1.0), x);
     u0[0] = (Real)(j[0] * x);
     u0[1] = (Real)(j[1] * x);
     u0[2] = (Real)(j[2] * x);
   } else {
     Real j[3];
     cell_moments<Real>(ff, rho_out, j);
-    moment_velocity<Real>(shifted ? Real(1) + rho_out : rho_out, j, u0);
+    moment_velocity<Real>(rho_out, j, u0);
   }
 }
 
@@ -739,135 +715,11 @@ struct RawCell {
     });
     cell_rho_u<Real>(ff, rho, u0);
   }
-  // shifted populations h = f - w (see EqShift), drho = sum h and the
-  // momentum velocity u0 = j / (1 + drho); f - w is exact for FP32 f within
-  // a factor 2 of w
-  __device__ __forceinline__ void decode_shift(const KParams& P, Real (&h)[Q], Real& drho, Real (&u0)[3]) const {
-    static_for<Q>([&](auto I) {
-      constexpr int ip = decltype(I)::value;
-      if constexpr (std::is_same<Store, __half>::value)
-        h[ip] = Real(wgt(ip)) * ((Real)__half2float(__ushort_as_half((unsigned short)v[ip])) + (P.rho0f - 1.0f));
-      else
-        h[ip] = (Real)v[ip] - Real(wgt(ip));
-    });
-    cell_rho_u<Real>(h, drho, u0, true);
-  }
   // the rho and j only (FP32 storage path of the adjoint-face pass)
   __device__ __forceinline__ void moments(const Real (&ff)[Q], Real& rho, Real (&j)[3]) const {
     cell_moments<Real>(ff, rho, j);
   }
 };
-template <class Real>
-struct RawCell<Real, NeqHalf> {
-  unsigned v[Q];  // FP16 bits, zero-extended (see RawSlot)
-  float m[4];
-  __device__ __forceinline__ void load(const StateBuf<NeqHalf>& b, unsigned cell, unsigned N) {
-    const unsigned vf = cell * 4u, vh = cell * 2u;
-    for (int q = 0; q < 4; q++) m[q] = b.rawf(vf, q * 4u * N);
-    static_for<Q>([&](auto I) {
-      constexpr int ip = decltype(I)::value;
-      v[ip] = b.raw32(vh, 16u * N + ip * 2u * N);
-    });
-  }
-  // as RawCell::settle
-  __device__ __forceinline__ void settle() {
-    for (int q = 0; q < 4; q++) asm volatile("" : "+v"(m[q]));
-    static_for<Q>([&](auto I) {
-      constexpr int ip = decltype(I)::value;
-      asm volatile("" : "+v"(v[ip]));
-    });
-  }
-  __device__ __forceinline__ void decode(const KParams& P, Real (&ff)[Q], Real& rho, Real (&u0)[3]) const {
-    rho = Real(1) + (Real)m[0];
-    u0[0] = (Real)m[1];
-    u0[1] = (Real)m[2];
-    u0[2] = (Real)m[3];
-    __half s[Q];
-    static_for<Q>([&](auto I) {
-      constexpr int ip = decltype(I)::value;
-      s[ip] = __ushort_as_half((unsigned short)v[ip]);
-    });
-    neq_decode<Real>(rho, u0, s, ff);
-  }
-  // shifted populations h_i = f_i - w_i = w_i rho eps_i + w_i drho + w_i s_i / kNeqScale
-  // straight from the stored drho, u and s (see EqShift), with the
-  // per-class products w rho and w drho rounded once (NeqEq; as in the
-  // centre stage, products rounded twice bias the flow's dissipation.  On
-  // the Re = 1600 Taylor-Green vortex, against FP64: this decode and the
-  // centre stage's EqShift products both rounded twice, 0.67 % less
-  // dissipation; only EqShift's once, 0.54 % more; only the decode's once,
-  // 1.2 % less; both once, 0.01 %)
-  __device__ __forceinline__ void decode_shift(const KParams& P, Real (&h)[Q], Real& drho, Real (&u0)[3]) const {
-    drho = (Real)m[0];
-    u0[0] = (Real)m[1];
-    u0[1] = (Real)m[2];
-    u0[2] = (Real)m[3];
-    const NeqEq<Real> eq(drho, u0);
-    static_for<Q>([&](auto I) {
-      constexpr int ip = decltype(I)::value;
-      const Real sv = (Real)__half2float(__ushort_as_half((unsigned short)v[ip]));
-      h[ip] = eq.template shift_of<ip>(sv);
-    });
-  }
-};
-
-// Stores population ip of a cell given in shifted form h = f - w (FP32 f =
-// h + w, or the FP16 deviation h / w + 1 - rho0); not FP16 non-equilibrium
-// storage, which encodes whole cells (store_neq_shift).
-template <class Real, class Store>
-__device__ __forceinline__ void st_state_shift(const StateBuf<Store>& b, unsigned vb, unsigned sb, Real h,
-                                               const KParams& P, int ip) {
-  if constexpr (std::is_same<Store, __half>::value)
-    b.put(__float2half((float)h * (float)(1.0 / wgt(ip)) + (1.0f - P.rho0f)), vb, sb);
-  else
-    b.put((Store)(h + Real(wgt(ip))), vb, sb);
-}
-
-// FP16 non-equilibrium encoding of a cell given in shifted form: drho = sum
-// h, u0 = j / (1 + drho), s_i = (h_i / w_i - drho - rho eps_i) kNeqScale.
-// Returns drho and u0.
-template <class Real>
-__device__ __forceinline__ void store_neq_shift(const StateBuf<NeqHalf>& b, unsigned cell, unsigned N,
-                                                const Real (&h)[Q], Real& drho, Real (&u0)[3]) {
-  cell_rho_u<Real>(h, drho, u0, true);
-  const NeqEq<Real> eq(drho, u0);
-  const unsigned vf = cell * 4u, vh = cell * 2u;
-  b.putf((float)drho, vf, 0);
-  for (int q = 0; q < 3; q++) b.putf((float)u0[q], vf, (q + 1) * 4u * N);
-  static_for<Q>([&](auto I) {
-    constexpr int ip = decltype(I)::value;
-    const Real n = (h[ip] - eq.template eq<ip>()) * Real((double)kNeqScale / wgt(ip));
-    b.put(__float2half((float)n), vh, 16u * N + ip * 2u * N);
-  });
-}
-
-// Stores the new f of a cell through a StateBuf; returns its rho and momentum
-// velocity u0 (needed for the encoding, and by the flow-rate partials) when
-// `want_u` or the storage needs them.
-template <class Real, class Store>
-__device__ __forceinline__ void store_raw_cell(const StateBuf<Store>& b, unsigned cell, unsigned N,
-                                               const KParams& P, const Real (&ff)[Q], bool want_u, Real& rho,
-                                               Real (&u0)[3]) {
-  if constexpr (std::is_same<Store, NeqHalf>::value) {
-    __half s[Q];
-    neq_encode<Real>(ff, rho, u0, s);
-    const unsigned vf = cell * 4u, vh = cell * 2u;
-    b.putf((float)(rho - Real(1)), vf, 0);
-    for (int q = 0; q < 3; q++) b.putf((float)u0[q], vf, (q + 1) * 4u * N);
-    static_for<Q>([&](auto I) {
-      constexpr int ip = decltype(I)::value;
-      b.put(s[ip], vh, 16u * N + ip * 2u * N);
-    });
-  } else {
-    const unsigned vb = cell * (unsigned)sizeof(Store), Nb = N * (unsigned)sizeof(Store);
-    static_for<Q>([&](auto I) {
-      constexpr int ip = decltype(I)::value;
-      st_state<Real, Store>(b, vb, ip * Nb, ff[ip], P, ip);
-    });
-    if (want_u) cell_rho_u<Real>(ff, rho, u0);
-  }
-}
-
 // Adjoint of the equilibrium-with-force term (used by the adjoint of the
 // centre stage and of the face collision).
 // G = sum_i lam_i (B + C T_i) feq_i(rho, u), T_i = 3 (c_i - u).F,

@@ -54,6 +54,8 @@ struct Ctx;
 hipError_t launch_step_twopass(Ctx& c, const void* fin, void* fout);
 hipError_t launch_fbar_ghosts(Ctx& c, const void* fin, void* fbx);
 hipError_t launch_step_fused(Ctx& c, const void* fin, void* fout, bool* handled);
+// workgroups of that launch (each leaves one bulk-velocity partial)
+long long step_fused_blocks(const Setup& s, int precision);
 // Adjoint-face pass of the fused kernel (see adjoint.hip); handled = false
 // when the fused kernel does not cover the configuration.  Face record
 // formats: kFacesFull, the 19 reconstructed-value cotangents per face, lam'
@@ -222,8 +224,7 @@ struct Ctx {
   bool timing = false;
   std::vector<float> kernel_ms;
   int launches_per_step = 0;
-  // fused kernel: z-chunk length and the per-block flow-rate partial sums
-  int fused_tz = 0;
+  // fused kernel: the per-block flow-rate partial sums
   double* flow_partial = nullptr;
   size_t flow_partial_len = 0;
   // the step kernels leave the flow-rate controller alone (the adjoint's

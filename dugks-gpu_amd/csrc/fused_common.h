@@ -1,4 +1,4 @@
-// Building blocks of the fused step kernel and its adjoint-face mode:
+// Building blocks of the fused step kernel and the adjoint-face pass:
 // per-axis direction sets, f-bar+ of a (possibly wall-ghost) column, and the
 // face reconstruction record with its collision and the transpose of that
 // collision.  Included inside namespace dugks { namespace { ... } } of the
@@ -34,42 +34,35 @@ __device__ __forceinline__ void ambient_force(const KParams& P, Real F[3]) {
   F[2] = (Real)P.famb_dev[2];
 }
 
-// f-bar+ of interior cell (i, j, k) (0-based); SHIFT: in shifted form
-// f-bar+ - w (see EqShift).
-template <class Real, class Store, bool SHIFT>
+// f-bar+ of interior cell (i, j, k) (0-based).
+template <class Real, class Store>
 __device__ __forceinline__ void fbar_cell(const KParams& P, const StateBuf<Store>& f, unsigned Nb, int i, int j,
                                           int k, const Real Famb[3], Real (&fb)[Q]) {
   const unsigned c = ((unsigned)k * P.n[1] + j) * P.n[0] + i;
   RawCell<Real, Store> raw;
   raw.load(f, c, (unsigned)P.N);
   Real ff[Q], rho, u0[3];
-  if constexpr (SHIFT)
-    raw.decode_shift(P, ff, rho, u0);
-  else
-    raw.decode(P, ff, rho, u0);
+  raw.decode(P, ff, rho, u0);
   Real F[3] = {Famb[0], Famb[1], Famb[2]};
   if (P.fcell) {
     F[0] += (Real)P.fcell[c];
     F[1] += (Real)P.fcell[P.N + c];
     F[2] += (Real)P.fcell[2 * P.N + c];
   }
-  if constexpr (SHIFT)
-    centre_fbar_shift<Real>(ff, rho, u0, F, (Real)P.hdt, (Real)P.bw0, (Real)P.bw2, fb);
-  else
-    centre_fbar<Real>(ff, rho, u0, F, (Real)P.hdt, (Real)P.bw0, (Real)P.bw2, fb);
+  centre_fbar<Real>(ff, rho, u0, F, (Real)P.hdt, (Real)P.bw0, (Real)P.bw2, fb);
 }
 
 // f-bar+ of a column that may be a wall ghost in x and/or y: the ghost value
 // is the linear extrapolation q f(1) + (1-q) f(2) from the wall side.
 // gi, gj are 0-based; a wall ghost is -1 or n; periodic indices are wrapped
-// by the caller.  SHIFT: in shifted form (the extrapolation weights sum to 1).
-template <class Real, class Store, bool SHIFT>
+// by the caller.
+template <class Real, class Store>
 __device__ void fbar_column(const KParams& P, const StateBuf<Store>& f, unsigned Nb, int gi, int gj, int kz,
                             const Real Famb[3], Real (&fb)[Q]) {
   const bool gx = gi < 0 || gi >= P.n[0];
   const bool gy = gj < 0 || gj >= P.n[1];
   if (!gx && !gy) {
-    fbar_cell<Real, Store, SHIFT>(P, f, Nb, gi, gj, kz, Famb, fb);
+    fbar_cell<Real, Store>(P, f, Nb, gi, gj, kz, Famb, fb);
     return;
   }
   // the two columns (and weights) of the extrapolation along each ghost axis;
@@ -101,7 +94,7 @@ __device__ void fbar_column(const KParams& P, const StateBuf<Store>& f, unsigned
       // k = 0: the second column (x1 or y1), k = 1: the first
       const int ci = gx ? (k ? x0 : x1) : gi, cj = gy ? (k ? y0 : y1) : gj;
       Real t[Q];
-      fbar_cell<Real, Store, SHIFT>(P, f, Nb, ci, cj, kz, Famb, t);
+      fbar_cell<Real, Store>(P, f, Nb, ci, cj, kz, Famb, t);
       static_for<Q>([&](auto I) {
         constexpr int ip = decltype(I)::value;
         fb[ip] = k ? fma_rn(q, t[ip] - fb[ip], fb[ip]) : t[ip];
@@ -115,7 +108,7 @@ __device__ void fbar_column(const KParams& P, const StateBuf<Store>& f, unsigned
     const int a = k & 1, b = k >> 1;
     const Real w = (a ? Real(1) - qx : qx) * (b ? Real(1) - qy : qy);
     Real t[Q];
-    fbar_cell<Real, Store, SHIFT>(P, f, Nb, a ? x1 : x0, b ? y1 : y0, kz, Famb, t);
+    fbar_cell<Real, Store>(P, f, Nb, a ? x1 : x0, b ? y1 : y0, kz, Famb, t);
     static_for<Q>([&](auto I) {
       constexpr int ip = decltype(I)::value;
       fb[ip] = first ? w * t[ip] : fb[ip] + w * t[ip];
@@ -279,36 +272,6 @@ struct Face {
         if constexpr (cv(A, ip) < 0) cross[k] = cross[cross_index<A>(OPP[ip])];
       });
     }
-  }
-  // Face collision (f2ruvwh + feq_s, src/dugks.cu:675-709, 1201-1207):
-  // rho = sum fbar, u = j/rho + (h/2) F, out = fw1 fbar + (fw2 + fw0 (c-u).F/RT) feq
-  // for the crossing populations.
-  __device__ __forceinline__ void collide(const Real F[3], Real hdt, Real fw0, Real fw1, Real fw2,
-                                          Real (&out)[10]) {
-    moments();
-    const Real inv = rcp_real(rho);
-    const Real hh = Real(0.5) * hdt;
-    const EqTerm<Real> eq(rho, j[0] * inv + hh * F[0], j[1] * inv + hh * F[1], j[2] * inv + hh * F[2], F, fw2,
-                          fw0);
-    static_for<10>([&](auto K) {
-      constexpr int k = decltype(K)::value;
-      constexpr int ip = dirs<A>(k);
-      out[k] = eq.template relax<ip>(fw1, cross[k], cdot<ip>(F[0], F[1], F[2]));
-    });
-  }
-  // collide in shifted populations (the face holds f-bar - w, its rho the
-  // sum of those, drho): out - w for the crossing populations (see EqShift)
-  __device__ __forceinline__ void collide_shift(const Real F[3], Real hdt, Real fw0, Real fw2, Real (&out)[10]) {
-    moments();
-    const Real inv = rcp_real(Real(1) + rho);
-    const Real hh = Real(0.5) * hdt;
-    const EqShift<Real> eq(rho, j[0] * inv + hh * F[0], j[1] * inv + hh * F[1], j[2] * inv + hh * F[2], F, fw2,
-                           fw0);
-    static_for<10>([&](auto K) {
-      constexpr int k = decltype(K)::value;
-      constexpr int ip = dirs<A>(k);
-      out[k] = eq.template relax<ip>(-fw2, cross[k], cdot<ip>(F[0], F[1], F[2]));
-    });
   }
   // The transposed collision up to its equilibrium coefficients: the
   // cotangent of reconstructed value p is fw1 mu_p + Ac + B.c_p (mu_p = 0

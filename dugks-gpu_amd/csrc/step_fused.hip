@@ -1,16 +1,18 @@
-// Fused DUGKS step: one kernel per time step, f read once and written once.
+// Fused DUGKS step: one kernel per time step, f read once and written once;
+// and the adjoint-face pass.
 //
-// Decomposition.  A workgroup owns a TX x TY tile of (x, y) columns and
-// marches along z over a chunk of TZ planes.  Its threads are TY + 2 rows of
-// TX lanes (the interior rows and the two y-halo rows) plus one wave for the
-// two x-halo columns (corners included); every thread owns one column.  Each
-// plane it:
-//   - loads f of its column at plane p+1 and computes f-bar+ (calc_fb1 of
-//     the reference, src/dugks.cu:1131-1196); halo columns recompute it, wall
-//     ghost columns extrapolate it (src/dugks.cu:1234-1251 and the stretched
-//     form, src/fortran/channel/src/dugks.cuf:365-374);
+// Decomposition of the step (step_kernel.h).  A workgroup owns a TX x TY tile
+// of (x, y) columns and marches along z over a chunk of planes.  Its lanes
+// hold the tile's columns, the two y-halo rows and the two x-halo columns; a
+// column is a lane's with FP32 arithmetic and a pair of lanes' with FP64
+// (step_common.h).  Each plane it:
+//   - computes f-bar+ of its columns at plane p+1 (calc_fb1 of the reference,
+//     src/dugks.cu:1131-1196) from the f it loaded a plane ahead; halo columns
+//     recompute it, wall ghost columns extrapolate it
+//     (src/dugks.cu:1234-1251 and the stretched form,
+//     src/fortran/channel/src/dugks.cuf:365-374);
 //   - reconstructs every face once (the reference computes each interior face
-//     twice, quirk Q5): the trilinear interpolation of src/dugks.cu:756-906 is
+//     twice): the trilinear interpolation of src/dugks.cu:756-906 is
 //     evaluated z-lerp first, so the x- and y-faces of plane p read a single
 //     LDS plane Z(p) and the z-face between p and p+1 reads Zn(p+1/2);
 //   - applies wall bounce-back and the face collision (f2ruvwh + feq_s,
@@ -26,6 +28,24 @@
 // differences of the two-cell means), on uniform axes; the LDS then holds a
 // ring of the f-bar+ planes p-1, p and p+1, written as each is computed.
 // Other configurations use the two-pass kernels.
+//
+// What bounds it.  The step moves 38 values per cell (f in, f out; halos come
+// from L2) and does about 2300 operations per cell.  On 256x192x256 with one
+// MI355X (a large copy runs at 4.9 TB/s) the traffic alone takes 0.39 ms in
+// FP32 and 0.78 ms in FP64, the arithmetic with the memory accesses taken out
+// 0.55 and 1.13 ms: the kernel is bound by issue.  Two waves per SIMD fit, so
+// what counts is that a wave never waits: the loads of the next plane go out
+// in three groups between the phases (issued in one burst they fill the
+// memory pipeline and the wave stalls at issue: 0.83 against 0.68 ms in FP32,
+// 1.54 against 1.19 ms in FP64), loads and stores run without branches so
+// that a wait counts exactly, and the halo waves take their share of the
+// y-faces.  Measured per step, 256x192x256 periodic / channel with a
+// flow-rate controller (before: a lane per column with planes of single
+// values in LDS, one wave per SIMD in FP64, whole-plane loads at once):
+//   FP32          0.623 / 0.685 ms  (0.719 / 0.751)
+//   FP64          1.185 / 1.329     (1.88  / 1.92)
+//   FP16 dev.     0.649 / 0.710     (0.729 / 0.797)
+//   FP16 non-eq.  0.717 / 0.772     (0.966 / 0.964)
 #include "device_common.h"
 
 namespace dugks {
@@ -84,43 +104,26 @@ __device__ __forceinline__ Real grad_foot(Real m, Real h, Real gx, Real gy, Real
   }
 }
 
-// ADJ = false: one DUGKS step fin -> fout.
-// ADJ = true: the adjoint-face pass of the step taken from fin: every face is
-// reconstructed and its collision linearised as in the step, and the
-// cotangents of its 19 reconstructed values, driven by lam' (adj.lam), are
-// written to adj.faces; nothing else is written.  FADJ (with ADJ): also the
-// cotangent of the ambient force along the flow axis through the face
-// collisions, summed per block into partial[tile] (fixed order).
-template <class Real, class Store, int TX, int TY, bool ADJ = false, bool COMPACT = false, class LamT = double,
-          bool FADJ = false, bool GRAD = false>
+// The adjoint-face pass of the step taken from fin: every face is
+// reconstructed and its collision linearised as in the step (trilinear
+// reconstruction), and the cotangents of its 19 reconstructed values, driven
+// by lam' (adj.lam), are written to adj.faces; nothing else is written.  FADJ:
+// also the cotangent of the ambient force along the flow axis through the
+// face collisions, summed per block into partial[tile] (fixed order).
+template <class Real, class Store, int TX, int TY, bool COMPACT = false, class LamT = double, bool FADJ = false>
 // FP32 arithmetic: two blocks per CU (at most 256 registers per lane)
-__global__ void __launch_bounds__(((TY + 2) * TX + 2 * (TY + 2) + 63) / 64 * 64, sizeof(Real) == 4 ? 2 : 1) k_fused(
-    KParams P, const Store* __restrict__ fin,
-                                                          Store* __restrict__ fout, int TZ,
-                                                          double* __restrict__ partial, AdjFaceIO adj) {
+__global__ void __launch_bounds__(((TY + 2) * TX + 2 * (TY + 2) + 63) / 64 * 64, sizeof(Real) == 4 ? 2 : 1)
+    k_adj_faces(KParams P, const Store* __restrict__ fin, int TZ, double* __restrict__ partial, AdjFaceIO adj) {
   using T = Tile<TX, TY>;
   constexpr int AC = T::AC;
-  static_assert(!(GRAD && ADJ), "the adjoint differentiates the trilinear reconstruction");
-  // With FP16 non-equilibrium storage the step carries shifted populations
-  // h = f - w (see EqShift): f-bar+, the LDS planes, the face values and the
-  // update are all f - w, decoded from and encoded to the stored rho - 1, u
-  // and non-equilibrium part without forming f (fewer operations than
-  // through f).  The other storage modes and the adjoint-face pass work on f.
-  constexpr bool kShift = std::is_same<Store, NeqHalf>::value && !ADJ;
   // LDS planes indexed (row, column).  16-wide rows put four rows in a wave:
   // column-major planes (column stride TY + 2, even) then keep the lanes of
   // a ds_read on distinct banks; 32-wide rows are conflict-free row-major.
   constexpr bool CM = TX == 16;
   auto ia = [](int rr, int cc) { return CM ? cc * (TY + 2) + rr : rr * AC + cc; };       // A, An, Lam
-  auto ic = [](int rr, int cc) { return CM ? cc * TY + rr : rr * (TX + 1) + cc; };       // Cx (rows 0..TY-1)
-  auto id = [](int rr, int cc) { return CM ? cc * (TY + 1) + rr : rr * TX + cc; };       // Dy (rows 0..TY)
-  // GRAD: A holds the ring of f-bar+ planes, plane k in slot (k + 3) % 3
-  // (population ip of slot s at A[s * Q + ip]); An is unused
-  __shared__ Real A[GRAD ? 3 * Q : Q][(TY + 2) * AC];  // Z(p): tangential z-lerp of f-bar(p)
-  __shared__ Real An[GRAD ? 1 : Q][(TY + 2) * AC];     // Zn(p+1/2): normal z-lerp between p and p+1
-  __shared__ Real Cx[ADJ ? 1 : 10][TY * (TX + 1)];  // crossing populations of -x faces
-  __shared__ Real Dy[ADJ ? 1 : 10][(TY + 1) * TX];  // crossing populations of -y faces
-  __shared__ Real Lam[ADJ ? Q : 1][(TY + 2) * AC];  // adjoint-face pass: lam'(p) of the tile and halo
+  __shared__ Real A[Q][(TY + 2) * AC];    // Z(p): tangential z-lerp of f-bar(p)
+  __shared__ Real An[Q][(TY + 2) * AC];   // Zn(p+1/2): normal z-lerp between p and p+1
+  __shared__ Real Lam[Q][(TY + 2) * AC];  // lam'(p) of the tile and halo
   __shared__ Real WX[6][TX + 2];           // weights per tile column
   __shared__ Real WY[6][TY + 2];           // weights per tile row
 
@@ -142,7 +145,7 @@ __global__ void __launch_bounds__(((TY + 2) * TX + 2 * (TY + 2) + 63) / 64 * 64,
   const int zend = min(z0 + TZ, nz);
   const unsigned Nb = (unsigned)(P.N * (long long)sizeof(Store));  // bytes per population
   const unsigned span = (unsigned)state_bytes<Store>((unsigned long long)P.N);
-  const StateBuf<Store> bin(fin, span), bout(fout, span);
+  const StateBuf<Store> bin(fin, span);
 
   // column of this thread in tile coordinates: r = 0..TY+1 (y = j0-1+r),
   // c = -1..TX (x = i0+c).  Lanes: the TY interior rows first (whole waves
@@ -184,15 +187,6 @@ __global__ void __launch_bounds__(((TY + 2) * TX + 2 * (TY + 2) + 63) / 64 * 64,
   const Real wzt_p = tz(9 + 7);  // tangential, toward p-1 (c_z = +1)
   const Real wzn[3] = {tz(9 + 0), tz(9 + 1), tz(9 + 2)};  // normal, toward p+1
   const Real updz = tz(9 + 8);
-  // GRAD: 1/d and 1/(2d) per axis (every axis uniform)
-  Real gin[3] = {Real(0), Real(0), Real(0)}, gtn[3] = {Real(0), Real(0), Real(0)};
-  if constexpr (GRAD) {
-    for (int a = 0; a < 3; a++) {
-      gin[a] = (Real)(1.0 / P.du[a]);
-      gtn[a] = (Real)(0.5 / P.du[a]);
-    }
-  }
-  auto rslot = [](int k) { return (k + 3) % 3; };  // ring slot of plane k >= -1
   // Per-column and per-row weights of the tile, copied once into LDS: the
   // tables are not written by this kernel, but the compiler cannot prove that
   // against the f stores and would reload them (or hold them in registers)
@@ -217,8 +211,7 @@ __global__ void __launch_bounds__(((TY + 2) * TX + 2 * (TY + 2) + 63) / 64 * 64,
   auto yn = [&](int k) { return WY[k][r]; };
   auto yt = [&](int s) { return WY[3 + s][r]; };
 
-  Real fbm[5], fbc[Q], fbn[Q], zm[10];
-  double flow = 0;
+  Real fbm[5], fbc[Q], fbn[Q];
   const int as = P.flow_axis;
   // FADJ: the face collisions' force cotangents of this thread's faces
   double fsum[3] = {0, 0, 0};
@@ -256,69 +249,6 @@ __global__ void __launch_bounds__(((TY + 2) * TX + 2 * (TY + 2) + 63) / 64 * 64,
       fc.template put<ip>(v);
     });
   };
-  // GRAD: population ip of ring slot sl at LDS position (rr, cc)
-  auto ga = [&](int sl, int ip, int rr, int cc) -> Real { return A[sl * Q + ip][ia(rr, cc)]; };
-  // GRAD reconstructions from the ring (slots sm, s0, sp of planes p-1, p,
-  // p+1): the x-face between tile columns c-1 and c of row r, the y-face
-  // between rows r-1 and r of column c, both at plane p, and the z-face
-  // between planes p (s0) and p+1 (sp) of the thread's column
-  auto grad_face_x = [&](Face<Real, 0>& fc, int sm, int s0, int sp) {
-    static_for<Q>([&](auto I) {
-      constexpr int ip = decltype(I)::value;
-      constexpr int cx = CX[ip], cy = CY[ip], cz = CZ[ip];
-      const Real fl = ga(s0, ip, r, c), fr = ga(s0, ip, r, c + 1);
-      Real gy = Real(0), gz = Real(0);
-      if constexpr (cy != 0)
-        gy = (Real(0.5) * (ga(s0, ip, r + 1, c) + ga(s0, ip, r + 1, c + 1)) -
-              Real(0.5) * (ga(s0, ip, r - 1, c) + ga(s0, ip, r - 1, c + 1))) * gtn[1];
-      if constexpr (cz != 0)
-        gz = (Real(0.5) * (ga(sp, ip, r, c) + ga(sp, ip, r, c + 1)) -
-              Real(0.5) * (ga(sm, ip, r, c) + ga(sm, ip, r, c + 1))) * gtn[2];
-      fc.template put<ip>(grad_foot<cx, cy, cz>(Real(0.5) * (fr + fl), hdt, (fr - fl) * gin[0], gy, gz));
-    });
-  };
-  auto grad_face_y = [&](Face<Real, 1>& fc, int sm, int s0, int sp) {
-    static_for<Q>([&](auto I) {
-      constexpr int ip = decltype(I)::value;
-      constexpr int cx = CX[ip], cy = CY[ip], cz = CZ[ip];
-      const Real fl = ga(s0, ip, r - 1, c + 1), fr = ga(s0, ip, r, c + 1);
-      Real gx = Real(0), gz = Real(0);
-      if constexpr (cx != 0)
-        gx = (Real(0.5) * (ga(s0, ip, r - 1, c + 2) + ga(s0, ip, r, c + 2)) -
-              Real(0.5) * (ga(s0, ip, r - 1, c) + ga(s0, ip, r, c))) * gtn[0];
-      if constexpr (cz != 0)
-        gz = (Real(0.5) * (ga(sp, ip, r - 1, c + 1) + ga(sp, ip, r, c + 1)) -
-              Real(0.5) * (ga(sm, ip, r - 1, c + 1) + ga(sm, ip, r, c + 1))) * gtn[2];
-      fc.template put<ip>(grad_foot<cx, cy, cz>(Real(0.5) * (fr + fl), hdt, gx, (fr - fl) * gin[1], gz));
-    });
-  };
-  auto grad_face_z = [&](Face<Real, 2>& fc, int s0, int sp) {
-    static_for<Q>([&](auto I) {
-      constexpr int ip = decltype(I)::value;
-      constexpr int cx = CX[ip], cy = CY[ip], cz = CZ[ip];
-      const Real fl = ga(s0, ip, r, c + 1), fr = ga(sp, ip, r, c + 1);
-      Real gx = Real(0), gy = Real(0);
-      if constexpr (cx != 0)
-        gx = (Real(0.5) * (ga(s0, ip, r, c + 2) + ga(sp, ip, r, c + 2)) -
-              Real(0.5) * (ga(s0, ip, r, c) + ga(sp, ip, r, c))) * gtn[0];
-      if constexpr (cy != 0)
-        gy = (Real(0.5) * (ga(s0, ip, r + 1, c + 1) + ga(sp, ip, r + 1, c + 1)) -
-              Real(0.5) * (ga(s0, ip, r - 1, c + 1) + ga(sp, ip, r - 1, c + 1))) * gtn[1];
-      fc.template put<ip>(grad_foot<cx, cy, cz>(Real(0.5) * (fr + fl), hdt, gx, gy, (fr - fl) * gin[2]));
-    });
-  };
-  // the +z face of plane p (GRAD: from ring slots s0 and sp)
-  auto zface = [&](Real (&out)[10], int s0, int sp) {
-    Face<Real, 2> fc;
-    if constexpr (GRAD)
-      grad_face_z(fc, s0, sp);
-    else
-      zface_rec(fc);
-    if constexpr (kShift)
-      fc.collide_shift(Famb, hdt, fw0, fw2, out);
-    else
-      fc.collide(Famb, hdt, fw0, fw1, fw2, out);
-  };
   // adjoint-face mode: lam' of population ip at an interior cell (0 for a
   // ghost, cell < 0) and the store of a face's cotangents
   // (both arrays are < 2 GiB, checked at launch: 32-bit buffer offsets)
@@ -342,7 +272,7 @@ __global__ void __launch_bounds__(((TY + 2) * TX + 2 * (TY + 2) + 63) / 64 * 64,
   // the flow-rate controller's term of lam' (AdjFaceIO::ubar): rho and j_a
   // of f(n+1) at the column's cell of plane k, loaded with lam', added before
   // lam' is used: lam'_i += s (c_ia - u_a), s = ubar (dV/V) / rho
-  constexpr bool kFlowFuse = ADJ && FADJ && COMPACT && std::is_same<Store, Real>::value;
+  constexpr bool kFlowFuse = FADJ && COMPACT && std::is_same<Store, Real>::value;
   const bool fuse = kFlowFuse && adj.ubar != nullptr;
   const RawBuf momn(static_cast<Real*>(adj.faces) + 3LL * kCompact * P.eN + (1 - adj.mom) * 4LL * P.N,
                     (unsigned)(4 * P.N * sizeof(Real)));
@@ -374,13 +304,11 @@ __global__ void __launch_bounds__(((TY + 2) * TX + 2 * (TY + 2) + 63) / 64 * 64,
     }
   };
   Real lamc[Q], lamn[Q], rnn = Real(0), jnn = Real(0);
-  if constexpr (ADJ) {
-    load_lam(z0, lamc);
-    if constexpr (kFlowFuse) {
-      Real rn = Real(0), jn = Real(0);
-      load_flow(z0, rn, jn);
-      add_flow(lamc, rn, jn);
-    }
+  load_lam(z0, lamc);
+  if constexpr (kFlowFuse) {
+    Real rn = Real(0), jn = Real(0);
+    load_flow(z0, rn, jn);
+    add_flow(lamc, rn, jn);
   }
   // compact form (COMPACT): per face the kCompact values of compact_record
   auto store_compact = [&](int a, long long slot, const Real (&rec)[kCompact]) {
@@ -418,72 +346,26 @@ __global__ void __launch_bounds__(((TY + 2) * TX + 2 * (TY + 2) + 63) / 64 * 64,
       F[2] += (Real)P.fcell[2 * P.N + cc];
     }
   };
-  // The update of plane p needs 4/3 f-bar+(p) - 1/3 f(p); it is formed when
-  // f(p) arrives for f-bar+(p), so f is read once per step: gc holds it for
-  // the current plane, gn for the next.  Written f-bar+ + (f-bar+ - f)/3:
-  // the two terms of the difference carry the same mass, so the rounding of
-  // 1/3 biases nothing (the rounded 4/3 and 1/3 of the plain form add about
-  // 3e-8 of the mass per step in FP32).
-  Real gc[Q], gn[Q];
-  auto form_g = [&](const Real (&fb)[Q], const Real (&ff)[Q], Real (&g)[Q]) {
-    static_for<Q>([&](auto I) {
-      constexpr int ip = decltype(I)::value;
-      g[ip] = fb[ip] + (fb[ip] - ff[ip]) * Real(1.0 / 3.0);
-    });
-  };
-
   // f of the own column one plane ahead of its f-bar: the loads are issued
   // one iteration before their f-bar needs them.  The first (plane z0+1) is
   // issued ahead of the pre-loop's loads, so it arrives with them.
-  constexpr bool kPrefetch = true;
   RawCell<Real, Store> fpre;
-  if (kPrefetch && own) load_own((z0 + 1) % nz, fpre);
+  if (own) load_own((z0 + 1) % nz, fpre);
 
-  // ---- pre-loop: f-bar at z0-1 and z0, and the -z face of plane z0 ----
+  // ---- pre-loop: f-bar at z0-1 and z0 ----
   {
     const int km = (z0 - 1 + nz) % nz;
     if (active) {
-      fbar_column<Real, Store, kShift>(P, bin, Nb, gi, gj, km, Famb, fbn);
-      if (!ADJ && own) {
-        RawCell<Real, Store> raw;
-        Real ff[Q], F[3], rho, u0[3];
-        load_own(z0, raw);
-        force_own(z0, F);
-        if constexpr (kShift) {
-          raw.decode_shift(P, ff, rho, u0);
-          centre_fbar_shift<Real>(ff, rho, u0, F, hdt, (Real)P.bw0, (Real)P.bw2, fbc);
-        } else {
-          raw.decode(P, ff, rho, u0);
-          centre_fbar<Real>(ff, rho, u0, F, hdt, (Real)P.bw0, (Real)P.bw2, fbc);
-        }
-        if constexpr (!ADJ) form_g(fbc, ff, gc);
-      } else {
-        fbar_column<Real, Store, kShift>(P, bin, Nb, gi, gj, z0, Famb, fbc);
-      }
+      fbar_column<Real, Store>(P, bin, Nb, gi, gj, km, Famb, fbn);
+      fbar_column<Real, Store>(P, bin, Nb, gi, gj, z0, Famb, fbc);
       static_for<5>([&](auto K) {
         constexpr int k = decltype(K)::value;
         fbm[k] = fbn[ZP[k]];
       });
     }
-    if constexpr (GRAD) {
-      if (active) {
-        static_for<Q>([&](auto I) {
-          constexpr int ip = decltype(I)::value;
-          A[rslot(z0 - 1) * Q + ip][ia(r, c + 1)] = fbn[ip];
-          A[rslot(z0) * Q + ip][ia(r, c + 1)] = fbc[ip];
-        });
-      }
-    } else {
-      store_zn(fbn, fbc);
-    }
-    __syncthreads();
-    if constexpr (!ADJ) {
-      if (interior) zface(zm, rslot(z0 - 1), rslot(z0));
-    }
-    __syncthreads();
   }
 
-  if constexpr (kPrefetch) fpre.settle();
+  fpre.settle();
   // compact adjoint-face records with the state stored in the arithmetic
   // type (FP32 or FP64): rho and j of every cell
   // for the gather, written by the interior lanes from the prefetched f.
@@ -499,54 +381,33 @@ __global__ void __launch_bounds__(((TY + 2) * TX + 2 * (TY + 2) + 63) / 64 * 64,
     mb.st(jm[1], vb, 2 * pop);
     mb.st(jm[2], vb, 3 * pop);
   };
-  // One plane p: fbc / gc / lamc hold f-bar+, 4/3 f-bar+ - 1/3 f and lam' of
-  // plane p, and the plane computes those of p + 1 into fbn / gn / lamn.  The
-  // step's loop below runs the planes in pairs with the two register sets
-  // swapped, so no copy moves plane p+1's values into plane p's registers.
-  auto plane = [&](int p, Real (&fbc)[Q], Real (&fbn)[Q], Real (&gc)[Q], Real (&gn)[Q], Real (&lamc)[Q],
-                   Real (&lamn)[Q]) {
+  // One plane p: fbc / lamc hold f-bar+ and lam' of plane p, and the plane
+  // computes those of p + 1 into fbn / lamn.
+  // (Parameters, not captures: captured arrays that the loop also copies stay
+  // in scratch memory, 3.8 against 2.7 ms an adjoint step on 256x192x256.)
+  auto plane = [&](int p, Real (&fbc)[Q], Real (&fbn)[Q], Real (&lamc)[Q], Real (&lamn)[Q]) {
     const int kn = (p + 1) % nz;
-    if constexpr (ADJ) {
-      load_lam(kn, lamn);
-      load_flow(kn, rnn, jnn);
-    }
+    load_lam(kn, lamn);
+    load_flow(kn, rnn, jnn);
     if (own) {
-      if constexpr (!kPrefetch) load_own(kn, fpre);
       Real F[3];
       force_own(kn, F);
       Real ff[Q], rho, u0[3];
-      if constexpr (kShift) {
-        fpre.decode_shift(P, ff, rho, u0);
-        centre_fbar_shift<Real>(ff, rho, u0, F, hdt, (Real)P.bw0, (Real)P.bw2, fbn);
-      } else {
-        fpre.decode(P, ff, rho, u0);
-        if constexpr (ADJ && COMPACT && std::is_same<Store, Real>::value) {
-          if (interior) {
-            Real jm[3];
-            cell_moments<Real>(ff, rho, jm);
-            store_moments(kn, rho, jm);
-          }
+      fpre.decode(P, ff, rho, u0);
+      if constexpr (COMPACT && std::is_same<Store, Real>::value) {
+        if (interior) {
+          Real jm[3];
+          cell_moments<Real>(ff, rho, jm);
+          store_moments(kn, rho, jm);
         }
-        centre_fbar<Real>(ff, rho, u0, F, hdt, (Real)P.bw0, (Real)P.bw2, fbn);
       }
-      if constexpr (!ADJ) {
-        if (interior) form_g(fbn, ff, gn);
-      }
-      if (kPrefetch && p + 1 < zend) load_own((p + 2) % nz, fpre);
+      centre_fbar<Real>(ff, rho, u0, F, hdt, (Real)P.bw0, (Real)P.bw2, fbn);
+      if (p + 1 < zend) load_own((p + 2) % nz, fpre);
     } else if (active) {
-      fbar_column<Real, Store, kShift>(P, bin, Nb, gi, gj, kn, Famb, fbn);
+      fbar_column<Real, Store>(P, bin, Nb, gi, gj, kn, Famb, fbn);
     }
     // ---- phase 1: Z(p) (tangential z-lerp of f-bar(p)) and Zn(p+1/2) ----
-    // (GRAD: f-bar+(p+1) into its ring slot)
-    const int sm = rslot(p - 1), s0 = rslot(p), sp = rslot(p + 1);
-    if constexpr (GRAD) {
-      if (active) {
-        static_for<Q>([&](auto I) {
-          constexpr int ip = decltype(I)::value;
-          A[sp * Q + ip][ia(r, c + 1)] = fbn[ip];
-        });
-      }
-    } else if (active) {
+    if (active) {
       static_for<Q>([&](auto I) {
         constexpr int ip = decltype(I)::value;
         constexpr int cz = CZ[ip];
@@ -560,27 +421,23 @@ __global__ void __launch_bounds__(((TY + 2) * TX + 2 * (TY + 2) + 63) / 64 * 64,
         }
       });
     }
-    if constexpr (!GRAD) store_zn(fbc, fbn);
-    if constexpr (ADJ) {
-      if (active) {
-        static_for<Q>([&](auto I) {
-          constexpr int ip = decltype(I)::value;
-          if constexpr (ip != 0) Lam[ip][ia(r, c + 1)] = lamc[ip];
-        });
-      }
+    store_zn(fbc, fbn);
+    if (active) {
+      static_for<Q>([&](auto I) {
+        constexpr int ip = decltype(I)::value;
+        if constexpr (ip != 0) Lam[ip][ia(r, c + 1)] = lamc[ip];
+      });
     }
     __syncthreads();
     // ---- phase 2: the faces of plane p (-x, -y from Z; +z from Zn) ----
-    // the forward needs the tile's right and top boundary faces too; the
-    // adjoint-face pass leaves them to the next tile except at a wall
+    // the tile's right and top boundary faces are the next tile's, except at a wall
     const bool xhalo = active && t >= T::NROW && c == TX && r >= 1 && r <= TY;
-    const bool do_x = interior || (xhalo && (!ADJ || (!P.periodic[0] && gi == nx)));
-    const bool do_y = t < T::NROW && r >= 1 && (!ADJ || r <= TY || (!P.periodic[1] && gj == ny));
+    const bool do_x = interior || (xhalo && !P.periodic[0] && gi == nx);
+    const bool do_y = t < T::NROW && r >= 1 && (r <= TY || (!P.periodic[1] && gj == ny));
     if (do_x) {
       // face between x-columns gi-1 (left, ghost-inclusive index mi-1) and gi
       Face<Real, 0> fc;
-      if constexpr (GRAD) grad_face_x(fc, sm, s0, sp);
-      else static_for<Q>([&](auto I) {
+      static_for<Q>([&](auto I) {
         constexpr int ip = decltype(I)::value;
         constexpr int cx = CX[ip], cy = CY[ip];
         if constexpr (ip == 0) {
@@ -598,45 +455,32 @@ __global__ void __launch_bounds__(((TY + 2) * TX + 2 * (TY + 2) + 63) / 64 * 64,
       });
       const bool lw = !P.periodic[0] && gi == 0, hw = !P.periodic[0] && gi == nx;
       if (!P.periodic[0]) fc.bounce(lw, hw);
-      if constexpr (ADJ) {
-        const Real uL = WX[5][c], uR = WX[5][c + 1];
-        Real mu[10], lam[Q];
-        static_for<10>([&](auto K) {
-          constexpr int k = decltype(K)::value;
-          constexpr int ip = XD[k];
-          mu[k] = Real(CX[ip]) * (uR * Lam[ip][ia(r, c + 1)] - uL * Lam[ip][ia(r, c)]);
-        });
-        // (no "cond ? nx : gi": the optimiser turns a select between two
-        // captured variables into a select between their addresses, which
-        // keeps them in scratch memory)
-        const int slot = gi + ((gi == 0 && P.periodic[0]) ? nx : 0);
-        const long long fs = ((long long)(p + 1) * e1 + (gj + 1)) * e0 + slot;
-        if constexpr (COMPACT) {
-          Real Ac, B[3], rec[kCompact];
-          fc.template adjoint_coeffs<FADJ>(Famb, hdt, fw0, fw2, mu, Ac, B, fsum);
-          compact_record<Real, 0>(mu, Ac, B, fw1, rec);
-          store_compact(0, fs, rec);
-        } else {
-          fc.template adjoint<FADJ>(Famb, hdt, fw0, fw1, fw2, mu, lw, hw, lam, fsum);
-          store_face(0, fs, lam);
-        }
+      const Real uL = WX[5][c], uR = WX[5][c + 1];
+      Real mu[10], lam[Q];
+      static_for<10>([&](auto K) {
+        constexpr int k = decltype(K)::value;
+        constexpr int ip = XD[k];
+        mu[k] = Real(CX[ip]) * (uR * Lam[ip][ia(r, c + 1)] - uL * Lam[ip][ia(r, c)]);
+      });
+      // (no "cond ? nx : gi": the optimiser turns a select between two
+      // captured variables into a select between their addresses, which
+      // keeps them in scratch memory)
+      const int slot = gi + ((gi == 0 && P.periodic[0]) ? nx : 0);
+      const long long fs = ((long long)(p + 1) * e1 + (gj + 1)) * e0 + slot;
+      if constexpr (COMPACT) {
+        Real Ac, B[3], rec[kCompact];
+        fc.template adjoint_coeffs<FADJ>(Famb, hdt, fw0, fw2, mu, Ac, B, fsum);
+        compact_record<Real, 0>(mu, Ac, B, fw1, rec);
+        store_compact(0, fs, rec);
       } else {
-        Real out[10];
-        if constexpr (kShift)
-          fc.collide_shift(Famb, hdt, fw0, fw2, out);
-        else
-          fc.collide(Famb, hdt, fw0, fw1, fw2, out);
-        static_for<10>([&](auto K) {
-          constexpr int k = decltype(K)::value;
-          Cx[k][ic(r - 1, c)] = out[k];
-        });
+        fc.template adjoint<FADJ>(Famb, hdt, fw0, fw1, fw2, mu, lw, hw, lam, fsum);
+        store_face(0, fs, lam);
       }
     }
     if (do_y) {
       // face between y-rows gj-1 (below) and gj
       Face<Real, 1> fc;
-      if constexpr (GRAD) grad_face_y(fc, sm, s0, sp);
-      else static_for<Q>([&](auto I) {
+      static_for<Q>([&](auto I) {
         constexpr int ip = decltype(I)::value;
         constexpr int cx = CX[ip], cy = CY[ip];
         if constexpr (ip == 0) {
@@ -654,174 +498,68 @@ __global__ void __launch_bounds__(((TY + 2) * TX + 2 * (TY + 2) + 63) / 64 * 64,
       });
       const bool lw = !P.periodic[1] && gj == 0, hw = !P.periodic[1] && gj == ny;
       if (!P.periodic[1]) fc.bounce(lw, hw);
-      if constexpr (ADJ) {
-        const Real uL = WY[5][r - 1], uR = WY[5][r];
-        Real mu[10], lam[Q];
-        static_for<10>([&](auto K) {
-          constexpr int k = decltype(K)::value;
-          constexpr int ip = YD[k];
-          mu[k] = Real(CY[ip]) * (uR * Lam[ip][ia(r, c + 1)] - uL * Lam[ip][ia(r - 1, c + 1)]);
-        });
-        const int slot = gj + ((gj == 0 && P.periodic[1]) ? ny : 0);
-        const long long fs = ((long long)(p + 1) * e1 + slot) * e0 + (gi + 1);
-        if constexpr (COMPACT) {
-          Real Ac, B[3], rec[kCompact];
-          fc.template adjoint_coeffs<FADJ>(Famb, hdt, fw0, fw2, mu, Ac, B, fsum);
-          compact_record<Real, 1>(mu, Ac, B, fw1, rec);
-          store_compact(1, fs, rec);
-        } else {
-          fc.template adjoint<FADJ>(Famb, hdt, fw0, fw1, fw2, mu, lw, hw, lam, fsum);
-          store_face(1, fs, lam);
-        }
+      const Real uL = WY[5][r - 1], uR = WY[5][r];
+      Real mu[10], lam[Q];
+      static_for<10>([&](auto K) {
+        constexpr int k = decltype(K)::value;
+        constexpr int ip = YD[k];
+        mu[k] = Real(CY[ip]) * (uR * Lam[ip][ia(r, c + 1)] - uL * Lam[ip][ia(r - 1, c + 1)]);
+      });
+      const int slot = gj + ((gj == 0 && P.periodic[1]) ? ny : 0);
+      const long long fs = ((long long)(p + 1) * e1 + slot) * e0 + (gi + 1);
+      if constexpr (COMPACT) {
+        Real Ac, B[3], rec[kCompact];
+        fc.template adjoint_coeffs<FADJ>(Famb, hdt, fw0, fw2, mu, Ac, B, fsum);
+        compact_record<Real, 1>(mu, Ac, B, fw1, rec);
+        store_compact(1, fs, rec);
       } else {
-        Real out[10];
-        if constexpr (kShift)
-          fc.collide_shift(Famb, hdt, fw0, fw2, out);
-        else
-          fc.collide(Famb, hdt, fw0, fw1, fw2, out);
-        static_for<10>([&](auto K) {
-          constexpr int k = decltype(K)::value;
-          Dy[k][id(r - 1, c)] = out[k];
-        });
+        fc.template adjoint<FADJ>(Famb, hdt, fw0, fw1, fw2, mu, lw, hw, lam, fsum);
+        store_face(1, fs, lam);
       }
     }
-    Real zp[10];
     // lam' of plane p+1 complete (its loads were issued at the top of the plane)
     if constexpr (kFlowFuse) add_flow(lamn, rnn, jnn);
-    if constexpr (ADJ) {
-      if (interior) {
-        // +z face of the cell: between planes p and p+1 (z is periodic)
-        Face<Real, 2> fc;
-        zface_rec(fc);
-        Real mu[10], lam[Q];
-        static_for<10>([&](auto K) {
-          constexpr int k = decltype(K)::value;
-          constexpr int ip = ZD[k];
-          mu[k] = Real(CZ[ip]) * updz * (lamn[ip] - lamc[ip]);
-        });
-        const long long fs = ((long long)(p + 1) * e1 + (gj + 1)) * e0 + (gi + 1);
-        if constexpr (COMPACT) {
-          Real Ac, B[3], rec[kCompact];
-          fc.template adjoint_coeffs<FADJ>(Famb, hdt, fw0, fw2, mu, Ac, B, fsum);
-          compact_record<Real, 2>(mu, Ac, B, fw1, rec);
-          store_compact(2, fs, rec);
-        } else {
-          fc.template adjoint<FADJ>(Famb, hdt, fw0, fw1, fw2, mu, false, false, lam, fsum);
-          store_face(2, fs, lam);
-        }
+    if (interior) {
+      // +z face of the cell: between planes p and p+1 (z is periodic)
+      Face<Real, 2> fc;
+      zface_rec(fc);
+      Real mu[10], lam[Q];
+      static_for<10>([&](auto K) {
+        constexpr int k = decltype(K)::value;
+        constexpr int ip = ZD[k];
+        mu[k] = Real(CZ[ip]) * updz * (lamn[ip] - lamc[ip]);
+      });
+      const long long fs = ((long long)(p + 1) * e1 + (gj + 1)) * e0 + (gi + 1);
+      if constexpr (COMPACT) {
+        Real Ac, B[3], rec[kCompact];
+        fc.template adjoint_coeffs<FADJ>(Famb, hdt, fw0, fw2, mu, Ac, B, fsum);
+        compact_record<Real, 2>(mu, Ac, B, fw1, rec);
+        store_compact(2, fs, rec);
+      } else {
+        fc.template adjoint<FADJ>(Famb, hdt, fw0, fw1, fw2, mu, false, false, lam, fsum);
+        store_face(2, fs, lam);
       }
-    } else {
-      if (interior) zface(zp, s0, sp);
     }
     __syncthreads();
-    // ---- phase 3: update of plane p ----
-    // The f prefetched in phase 1 is taken before this plane's stores, so
-    // that the next plane's decode does not wait for them (see
-    // RawCell::settle).  FP32 storage takes it after the update's arithmetic,
-    // which then overlaps the loads still in flight (0.831 against 0.850 ms
-    // on the 256x192x256 channel); the other storage modes lost with that
-    // order (FP64 2.005 against 1.919 ms, FP16 non-equilibrium 1.028
-    // against 0.927 ms) and take it first.
-    constexpr bool kLateSettle = std::is_same<Store, float>::value;
-    if constexpr (!ADJ && kPrefetch && !kLateSettle) fpre.settle();
-    if constexpr (!ADJ) {
-      if (interior) {
-        const unsigned cell = ((unsigned)p * ny + gj) * nx + gi;
-        const unsigned vb = cell * (unsigned)sizeof(Store);
-        const Real updx = WX[5][c + 1], updy = WY[5][r];
-        // f~(p+1) = 4/3 f-bar+ - 1/3 f~ - sum_a (dt/dx_a) c_a (F_a+ - F_a-)
-        constexpr bool kNeq = std::is_same<Store, NeqHalf>::value;
-        Real fnew[Q];
-        static_for<Q>([&](auto I) {
-          constexpr int ip = decltype(I)::value;
-          Real v = gc[ip];
-          constexpr int kx = cross_index<0>(ip), ky = cross_index<1>(ip), kz = cross_index<2>(ip);
-          if constexpr (kx >= 0) v -= Real(CX[ip]) * updx * (Cx[kx][ic(r - 1, c + 1)] - Cx[kx][ic(r - 1, c)]);
-          if constexpr (ky >= 0) v -= Real(CY[ip]) * updy * (Dy[ky][id(r, c)] - Dy[ky][id(r - 1, c)]);
-          if constexpr (kz >= 0) {
-            v -= Real(CZ[ip]) * updz * (zp[kz] - zm[kz]);
-            zm[kz] = zp[kz];
-          }
-          // per-population stores go out as each value is ready (FP32
-          // storage: after the prefetch is taken, below); FP16
-          // non-equilibrium storage encodes the whole cell below
-          if constexpr (!kNeq && !kLateSettle) {
-            if constexpr (kShift)
-              st_state_shift<Real, Store>(bout, vb, ip * Nb, v, P, ip);
-            else
-              st_state<Real, Store>(bout, vb, ip * Nb, v, P, ip);
-          }
-          fnew[ip] = v;
-        });
-        if constexpr (kLateSettle) {
-          if constexpr (kPrefetch) fpre.settle();
-          static_for<Q>([&](auto I) {
-            constexpr int ip = decltype(I)::value;
-            st_state<Real, Store>(bout, vb, ip * Nb, fnew[ip], P, ip);
-          });
-        }
-        Real rr, u0n[3];
-        if constexpr (kNeq && kShift) {
-          store_neq_shift<Real>(bout, cell, (unsigned)P.N, fnew, rr, u0n);
-        } else if constexpr (kNeq) {
-          store_raw_cell<Real, Store>(bout, cell, (unsigned)P.N, P, fnew, true, rr, u0n);
-        } else if (partial) {
-          // the controller's reading only: FP32 sums suffice (the moments
-          // that feed the step are summed in FP64, cell_rho_u)
-          Real jn[3];
-          cell_moments<Real>(fnew, rr, jn);
-          if constexpr (kShift) rr += Real(1);
-          moment_velocity<Real>(rr, jn, u0n);
-        }
-        // bulk velocity of the new state for the flow-rate controller
-        // (per-cell moments in the arithmetic type, the sum over cells in FP64)
-        if (partial) flow += (double)(as == 0 ? u0n[0] : (as == 1 ? u0n[1] : u0n[2]));
-      } else if constexpr (kPrefetch && kLateSettle) {
-        fpre.settle();
-      }
-    }
-    if (!GRAD && active) {
+    if (active) {
       static_for<5>([&](auto K) {
         constexpr int k = decltype(K)::value;
         fbm[k] = fbc[ZP[k]];
       });
     }
-    // no barrier: the next phase 1 writes A/An (GRAD: the ring slot of p-1,
-    // last read in this plane's phase 2), which phase 3 does not read, and
-    // the next phase 2 writes Cx/Dy only after the next phase-1 barrier
   };
-  // The step runs planes in pairs; the adjoint-face pass (more registers
-  // live across the loop) one plane per iteration with the values of p+1
-  // copied down.
-  constexpr bool kPairs = !ADJ;
-  if constexpr (kPairs) {
-    for (int p = z0; p < zend; p += 2) {
-      plane(p, fbc, fbn, gc, gn, lamc, lamn);
-      if (p + 1 < zend) plane(p + 1, fbn, fbc, gn, gc, lamn, lamc);
-    }
-  } else {
-    for (int p = z0; p < zend; p++) {
-      plane(p, fbc, fbn, gc, gn, lamc, lamn);
-      if (active) {
-        static_for<Q>([&](auto I) {
-          constexpr int ip = decltype(I)::value;
-          fbc[ip] = fbn[ip];
-          if constexpr (ADJ && ip != 0) lamc[ip] = lamn[ip];
-          if constexpr (!ADJ) gc[ip] = gn[ip];
-        });
-      }
+  for (int p = z0; p < zend; p++) {
+    plane(p, fbc, fbn, lamc, lamn);
+    if (active) {
+      static_for<Q>([&](auto I) {
+        constexpr int ip = decltype(I)::value;
+        fbc[ip] = fbn[ip];
+        if constexpr (ip != 0) lamc[ip] = lamn[ip];
+      });
     }
   }
 
-  if (!ADJ && partial) {
-    // fixed-order block reduction of the flow sums; every column of the tile
-    // has the same z width (z is uniform here)
-    double v[1] = {interior ? flow * (P.wd[0][mi] * P.wd[1][mj] * P.wd[2][1]) : 0.0};
-    constexpr int kSum[1] = {0};
-    block_reduce<1, T::NT>(v, kSum);
-    if (t == 0) partial[tt] = v[0];
-  }
-  if constexpr (ADJ && FADJ) {
+  if constexpr (FADJ) {
     // the flow-axis component (assigned, not selected as an lvalue: a select
     // between array elements can keep the array in scratch memory)
     double v[1] = {fsum[0]};
@@ -832,6 +570,9 @@ __global__ void __launch_bounds__(((TY + 2) * TX + 2 * (TY + 2) + 63) / 64 * 64,
     if (t == 0) partial[tt] = v[0];
   }
 }
+
+#include "step_common.h"
+#include "step_kernel.h"
 
 // Final reduction of the per-block flow sums <j/rho> dV and the flow-rate
 // controller update (the law of k_flow_control).
@@ -852,53 +593,73 @@ __global__ void __launch_bounds__(256) k_flow_finish(const double* partial, int 
   }
 }
 
-// z-chunk length.  A chunk recomputes f-bar+ of the two planes before it.
-// With two resident workgroups per CU (FP32 arithmetic on 4-wave tiles) the
-// other workgroup covers that prologue, and more rounds of workgroups even
-// out the finish: 32 planes, on the 256x192x256 channel (256 columns of
-// 16x12, 2048 tiles) FP32 0.823 ms against 0.833 with 64 planes and 0.833
-// with 16, FP16 deviation storage 0.738 against 0.758 and 0.740 (128
-// planes: 0.865 / 0.783); on 128^3 (128 columns of 32x4, 512 tiles) 32
-// planes against 8: Taylor-Green FP32 0.148 against 0.166 ms, FP64 0.397
-// against 0.444 ms.  With one workgroup per CU (FP64, and the 8-wave
-// 32x12 tiles) nothing covers it and long chunks win for the step: 128
-// planes, FP32 on 32x12 0.724 ms against 0.731 with 64 and 0.751 with 32,
-// FP64 on 16x12 1.921 against 1.945 and 1.974.  The adjoint-face passes
-// (adj) keep 32 planes (with 128 their adjoint steps were 0.7 % slower).
-// Either start is halved, down to 8, while the grid has fewer tiles than one
-// round of resident workgroups on the 256 CUs.
+// z-chunk length of the adjoint-face pass: 32 planes (a chunk recomputes
+// f-bar+ of the two planes before it; 128 planes were 0.7 % slower on
+// 256x192x256), halved down to 8 while the grid has fewer tiles than one round
+// of resident workgroups on the 256 CUs.
 int blocks_per_cu(bool fp64, int TX, int TY) { return fp64 || Tile_nt(TX, TY) > 256 ? 1 : 2; }
-int z_chunk(const Ctx& cx, int TX, int TY, bool adj = false) {
-  if (cx.fused_tz > 0) return cx.fused_tz;
+int z_chunk(const Ctx& cx, int TX, int TY) {
   const long long cols = (long long)(cx.kp.n[0] / TX) * (cx.kp.n[1] / TY);
   const int per_cu = blocks_per_cu(cx.precision == 0, TX, TY);
-  int tz = per_cu == 1 && !adj ? 128 : 32;
+  int tz = 32;
   while (tz > 8 && cols * ((cx.kp.n[2] + tz - 1) / tz) < per_cu * 256) tz /= 2;
   return tz;
 }
 
+// The step's tiles and z-chunks.
+struct StepPlan {
+  int nchunk;         // z-chunks of every tile
+  long long nblocks;  // workgroups
+};
+// Tiles of 32 x 12 cells with FP32 arithmetic and 16 x 12 with FP64: the
+// tallest whose two LDS planes and face values fit 160 KB, one workgroup of
+// eight waves per CU, f-bar+ formed on 1.24 and 1.31 times the cells.  (FP32
+// on 16 x 12, two workgroups per CU: 0.80 against 0.68 ms on the 256x192x256
+// channel.)
+// Each of a chunk's planes takes the same time whatever the grid, and its
+// prologue about 2.2 planes' time (f-bar+ of two planes and one face).  The
+// number of chunks is the one with the least (rounds of 256 workgroups) x
+// (planes of the longest chunk + 2.2), the fewest at a tie.  Measured on
+// 64x64x32 FP64 (24 tiles): 8 chunks 30.5 us, 16 36.6, 32 39.4; on 64x72x32
+// FP32 (12 tiles): 8 chunks 28.0 us, 16 20.3, 32 24.3.
+template <int TX, int TY>
+StepPlan plan_tiles(const Setup& s) {
+  const long long tiles = (long long)((s.n[0] + TX - 1) / TX) * ((s.n[1] + TY - 1) / TY);
+  StepPlan best{1, tiles};
+  double least = 0;
+  for (int nc = 1; nc <= s.n[2]; nc++) {
+    const long long rounds = (tiles * nc + 255) / 256;
+    const double cost = (double)rounds * ((s.n[2] + nc - 1) / nc + 2.2);
+    if (nc == 1 || cost < least * (1 - 1e-9)) {
+      best = {nc, tiles * nc};
+      least = cost;
+    }
+    if ((double)rounds * 3.2 > least) break;  // only dearer from here
+  }
+  return best;
+}
+StepPlan step_plan(const Setup& s, int precision) {
+  return precision == 0 ? plan_tiles<16, 12>(s) : plan_tiles<32, 12>(s);
+}
+
 template <class Real, class Store, int TX, int TY, bool GRAD>
-hipError_t run_fused(Ctx& cx, const void* fin, void* fout) {
-  const KParams& P = cx.kp;
-  using T = Tile<TX, TY>;
-  const int TZ = z_chunk(cx, TX, TY);
-  dim3 grid(P.n[0] / TX, P.n[1] / TY, (P.n[2] + TZ - 1) / TZ);
-  const long long nblocks = (long long)grid.x * grid.y * grid.z;
+hipError_t run_step(Ctx& cx, const void* fin, void* fout) {
+  using T = StepTile<Real, TX, TY, GRAD>;
+  const StepPlan plan = step_plan(cx.s, cx.precision);
   double* partial = nullptr;
   const bool flow = cx.s.flow_rate != 0 && !cx.flow_frozen;
   if (flow) {
-    if ((size_t)nblocks > cx.flow_partial_len) return hipErrorInvalidValue;
+    if ((size_t)plan.nblocks > cx.flow_partial_len) return hipErrorInvalidValue;
     partial = cx.flow_partial;
   }
   if (cx.timing) hipEventRecord(cx.tev[0], cx.stream);
-  hipLaunchKernelGGL((k_fused<Real, Store, TX, TY, false, false, double, false, GRAD>), grid, dim3(T::NT), 0,
-                     cx.stream, P,
-                     static_cast<const Store*>(fin), static_cast<Store*>(fout), TZ, partial, AdjFaceIO{});
+  hipLaunchKernelGGL((k_step<Real, Store, TX, TY, GRAD>), dim3((unsigned)plan.nblocks), dim3(T::NT), 0, cx.stream,
+                     cx.kp, static_cast<const Store*>(fin), static_cast<Store*>(fout), plan.nchunk, partial);
   if (cx.timing) hipEventRecord(cx.tev[1], cx.stream);
   if (flow) {
     const Setup& s = cx.s;
     const double vol = s.width[0] * s.width[1] * s.width[2];
-    hipLaunchKernelGGL(k_flow_finish, dim3(1), dim3(256), 0, cx.stream, partial, (int)nblocks, cx.famb_dev,
+    hipLaunchKernelGGL(k_flow_finish, dim3(1), dim3(256), 0, cx.stream, partial, (int)plan.nblocks, cx.famb_dev,
                        s.stream_axis(), vol, s.flow_rate, s.flow_gain, s.dt);
   }
   cx.launches_per_step = flow ? 2 : 1;
@@ -908,7 +669,7 @@ hipError_t run_fused(Ctx& cx, const void* fin, void* fout) {
 template <int TX, int TY>
 dim3 adj_faces_grid(const Ctx& cx, int* TZ) {
   const KParams& P = cx.kp;
-  *TZ = z_chunk(cx, TX, TY, true);
+  *TZ = z_chunk(cx, TX, TY);
   return dim3(P.n[0] / TX, P.n[1] / TY, (P.n[2] + *TZ - 1) / *TZ);
 }
 
@@ -926,8 +687,8 @@ hipError_t run_adj_faces(Ctx& cx, const void* f, const void* lam, void* faces, d
     if (nb > fpart_len) return hipErrorInvalidValue;
     *nparts = nb;
   }
-  hipLaunchKernelGGL((k_fused<Real, Store, TX, TY, true, COMPACT, LamT, FADJ>), grid, dim3(T::NT), 0, cx.stream, P,
-                     static_cast<const Store*>(f), static_cast<Store*>(nullptr), TZ, FADJ ? fpart : nullptr,
+  hipLaunchKernelGGL((k_adj_faces<Real, Store, TX, TY, COMPACT, LamT, FADJ>), grid, dim3(T::NT), 0, cx.stream, P,
+                     static_cast<const Store*>(f), TZ, FADJ ? fpart : nullptr,
                      AdjFaceIO{lam, faces, mom, ubar, 1.0 / (cx.s.width[0] * cx.s.width[1] * cx.s.width[2])});
   return hipGetLastError();
 }
@@ -963,20 +724,16 @@ bool fused_supported(const Ctx& c, int* tx, int* ty) {
 
 namespace {
 template <bool GRAD>
-hipError_t launch_fused_recon(Ctx& c, const void* fin, void* fout, bool tall) {
+hipError_t launch_step_recon(Ctx& c, const void* fin, void* fout) {
   switch (c.precision) {
     case 0:
-      return tall ? run_fused<double, double, 16, 12, GRAD>(c, fin, fout)
-                  : run_fused<double, double, 32, 4, GRAD>(c, fin, fout);
+      return run_step<double, double, 16, 12, GRAD>(c, fin, fout);
     case 1:
-      return tall ? run_fused<float, float, 16, 12, GRAD>(c, fin, fout)
-                  : run_fused<float, float, 32, 4, GRAD>(c, fin, fout);
+      return run_step<float, float, 32, 12, GRAD>(c, fin, fout);
     case 2:
-      return tall ? run_fused<float, __half, 16, 12, GRAD>(c, fin, fout)
-                  : run_fused<float, __half, 32, 4, GRAD>(c, fin, fout);
+      return run_step<float, __half, 32, 12, GRAD>(c, fin, fout);
     default:
-      return tall ? run_fused<float, NeqHalf, 16, 12, GRAD>(c, fin, fout)
-                  : run_fused<float, NeqHalf, 32, 4, GRAD>(c, fin, fout);
+      return run_step<float, NeqHalf, 32, 12, GRAD>(c, fin, fout);
   }
 }
 }  // namespace
@@ -986,18 +743,10 @@ hipError_t launch_step_fused(Ctx& c, const void* fin, void* fout, bool* handled)
   *handled = false;
   if (!fused_supported(c, &tx, &ty)) return hipSuccess;
   *handled = true;
-  // FP32 storage takes 32 x 12 tiles where the grid divides: one workgroup
-  // of 8 waves per CU, rows of 32 floats that are whole 128-byte lines for
-  // every load and store (16-wide rows store half lines), f-bar+ on 1.24x the
-  // cells.  On the 256x192x256 channel 0.751 ms against 0.819 on 16 x 12;
-  // the FP16 storage modes lost with them (non-equilibrium 1.080 against
-  // 0.967 ms, deviation 0.809 against 0.771) and FP64 would need 210 KB of
-  // LDS.
-  if (c.precision == 1 && c.s.recon == 0 && c.kp.n[0] % 32 == 0 && c.kp.n[1] % 12 == 0)
-    return run_fused<float, float, 32, 12, false>(c, fin, fout);
-  return c.s.recon == 0 ? launch_fused_recon<false>(c, fin, fout, tx == 16)
-                        : launch_fused_recon<true>(c, fin, fout, tx == 16);
+  return c.s.recon == 0 ? launch_step_recon<false>(c, fin, fout) : launch_step_recon<true>(c, fin, fout);
 }
+
+long long step_fused_blocks(const Setup& s, int precision) { return step_plan(s, precision).nblocks; }
 
 bool adjoint_faces_fused_covers(const Ctx& c) {
   int tx = 32, ty = 4;
