@@ -113,7 +113,7 @@ __device__ __forceinline__ Real grad_foot(Real m, Real h, Real gx, Real gy, Real
 template <class Real, class Store, int TX, int TY, bool COMPACT = false, class LamT = double, bool FADJ = false>
 // FP32 arithmetic: two blocks per CU (at most 256 registers per lane)
 __global__ void __launch_bounds__(((TY + 2) * TX + 2 * (TY + 2) + 63) / 64 * 64, sizeof(Real) == 4 ? 2 : 1)
-    k_adj_faces(KParams P, const Store* __restrict__ fin, int TZ, double* __restrict__ partial, AdjFaceIO adj) {
+    k_adj_tile_faces(KParams P, const Store* __restrict__ fin, int TZ, double* __restrict__ partial, AdjFaceIO adj) {
   using T = Tile<TX, TY>;
   constexpr int AC = T::AC;
   // LDS planes indexed (row, column).  16-wide rows put four rows in a wave:
@@ -687,7 +687,7 @@ hipError_t run_adj_faces(Ctx& cx, const void* f, const void* lam, void* faces, d
     if (nb > fpart_len) return hipErrorInvalidValue;
     *nparts = nb;
   }
-  hipLaunchKernelGGL((k_adj_faces<Real, Store, TX, TY, COMPACT, LamT, FADJ>), grid, dim3(T::NT), 0, cx.stream, P,
+  hipLaunchKernelGGL((k_adj_tile_faces<Real, Store, TX, TY, COMPACT, LamT, FADJ>), grid, dim3(T::NT), 0, cx.stream, P,
                      static_cast<const Store*>(f), TZ, FADJ ? fpart : nullptr,
                      AdjFaceIO{lam, faces, mom, ubar, 1.0 / (cx.s.width[0] * cx.s.width[1] * cx.s.width[2])});
   return hipGetLastError();
@@ -695,19 +695,30 @@ hipError_t run_adj_faces(Ctx& cx, const void* f, const void* lam, void* faces, d
 
 }  // namespace
 
-// Either reconstruction (gradient reconstruction needs uniform axes, which
-// the configuration enforces); the adjoint-face mode trilinear only.
-bool fused_supported(const Ctx& c, int* tx, int* ty) {
+namespace {
+// What the tile kernels need of the grid, whatever its size.  Either
+// reconstruction (gradient reconstruction needs uniform axes, which the
+// configuration enforces).
+bool tiles_cover(const Ctx& c) {
   const Setup& s = c.s;
   if (!s.periodic[2] || !s.uniform[2]) return false;
   // buffer offsets are 32-bit: one state array must span < 4 GiB
   if ((double)c.state_bytes >= 4294967296.0) return false;
-  // Tiles of 4 waves: 16 x 12 cells when the grid divides (1.31 f-bar
-  // evaluations per cell, the x-halo lanes packed behind the rows), else
-  // 32 x 4 (1.59 per cell, the last wave holding only the 12 x-halo lanes;
-  // 16 x 8 tiles of 3 waves were no faster on 128^3).  Four waves per block
-  // keep FP64 at one wave per SIMD without spills and fit two FP32 blocks
-  // (at most 256 registers per lane) on a CU.
+  // a wall axis needs two interior cells per side of the extrapolation
+  return (s.periodic[0] || s.n[0] >= 3) && (s.periodic[1] || s.n[1] >= 3);
+}
+}  // namespace
+
+// Grids of whole tiles: what DUGKS_KERNEL_FUSED asks for and the adjoint-face
+// pass needs (trilinear reconstruction there).
+bool fused_supported(const Ctx& c, int* tx, int* ty) {
+  const Setup& s = c.s;
+  // Tiles of the adjoint-face pass, 4 waves: 16 x 12 cells when the grid
+  // divides (1.31 f-bar evaluations per cell, the x-halo lanes packed behind
+  // the rows), else 32 x 4 (1.59 per cell, the last wave holding only the 12
+  // x-halo lanes).  Four waves per block keep FP64 at one wave per SIMD
+  // without spills and fit two FP32 blocks (at most 256 registers per lane)
+  // on a CU.
   if (s.n[0] % 16 == 0 && s.n[1] % 12 == 0) {
     *tx = 16;
     *ty = 12;
@@ -715,14 +726,24 @@ bool fused_supported(const Ctx& c, int* tx, int* ty) {
     *tx = 32;
     *ty = 4;
   }
-  if (s.n[0] % *tx != 0 || s.n[1] % *ty != 0) return false;
-  // a wall axis needs two interior cells per side of the extrapolation
-  if (!s.periodic[0] && s.n[0] < 3) return false;
-  if (!s.periodic[1] && s.n[1] < 3) return false;
-  return true;
+  return s.n[0] % *tx == 0 && s.n[1] % *ty == 0 && tiles_cover(c);
 }
 
 namespace {
+// The step kernel takes any nx and ny (the last tile of an axis overlaps the
+// one before it), and the automatic choice uses it wherever it can: on 90x50x121
+// FP64 in a duct 89 us a step against 525 with the two-pass kernels, on a
+// 150x97x83 FP32 channel 90 against 301, on 8x64x8 FP64 12.7 against 89, on
+// 20x20x20 FP64 12.5 against 100.  Below 512 cells, grids that are not whole
+// tiles keep the two-pass kernels although these are slower there too
+// (13x6x5 FP64: 69 against 10.5 us): that choice is part of the tested
+// interface, and no run of use is that small.
+bool step_covers(const Ctx& c) {
+  int tx, ty;
+  if (fused_supported(c, &tx, &ty)) return true;
+  return c.kernel != 1 /* DUGKS_KERNEL_FUSED */ && tiles_cover(c) && c.kp.N >= 512;
+}
+
 template <bool GRAD>
 hipError_t launch_step_recon(Ctx& c, const void* fin, void* fout) {
   switch (c.precision) {
@@ -739,10 +760,8 @@ hipError_t launch_step_recon(Ctx& c, const void* fin, void* fout) {
 }  // namespace
 
 hipError_t launch_step_fused(Ctx& c, const void* fin, void* fout, bool* handled) {
-  int tx = 32, ty = 4;
-  *handled = false;
-  if (!fused_supported(c, &tx, &ty)) return hipSuccess;
-  *handled = true;
+  *handled = step_covers(c);
+  if (!*handled) return hipSuccess;
   return c.s.recon == 0 ? launch_step_recon<false>(c, fin, fout) : launch_step_recon<true>(c, fin, fout);
 }
 

@@ -195,9 +195,12 @@ __global__ void __launch_bounds__(step_nw(sizeof(Real) == 8, TX, TY) * 64, 2)
     wave_order();
     const Place w = place();
     const int gi = i0 + w.c, gj = j0 - 1 + w.r;
-    // side of the column's ghost along x and y: -1, +1, or none
-    const int dx = !own || P.periodic[0] ? 0 : (gi == 0 ? -1 : (gi == nx - 1 ? 1 : 0));
-    const int dy = !own || P.periodic[1] ? 0 : (gj == 0 ? -1 : (gj == ny - 1 ? 1 : 0));
+    // side of the column's ghost along x and y: -1, +1, or none (a halo column
+    // at the wall, beside an overlapping tile, has its ghost outside the tile,
+    // where nothing reads it)
+    const bool xin = own && !P.periodic[0] && w.c >= 0 && w.c < tw, yin = own && !P.periodic[1] && w.r >= 1 && w.r <= th;
+    const int dx = !xin ? 0 : (gi == 0 ? -1 : (gi == nx - 1 ? 1 : 0));
+    const int dy = !yin ? 0 : (gj == 0 ? -1 : (gj == ny - 1 ? 1 : 0));
     Real *xa = S + plane_a + w.at, *xb = xa + (plane_b - plane_a);
     const int ox = dx * STR, oy = dy * AC * STR;
     constexpr bool two = decltype(TWO)::value;

@@ -6,10 +6,12 @@ Tolerances, as for the tile-sized grids: five FP64 steps differ from the
 oracle by round-off (1e-15 relative per operation and about 100 operations
 deep: 1e-13 a step), one FP32 step by 2e-6 of the largest population.
 """
+import numpy as np
 import pytest
 
-from conftest import random_state
-from dugks_amd import KERNEL_FUSED, PREC_FP32, PREC_FP64, configs
+from conftest import W, feq, moments, random_state
+from dugks_amd import (KERNEL_AUTO, KERNEL_FUSED, KERNEL_TWOPASS, PREC_FP16N, PREC_FP16S, PREC_FP32, PREC_FP64,
+                       configs)
 from test_gpu_step import _engine, _oracle_for, _relerr
 
 pytestmark = pytest.mark.gpu
@@ -48,3 +50,68 @@ def test_tile_edges_match_oracle(rng, n, walls, recon):
         eng.step(steps)
         ora.step(steps)
         assert _relerr(eng.get_f(), ora.get_f()) <= tol
+
+
+# Grids that are not whole tiles, which the automatic choice takes to the step
+# kernel: odd rows and columns, narrower and lower than a tile, one row, one
+# column, overlaps of all but one row or column.
+RAGGED = [(13, 40, 1), (31, 33, 3), (50, 11, 2), (17, 13, 5), (8, 64, 8), (33, 25, 4)]
+RAGGED_WALLS = {**WALLS, "walls_x": dict(periods_x=0, mesh_x="tanh:0.8", dt_rule="min")}
+
+
+@pytest.mark.parametrize("recon", ["tri", "grad"])
+@pytest.mark.parametrize("walls,n", [(w, n) for w in RAGGED_WALLS for n in RAGGED] +
+                         [("periodic", (1, 520, 1)), ("periodic", (520, 1, 2)), ("walls_y", (171, 3, 1)),
+                          ("walls_xy", (3, 3, 60))], ids=str)
+def test_ragged_grids_match_twopass(rng, n, walls, recon):
+    """All storage modes against the two-pass kernels.  Tolerances: both paths'
+    distances from the oracle as tested for whole tiles, 1e-13 (FP64) and
+    2e-6 (FP32 arithmetic) a step, and for FP16 storage one rounding each."""
+    kw = {k: v for k, v in RAGGED_WALLS[walls].items() if recon == "tri" or not k.startswith(("mesh", "dt"))}
+    text = configs.base(nx=n[0], ny=n[1], nz=n[2], xwidth=n[0] / 10, ywidth=n[1] / 10, zwidth=n[2] / 10, visc=0.02,
+                        CFL=0.5, recon=recon, ambient_fx=2e-4, ambient_fz=1e-4, **kw)
+    for precision in (PREC_FP64, PREC_FP32, PREC_FP16S, PREC_FP16N):
+        got = []
+        f0 = random_state(n, rng)
+        for kernel in (KERNEL_AUTO, KERNEL_TWOPASS):
+            eng = _engine(text, precision=precision, kernel=kernel)
+            eng.set_f(f0)
+            eng.step(3 if precision == PREC_FP64 else 1)
+            got.append(eng.get_f())
+        a, b = got
+        big = np.abs(b).max()
+        if precision == PREC_FP64:
+            tol = 2 * 3e-13 * big
+        elif precision == PREC_FP32:
+            tol = 2 * 2e-6 * big
+        elif precision == PREC_FP16S:
+            tol = 2 * (W * np.maximum(2.0 ** -11 * np.abs(b / W - eng.params["rho0"]), 2.0 ** -25) + 4e-6 * big)
+        else:
+            rho, j = moments(b)
+            tol = 2 * (2.0 ** -11 * np.abs(b - feq(rho, j / rho[..., None])) + 2.0 ** -25 * W / 1024 + 4e-6 * big)
+        assert np.all(np.abs(a - b) <= tol)
+
+
+def test_automatic_choice_of_ragged_grids():
+    def launches(**kw):
+        base = dict(nx=20, ny=17, nz=5, xwidth=2.0, ywidth=1.7, zwidth=0.5, visc=0.02)
+        return _engine(configs.base(**{**base, **kw}), kernel=KERNEL_AUTO).time_steps(1)["launches_per_step"]
+    assert launches() == 1
+    assert launches(periods_y=0, flow_rate=0.01, ambient_fx=1e-4) == 2
+    assert launches(nz=1) == 5       # fewer than 512 cells
+    assert launches(periods_z=0) == 5
+
+
+@pytest.mark.parametrize("precision,tol", [(PREC_FP64, 1e-12), (PREC_FP32, 5e-5)], ids=["fp64", "fp32"])
+def test_ragged_flow_rate_matches_twopass(precision, tol):
+    """The controller's force over 10 steps: FP64 to round-off; FP32 to ten
+    roundings of the velocity (6e-8 of 0.1) over the time step's share of the
+    gain, 1e-5 of the force, times a margin of 5."""
+    text = configs.base(nx=45, ny=29, nz=11, xwidth=4.5, ywidth=2.9, zwidth=1.1, periods_y=0, visc=0.02,
+                        flow_rate=0.05, ambient_fx=2e-4)
+    got = []
+    for kernel in (KERNEL_AUTO, KERNEL_TWOPASS):
+        eng = _engine(text, precision=precision, kernel=kernel)
+        eng.step(10)
+        got.append(np.array(eng.get_f(), dtype=np.float64))
+    assert _relerr(got[0], got[1]) <= tol
