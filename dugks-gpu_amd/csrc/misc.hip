@@ -357,28 +357,38 @@ __global__ void __launch_bounds__(kRedThreads) k_stats(KParams P, const Store* _
 }
 
 // Per row: the profile sums; globally: rho, u, v, w sums, min, max.  out:
-// [np][9] row sums, then [4] global sums, [4] min, [4] max.
+// [np][9] row sums, then [4] global sums, [4] min, [4] max.  The last block
+// takes the global values, the others a row sum per thread: a chain of
+// dependent loads is kStatBlocks long, or a 256th of the slots (one block with
+// four threads walking all slots took 376 us for 192 rows; this takes 8).
 __global__ void __launch_bounds__(kRedThreads) k_stats_finish(const double* __restrict__ part,
                                                               const double* __restrict__ mm, int np,
                                                               double* __restrict__ out) {
-  for (int m = threadIdx.x; m < np; m += kRedThreads)
-    for (int q = 0; q < 9; q++) {
-      double a = 0;
-      for (int b = 0; b < kStatBlocks; b++) a += part[((long long)m * kStatBlocks + b) * kStatSums + q];
-      out[(long long)m * 9 + q] = a;
-    }
-  if (threadIdx.x < 4) {
-    const int q = threadIdx.x;
-    double a = 0, lo = 1e300, hi = -1e300;
-    for (long long s = 0; s < (long long)np * kStatBlocks; s++) {
-      a += part[s * kStatSums + 9 + q];
-      lo = fmin(lo, mm[s * 8 + q]);
-      hi = fmax(hi, mm[s * 8 + 4 + q]);
-    }
-    out[(long long)np * 9 + q] = a;
-    out[(long long)np * 9 + 4 + q] = lo;
-    out[(long long)np * 9 + 8 + q] = hi;
+  if (blockIdx.x + 1 < gridDim.x) {
+    const long long t = (long long)blockIdx.x * kRedThreads + threadIdx.x;
+    if (t >= (long long)np * 9) return;
+    const long long m = t / 9;
+    const int q = (int)(t % 9);
+    double a = 0;
+    for (int b = 0; b < kStatBlocks; b++) a += part[(m * kStatBlocks + b) * kStatSums + q];
+    out[t] = a;
+    return;
   }
+  double all[12];
+  int ops[12];
+  for (int q = 0; q < 12; q++) {
+    ops[q] = q / 4;
+    all[q] = q < 4 ? 0.0 : (q < 8 ? 1e300 : -1e300);
+  }
+  for (long long s = threadIdx.x; s < (long long)np * kStatBlocks; s += kRedThreads)
+    for (int q = 0; q < 4; q++) {
+      all[q] += part[s * kStatSums + 9 + q];
+      all[4 + q] = fmin(all[4 + q], mm[s * 8 + q]);
+      all[8 + q] = fmax(all[8 + q], mm[s * 8 + 4 + q]);
+    }
+  block_reduce<12, kRedThreads>(all, ops);
+  if (threadIdx.x == 0)
+    for (int q = 0; q < 12; q++) out[(long long)np * 9 + q] = all[q];
 }
 
 template <class Store>
@@ -388,7 +398,8 @@ hipError_t stats_t(Ctx& c, const void* f, int pa, double* scratch, double* out) 
   double* mm = scratch + (size_t)np * kStatBlocks * kStatSums;
   hipLaunchKernelGGL((k_stats<Store>), dim3(kStatBlocks, np), dim3(kRedThreads), 0, c.stream, c.kp,
                      static_cast<const Store*>(f), pa, part, mm);
-  hipLaunchKernelGGL(k_stats_finish, dim3(1), dim3(kRedThreads), 0, c.stream, part, mm, np, out);
+  const unsigned row_blocks = (unsigned)(((long long)np * 9 + kRedThreads - 1) / kRedThreads);
+  hipLaunchKernelGGL(k_stats_finish, dim3(row_blocks + 1), dim3(kRedThreads), 0, c.stream, part, mm, np, out);
   return hipGetLastError();
 }
 

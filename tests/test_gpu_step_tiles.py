@@ -115,3 +115,23 @@ def test_ragged_flow_rate_matches_twopass(precision, tol):
         eng.step(10)
         got.append(np.array(eng.get_f(), dtype=np.float64))
     assert _relerr(got[0], got[1]) <= tol
+
+
+@pytest.mark.parametrize("nx", [1, 28, 29, 300], ids=lambda v: f"rows{v}")
+def test_planar_statistics_over_row_counts(rng, nx):
+    """Row sums and the global mean, minimum and maximum where the last block of
+    row sums is nearly full (9 x 28 of 256 threads), just over, and with several
+    slots per thread (300 rows).  Means of O(1) values in FP64: 1e-12."""
+    eng = _engine(configs.base(nx=nx, ny=3, nz=200, xwidth=0.1 * nx, ywidth=0.3, zwidth=20.0, visc=0.02))
+    eng.set_f(random_state(eng.shape, rng))
+    prof, diag = eng.statistics()
+    rho, ux, uy, uz = eng.macro()
+    mean = lambda a: a.mean(axis=(0, 1))
+    U, V, Wv = mean(ux), mean(uy), mean(uz)
+    expect = np.stack([U, V, Wv, mean(ux * uz) - U * Wv, mean(ux * uy) - U * V, mean(uy * uz) - V * Wv,
+                       mean(ux * ux) - U * U, mean(uy * uy) - V * V, mean(uz * uz) - Wv * Wv], axis=1)
+    assert np.abs(prof - expect).max() <= 1e-12
+    fields = (rho, ux, uy, uz)
+    assert np.abs(diag[0:4] - [a.mean() for a in fields]).max() <= 1e-12
+    assert np.abs(diag[4:8] - [a.min() for a in fields]).max() <= 1e-15
+    assert np.abs(diag[8:12] - [a.max() for a in fields]).max() <= 1e-15
