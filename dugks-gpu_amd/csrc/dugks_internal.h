@@ -50,6 +50,25 @@ struct KParams {
 
 struct Ctx;
 
+// The number of z-chunks for `tiles` columns of nz planes, `slots` workgroups
+// resident at once and a prologue that costs as much as `prologue` planes: the
+// least (rounds of workgroups) x (planes of the longest chunk + prologue), the
+// fewest chunks at a tie, from `first` chunks on.
+inline int plan_z_chunks(long long tiles, int nz, int slots, double prologue, int first = 1) {
+  int best = first;
+  double least = 0;
+  for (int nc = first; nc <= nz; nc++) {
+    const double rounds = (double)((tiles * nc + slots - 1) / slots);
+    const double cost = rounds * ((nz + nc - 1) / nc + prologue);
+    if (nc == first || cost < least * (1 - 1e-9)) {
+      best = nc;
+      least = cost;
+    }
+    if (rounds * (1 + prologue) > least) break;  // only dearer from here
+  }
+  return best;
+}
+
 // Launchers (implemented in the .hip files; all stream-ordered).
 hipError_t launch_step_twopass(Ctx& c, const void* fin, void* fout);
 hipError_t launch_fbar_ghosts(Ctx& c, const void* fin, void* fbx);

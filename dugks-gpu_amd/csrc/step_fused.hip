@@ -593,17 +593,17 @@ __global__ void __launch_bounds__(256) k_flow_finish(const double* partial, int 
   }
 }
 
-// z-chunk length of the adjoint-face pass: 32 planes (a chunk recomputes
-// f-bar+ of the two planes before it; 128 planes were 0.7 % slower on
-// 256x192x256), halved down to 8 while the grid has fewer tiles than one round
-// of resident workgroups on the 256 CUs.
+// z-chunk length of the adjoint-face pass (plan_z_chunks; a chunk recomputes
+// f-bar+ of the two planes before it, about as long as one plane).  At most
+// 32 planes: several rounds even out the finish (256x192x256 FP32: 128 planes
+// 0.3 % slower).  On 64x64x32 FP64 (32 tiles, one workgroup per CU): 51 us
+// with 4-plane chunks, 86 with 8.
 int blocks_per_cu(bool fp64, int TX, int TY) { return fp64 || Tile_nt(TX, TY) > 256 ? 1 : 2; }
 int z_chunk(const Ctx& cx, int TX, int TY) {
   const long long cols = (long long)(cx.kp.n[0] / TX) * (cx.kp.n[1] / TY);
-  const int per_cu = blocks_per_cu(cx.precision == 0, TX, TY);
-  int tz = 32;
-  while (tz > 8 && cols * ((cx.kp.n[2] + tz - 1) / tz) < per_cu * 256) tz /= 2;
-  return tz;
+  const int nz = cx.kp.n[2], nc = plan_z_chunks(cols, nz, 256 * blocks_per_cu(cx.precision == 0, TX, TY), 1.2,
+                                                  (cx.kp.n[2] + 31) / 32);
+  return (nz + nc - 1) / nc;
 }
 
 // The step's tiles and z-chunks.
@@ -617,26 +617,15 @@ struct StepPlan {
 // on 16 x 12, two workgroups per CU: 0.80 against 0.68 ms on the 256x192x256
 // channel.)
 // Each of a chunk's planes takes the same time whatever the grid, and its
-// prologue about 2.2 planes' time (f-bar+ of two planes and one face).  The
-// number of chunks is the one with the least (rounds of 256 workgroups) x
-// (planes of the longest chunk + 2.2), the fewest at a tie.  Measured on
-// 64x64x32 FP64 (24 tiles): 8 chunks 30.5 us, 16 36.6, 32 39.4; on 64x72x32
-// FP32 (12 tiles): 8 chunks 28.0 us, 16 20.3, 32 24.3.
+// prologue about 2.2 planes' time (f-bar+ of two planes and one face); the
+// number of chunks follows from that (plan_z_chunks).  Measured on 64x64x32
+// FP64 (24 tiles): 8 chunks 30.5 us, 16 36.6, 32 39.4; on 64x72x32 FP32 (12
+// tiles): 8 chunks 28.0 us, 16 20.3, 32 24.3.
 template <int TX, int TY>
 StepPlan plan_tiles(const Setup& s) {
   const long long tiles = (long long)((s.n[0] + TX - 1) / TX) * ((s.n[1] + TY - 1) / TY);
-  StepPlan best{1, tiles};
-  double least = 0;
-  for (int nc = 1; nc <= s.n[2]; nc++) {
-    const long long rounds = (tiles * nc + 255) / 256;
-    const double cost = (double)rounds * ((s.n[2] + nc - 1) / nc + 2.2);
-    if (nc == 1 || cost < least * (1 - 1e-9)) {
-      best = {nc, tiles * nc};
-      least = cost;
-    }
-    if ((double)rounds * 3.2 > least) break;  // only dearer from here
-  }
-  return best;
+  const int nc = plan_z_chunks(tiles, s.n[2], 256, 2.2);
+  return {nc, tiles * nc};
 }
 StepPlan step_plan(const Setup& s, int precision) {
   return precision == 0 ? plan_tiles<16, 12>(s) : plan_tiles<32, 12>(s);
