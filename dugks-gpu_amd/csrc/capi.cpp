@@ -294,7 +294,8 @@ hipError_t build_params(Ctx& c) {
   P.famb_dev = c.famb_dev;
   c.red_len = reduction_scratch_doubles() + 64;
   if ((e = c.alloc((void**)&c.red, c.red_len * sizeof(double))) != hipSuccess) return e;
-  c.flow_partial_len = (size_t)step_fused_blocks(s, c.precision);
+  c.plan = step_plan(s, c.precision);
+  c.flow_partial_len = (size_t)c.plan.nblocks;
   if ((e = c.alloc((void**)&c.flow_partial, c.flow_partial_len * sizeof(double))) != hipSuccess) return e;
   return hipSuccess;
 }

@@ -69,12 +69,19 @@ inline int plan_z_chunks(long long tiles, int nz, int slots, double prologue, in
   return best;
 }
 
+// The step kernel's tiles and how their planes are dealt to the workgroups.
+struct StepPlan {
+  int rows = 0;           // tile height: 12, 8 or 4 (32 columns wide with FP32 arithmetic, 16 with FP64)
+  int nchunk = 0;         // z-chunks of every tile
+  int len = 0;            // > 0: of len planes each, and runs over the planes behind them (k_step, RUNS)
+  long long nblocks = 0;  // workgroups (each leaves one bulk-velocity partial)
+};
+StepPlan step_plan(const Setup& s, int precision);
+
 // Launchers (implemented in the .hip files; all stream-ordered).
 hipError_t launch_step_twopass(Ctx& c, const void* fin, void* fout);
 hipError_t launch_fbar_ghosts(Ctx& c, const void* fin, void* fbx);
 hipError_t launch_step_fused(Ctx& c, const void* fin, void* fout, bool* handled);
-// workgroups of that launch (each leaves one bulk-velocity partial)
-long long step_fused_blocks(const Setup& s, int precision);
 // Adjoint-face pass of the fused kernel (see adjoint.hip); handled = false
 // when the fused kernel does not cover the configuration.  Face record
 // formats: kFacesFull, the 19 reconstructed-value cotangents per face, lam'
@@ -243,7 +250,8 @@ struct Ctx {
   bool timing = false;
   std::vector<float> kernel_ms;
   int launches_per_step = 0;
-  // fused kernel: the per-block flow-rate partial sums
+  // step kernel: its plan and the per-block flow-rate partial sums
+  StepPlan plan;
   double* flow_partial = nullptr;
   size_t flow_partial_len = 0;
   // the step kernels leave the flow-rate controller alone (the adjoint's

@@ -46,6 +46,7 @@
 //   FP64          1.185 / 1.329     (1.88  / 1.92)
 //   FP16 dev.     0.649 / 0.710     (0.729 / 0.797)
 //   FP16 non-eq.  0.717 / 0.772     (0.966 / 0.964)
+#include <algorithm>
 #include "device_common.h"
 
 namespace dugks {
@@ -606,35 +607,73 @@ int z_chunk(const Ctx& cx, int TX, int TY) {
   return (nz + nc - 1) / nc;
 }
 
-// The step's tiles and z-chunks.
-struct StepPlan {
-  int nchunk;         // z-chunks of every tile
-  long long nblocks;  // workgroups
-};
-// Tiles of 32 x 12 cells with FP32 arithmetic and 16 x 12 with FP64: the
-// tallest whose two LDS planes and face values fit 160 KB, one workgroup of
+}  // namespace
+
+// Tiles of 32 x 12 cells with FP32 arithmetic and 16 x 12 with FP64 are the
+// tallest whose two LDS planes and face values fit 160 KB: one workgroup of
 // eight waves per CU, f-bar+ formed on 1.24 and 1.31 times the cells.  (FP32
 // on 16 x 12, two workgroups per CU: 0.80 against 0.68 ms on the 256x192x256
 // channel.)
-// Each of a chunk's planes takes the same time whatever the grid, and its
-// prologue about 2.2 planes' time (f-bar+ of two planes and one face); the
-// number of chunks follows from that (plan_z_chunks).  Measured on 64x64x32
-// FP64 (24 tiles): 8 chunks 30.5 us, 16 36.6, 32 39.4; on 64x72x32 FP32 (12
-// tiles): 8 chunks 28.0 us, 16 20.3, 32 24.3.
-template <int TX, int TY>
-StepPlan plan_tiles(const Setup& s) {
-  const long long tiles = (long long)((s.n[0] + TX - 1) / TX) * ((s.n[1] + TY - 1) / TY);
-  const int nc = plan_z_chunks(tiles, s.n[2], 256, 2.2);
-  return {nc, tiles * nc};
-}
+// A plane takes the same time whatever the grid, and the start of a tile or
+// chunk about 2.2 planes' time (f-bar+ of two planes and one face).  So a
+// round of 256 workgroups costs the planes of the longest one + 2.2, and the
+// plan is the cheapest of:
+//  - z-chunks of every tile (plan_z_chunks).  64x64x32 FP64 (24 tiles): 8
+//    chunks 30.5 us, 16 36.6, 32 39.4; 64x72x32 FP32 (12 tiles): 8 chunks
+//    28.0 us, 16 20.3, 32 24.3;
+//  - the same with lower tiles, whose plane takes 0.88 (8 rows) or 0.62 to
+//    0.66 (4 rows) of the time: 8 rows where they fill more CUs (64x64x32 FP64
+//    25.2 us against 28.0), 4 rows where a workgroup has a single plane
+//    (8x64x8 FP64 10.0 against 12.7 us, 20x20x20 FP64 9.5 against 12.5);
+//    elsewhere they lose (90x50x121 FP64 88.7, 96.9 and 131 us);
+//  - full chunks and runs over what they leave, in one round, where no chunk
+//    count fills the last round: 128^3 FP64 (88 tiles: 2 chunks of 46 planes
+//    each, and 80 workgroups with 39 or 40 planes of the rest, against 3 rounds
+//    of 16 planes) 242 us against 251, FP32 (44 tiles: 5 chunks of 23, 36
+//    workgroups with 16, against 26 planes) 115 against 123, FP16
+//    non-equilibrium storage 142 against 158.  (Runs over all planes put
+//    neighbouring tiles out of step, so that their halos miss L2: 263 us in
+//    FP64 and 137 in FP32.)  Only where the model gives 7 %: at 5 % a
+//    150x97x83 FP32 channel gained 2 % and a 90x50x121 FP64 duct lost 3.
+// Gradient reconstruction has only the first form (its kernel has no registers
+// left for the runs).
 StepPlan step_plan(const Setup& s, int precision) {
-  return precision == 0 ? plan_tiles<16, 12>(s) : plan_tiles<32, 12>(s);
+  const int tx = precision == 0 ? 16 : 32, nz = s.n[2];
+  const double start = 2.2;
+  StepPlan best{};
+  double least = 0;
+  for (const int rows : {12, 8, 4}) {
+    const double plane = rows == 12 ? 1.0 : (rows == 8 ? 0.88 : (precision == 0 ? 0.62 : 0.66));
+    const long long tiles = (long long)((s.n[0] + tx - 1) / tx) * ((s.n[1] + rows - 1) / rows);
+    const int nc = plan_z_chunks(tiles, nz, 256, start);
+    const double cost = plane * (double)((tiles * nc + 255) / 256) * ((nz + nc - 1) / nc + start);
+    if (rows == 12 || cost < 0.97 * least) {
+      best = {rows, nc, 0, tiles * nc};
+      least = cost;
+    }
+    if (s.recon != 0) return best;
+    if (rows != 12) continue;
+    const double chunks = 0.93 * least;
+    for (int m = 1; m * tiles < 256; m++)
+      for (int len = 1; m * len < nz && len + start < chunks; len++) {
+        const int rest = nz - m * len;
+        const long long nb = 256 - m * tiles, run = (rest * tiles + nb - 1) / nb;
+        const double cost_runs = std::max(len + start, run + start * ((run + rest - 2) / rest + 1));
+        // (at a tie more chunks, which keep neighbouring tiles in step)
+        if (cost_runs < chunks && (cost_runs < least || (best.len > 0 && cost_runs <= least))) {
+          best = {12, m, len, 256};
+          least = cost_runs;
+        }
+      }
+  }
+  return best;
 }
 
-template <class Real, class Store, int TX, int TY, bool GRAD>
-hipError_t run_step(Ctx& cx, const void* fin, void* fout) {
+namespace {
+
+template <class Real, class Store, int TX, int TY, bool GRAD, bool RUNS>
+hipError_t run_step(Ctx& cx, const void* fin, void* fout, const StepPlan& plan) {
   using T = StepTile<Real, TX, TY, GRAD>;
-  const StepPlan plan = step_plan(cx.s, cx.precision);
   double* partial = nullptr;
   const bool flow = cx.s.flow_rate != 0 && !cx.flow_frozen;
   if (flow) {
@@ -642,8 +681,9 @@ hipError_t run_step(Ctx& cx, const void* fin, void* fout) {
     partial = cx.flow_partial;
   }
   if (cx.timing) hipEventRecord(cx.tev[0], cx.stream);
-  hipLaunchKernelGGL((k_step<Real, Store, TX, TY, GRAD>), dim3((unsigned)plan.nblocks), dim3(T::NT), 0, cx.stream,
-                     cx.kp, static_cast<const Store*>(fin), static_cast<Store*>(fout), plan.nchunk, partial);
+  hipLaunchKernelGGL((k_step<Real, Store, TX, TY, GRAD, RUNS>), dim3((unsigned)plan.nblocks), dim3(T::NT), 0, cx.stream,
+                     cx.kp, static_cast<const Store*>(fin), static_cast<Store*>(fout), plan.nchunk, plan.len,
+                     partial);
   if (cx.timing) hipEventRecord(cx.tev[1], cx.stream);
   if (flow) {
     const Setup& s = cx.s;
@@ -733,28 +773,32 @@ bool step_covers(const Ctx& c) {
   return c.kernel != 1 /* DUGKS_KERNEL_FUSED */ && tiles_cover(c) && c.kp.N >= 512;
 }
 
-template <bool GRAD>
-hipError_t launch_step_recon(Ctx& c, const void* fin, void* fout) {
-  switch (c.precision) {
-    case 0:
-      return run_step<double, double, 16, 12, GRAD>(c, fin, fout);
-    case 1:
-      return run_step<float, float, 32, 12, GRAD>(c, fin, fout);
-    case 2:
-      return run_step<float, __half, 32, 12, GRAD>(c, fin, fout);
-    default:
-      return run_step<float, NeqHalf, 32, 12, GRAD>(c, fin, fout);
-  }
+template <class Real, class Store>
+hipError_t launch_step_mode(Ctx& c, const void* fin, void* fout) {
+  constexpr int TX = sizeof(Real) == 8 ? 16 : 32;
+  const StepPlan& plan = c.plan;
+  if (c.s.recon != 0) return run_step<Real, Store, TX, 12, true, false>(c, fin, fout, plan);
+  if (plan.len > 0) return run_step<Real, Store, TX, 12, false, true>(c, fin, fout, plan);
+  if (plan.rows == 12) return run_step<Real, Store, TX, 12, false, false>(c, fin, fout, plan);
+  if (plan.rows == 8) return run_step<Real, Store, TX, 8, false, false>(c, fin, fout, plan);
+  return run_step<Real, Store, TX, 4, false, false>(c, fin, fout, plan);
 }
 }  // namespace
 
 hipError_t launch_step_fused(Ctx& c, const void* fin, void* fout, bool* handled) {
   *handled = step_covers(c);
   if (!*handled) return hipSuccess;
-  return c.s.recon == 0 ? launch_step_recon<false>(c, fin, fout) : launch_step_recon<true>(c, fin, fout);
+  switch (c.precision) {
+    case 0:
+      return launch_step_mode<double, double>(c, fin, fout);
+    case 1:
+      return launch_step_mode<float, float>(c, fin, fout);
+    case 2:
+      return launch_step_mode<float, __half>(c, fin, fout);
+    default:
+      return launch_step_mode<float, NeqHalf>(c, fin, fout);
+  }
 }
-
-long long step_fused_blocks(const Setup& s, int precision) { return step_plan(s, precision).nblocks; }
 
 bool adjoint_faces_fused_covers(const Ctx& c) {
   int tx = 32, ty = 4;

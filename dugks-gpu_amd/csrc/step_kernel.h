@@ -34,11 +34,15 @@ struct StepTile {
 };
 
 // One DUGKS step fin -> fout (see the top of step_fused.hip).  The grid is
-// one-dimensional: nchunk z-chunks of gx gy tiles.
-template <class Real, class Store, int TX, int TY, bool GRAD>
+// one-dimensional: nchunk z-chunks of gx gy tiles.  RUNS: chunks of `len`
+// planes, which leave the last nz - nchunk len planes of every tile; these, one
+// tile after the other, are dealt in equal runs to the workgroups behind, and
+// such a workgroup goes from the planes of one tile to those of the next.  (A
+// template argument: the loop over the runs costs registers.)
+template <class Real, class Store, int TX, int TY, bool GRAD, bool RUNS>
 __global__ void __launch_bounds__(step_nw(sizeof(Real) == 8, TX, TY) * 64, 2)
     k_step(KParams P, const Store* __restrict__ fin, Store* __restrict__ fout, int nchunk,
-           double* __restrict__ partial) {
+           int len, double* __restrict__ partial) {
   using T = StepTile<Real, TX, TY, GRAD>;
   constexpr bool PAIR = T::PAIR;
   constexpr int NQ = T::NQ, NX = T::NX, AC = T::AC, STR = T::STR, FS = T::FS, UNIT = T::UNIT;
@@ -57,17 +61,22 @@ __global__ void __launch_bounds__(step_nw(sizeof(Real) == 8, TX, TY) * 64, 2)
   // contiguous run of tiles (x fastest), so that tiles whose halos overlap
   // share an L2 and run at about the same time
   const int gx = (nx + TX - 1) / TX, gy = (ny + TY - 1) / TY;
-  const int ntiles = gx * gy * nchunk;
-  const int b = blockIdx.x, xcd = b % kXcds;
-  const int tt = xcd * (ntiles / kXcds) + min(xcd, ntiles % kXcds) + b / kXcds;
-  const int bx = tt % gx, by = (tt / gx) % gy, bz = tt / (gx * gy);
-  // the last tile of an axis that TX or TY does not divide starts early and
-  // overlaps the one before it; the first cx0 columns and ry0 rows of it are
-  // the other tile's to store
-  const int tw = min(TX, nx), th = min(TY, ny);  // columns and rows of a tile
-  const int i0 = min(bx * TX, nx - tw), j0 = min(by * TY, ny - th);
-  const int cx0 = bx * TX - i0, ry0 = by * TY - j0;
-  const int z0 = (int)((long long)bz * nz / nchunk), zend = (int)((long long)(bz + 1) * nz / nchunk);
+  const int nblocks = (int)gridDim.x, b = blockIdx.x, xcd = b % kXcds;
+  const int tt = xcd * (nblocks / kXcds) + min(xcd, nblocks % kXcds) + b / kXcds;
+  // the workgroup's planes q0..q1-1, plane zb + z of tile k counted as k per + z
+  int q0, q1, per = nz, zb = 0;
+  const int tiles = gx * gy;
+  if (!RUNS || tt < tiles * nchunk) {
+    const int tile = tt % tiles, bz = tt / tiles;
+    q0 = tile * nz + (RUNS ? bz * len : (int)((long long)bz * nz / nchunk));
+    q1 = RUNS ? q0 + len : tile * nz + (int)((long long)(bz + 1) * nz / nchunk);
+  } else {
+    zb = nchunk * len;
+    per = nz - zb;
+    const long long k = tt - tiles * nchunk, nk = nblocks - tiles * nchunk, planes = (long long)tiles * per;
+    q0 = (int)(k * planes / nk);
+    q1 = (int)((k + 1) * planes / nk);
+  }
   const unsigned N = (unsigned)P.N, nxy = (unsigned)nx * (unsigned)ny;
   const unsigned span = (unsigned)state_bytes<Store>((unsigned long long)P.N);
   const StateBuf<Store> bin(fin, span), bout(fout, span);
@@ -91,9 +100,46 @@ __global__ void __launch_bounds__(step_nw(sizeof(Real) == 8, TX, TY) * 64, 2)
     r = v % (TY + 2);
     c = v < TY + 2 ? -1 : TX;
   }
+  const int tw = min(TX, nx), th = min(TY, ny);  // columns and rows of a tile
   // on an axis shorter than the tile the far halo is at c = tw, r = th + 1
   const bool active = u < T::NSLOT && c <= tw && r <= th + 1;
   const bool interior = active && r >= 1 && r <= th && c >= 0 && c < tw;
+  auto sign = [](int half) { return half ? Real(-1) : Real(1); };
+
+  // uniform parameters in scalar registers; the lane's frame turns the sign
+  // of the force terms, of the c_z = +1 slots' z weights and of c dt/d
+  Real F0[3];
+  ambient_force<Real>(P, F0);
+  const Real F[3] = {uniform(F0[0]), uniform(F0[1]), uniform(F0[2])};
+  const Real fw1 = uniform((Real)P.fw1), fw2 = uniform((Real)P.fw2), bw2 = uniform((Real)P.bw2);
+  const Real hdt = uniform((Real)P.hdt), hh = uniform(Real(0.5) * (Real)P.hdt), fw0 = uniform((Real)P.fw0),
+             bw0 = uniform((Real)P.bw0);
+  auto tz = [&](int idx) { return tabv<Real>(P, 2, idx); };
+  // z weights (uniform axis): tangential (toward p-1 for c_z > 0, p+1 for
+  // c_z < 0: the same), normal toward p+1 for c_z = 0, +1, -1
+  const Real wzt = uniform(tz(9 + 6)), wzn0 = uniform(tz(9 + 1));
+  const Real wznp = uniform(tz(9 + 2)), wznm = uniform(tz(9 + 0)), updz = uniform(tz(9 + 8));
+  Real gin[3] = {Real(0), Real(0), Real(0)}, gtn[3] = {Real(0), Real(0), Real(0)};
+  if constexpr (GRAD) {
+    for (int a = 0; a < 3; a++) {
+      gin[a] = uniform((Real)(1.0 / P.du[a]));
+      gtn[a] = uniform((Real)(0.5 / P.du[a]));
+    }
+  }
+  double flow = 0;
+  const int as = P.flow_axis;
+
+  for (int q = q0; q < q1;) {  // (the body is one run, not indented)
+  const int tile = q / per, z0 = zb + q - tile * per, zend = RUNS ? min(zb + per, z0 + q1 - q) : z0 + q1 - q0;
+  // the next run's first barrier: this run's last plane still reads the weights
+  if (RUNS && q != q0) __syncthreads();
+  q += zend - z0;
+  const int bx = tile % gx, by = tile / gx;
+  // the last tile of an axis that TX or TY does not divide starts early and
+  // overlaps the one before it; the first cx0 columns and ry0 rows of it are
+  // the other tile's to store
+  const int i0 = min(bx * TX, nx - tw), j0 = min(by * TY, ny - th);
+  const int cx0 = bx * TX - i0, ry0 = by * TY - j0;
   const bool stored = interior && c >= cx0 && r > ry0;
   int gi = i0 + c, gj = j0 - 1 + r;
   if (P.periodic[0]) gi = (gi + nx) % nx;
@@ -119,28 +165,6 @@ __global__ void __launch_bounds__(step_nw(sizeof(Real) == 8, TX, TY) * 64, 2)
     q.fat = here(fbase0);
     return q;
   };
-  auto sign = [](int half) { return half ? Real(-1) : Real(1); };
-
-  // uniform parameters in scalar registers; the lane's frame turns the sign
-  // of the force terms, of the c_z = +1 slots' z weights and of c dt/d
-  Real F0[3];
-  ambient_force<Real>(P, F0);
-  const Real F[3] = {uniform(F0[0]), uniform(F0[1]), uniform(F0[2])};
-  const Real fw1 = uniform((Real)P.fw1), fw2 = uniform((Real)P.fw2), bw2 = uniform((Real)P.bw2);
-  const Real hdt = uniform((Real)P.hdt), hh = uniform(Real(0.5) * (Real)P.hdt), fw0 = uniform((Real)P.fw0),
-             bw0 = uniform((Real)P.bw0);
-  auto tz = [&](int idx) { return tabv<Real>(P, 2, idx); };
-  // z weights (uniform axis): tangential (toward p-1 for c_z > 0, p+1 for
-  // c_z < 0: the same), normal toward p+1 for c_z = 0, +1, -1
-  const Real wzt = uniform(tz(9 + 6)), wzn0 = uniform(tz(9 + 1));
-  const Real wznp = uniform(tz(9 + 2)), wznm = uniform(tz(9 + 0)), updz = uniform(tz(9 + 8));
-  Real gin[3] = {Real(0), Real(0), Real(0)}, gtn[3] = {Real(0), Real(0), Real(0)};
-  if constexpr (GRAD) {
-    for (int a = 0; a < 3; a++) {
-      gin[a] = uniform((Real)(1.0 / P.du[a]));
-      gtn[a] = uniform((Real)(0.5 / P.du[a]));
-    }
-  }
   // Weights of the tile's columns and rows, copied once into LDS, in each
   // half's frame.  Value k: 0-2 the -face normal weight toward the upper cell
   // of the slots with c = -1, 0, +1; 3-4 the tangential shift weights for c =
@@ -452,8 +476,7 @@ __global__ void __launch_bounds__(step_nw(sizeof(Real) == 8, TX, TY) * 64, 2)
     return 0;
   };
   Real fbm[NM], fbc[NQ], fbn[NQ], gc[NQ], gn[NQ], zm[NX];
-  double flow = 0;
-  const int as = P.flow_axis;
+  double run_flow = 0;
   // f of the own column one plane ahead of its f-bar+
   Raw fpre;
   load_own((z0 + 1) % nz, fpre);
@@ -578,7 +601,7 @@ __global__ void __launch_bounds__(step_nw(sizeof(Real) == 8, TX, TY) * 64, 2)
         un[0] = cell_diff<PAIR>(as == 0 ? jn[0] : (as == 1 ? jn[1] : jn[2])) * rcp_real(rr);
       }
       // bulk velocity of the new state for the flow-rate controller
-      if (partial && stored) flow += (double)(!kNeq || as == 0 ? un[0] : (as == 1 ? un[1] : un[2]));
+      if (partial && stored) run_flow += (double)(!kNeq || as == 0 ? un[0] : (as == 1 ? un[1] : un[2]));
     }
     // Stores without a branch (lanes that store nothing address the end of
     // the array): the compiler then knows how many stores follow the loads
@@ -633,11 +656,16 @@ __global__ void __launch_bounds__(step_nw(sizeof(Real) == 8, TX, TY) * 64, 2)
   }
 
   if (partial) {
-    // fixed-order block reduction of the flow sums; every column of the tile
-    // has the same z width (z is uniform here)
+    // every column of the tile has the same z width (z is uniform here)
     const Place w = place();
-    double v[1] = {0.0};
-    if (stored && !w.half) v[0] = flow * (P.wd[0][i0 + w.c + 1] * P.wd[1][j0 + w.r] * P.wd[2][1]);
+    if (stored && !w.half) flow += run_flow * (P.wd[0][i0 + w.c + 1] * P.wd[1][j0 + w.r] * P.wd[2][1]);
+  }
+  if constexpr (!RUNS) break;
+  }
+
+  if (partial) {
+    // fixed-order block reduction of the flow sums
+    double v[1] = {flow};
     constexpr int kSum[1] = {0};
     block_reduce<1, T::NT>(v, kSum);
     if (t == 0) partial[tt] = v[0];

@@ -166,3 +166,26 @@ def test_adjoint_step_over_chunk_counts(rng, precision, nz):
     want = (J[0] - J[1]) / 2e-6
     size = np.linalg.norm(lam) * np.linalg.norm(df)
     assert abs(got - want) <= (1e-8 if precision == PREC_FP64 else 1e-6) * size
+
+
+@pytest.mark.parametrize("precision,n,tol", [
+    (PREC_FP64, (82, 39, 41), 6e-13), (PREC_FP64, (51, 50, 49), 6e-13),      # chunks of 4 planes, runs over the rest
+    (PREC_FP32, (102, 61, 41), 4e-6), (PREC_FP32, (38, 54, 126), 4e-6),
+    (PREC_FP64, (48, 40, 20), 6e-13), (PREC_FP64, (64, 64, 32), 6e-13),      # tiles of 12 and of 8 rows
+    (PREC_FP32, (64, 64, 32), 4e-6), (PREC_FP32, (20, 20, 20), 4e-6)])       # of 8 rows, of 4 rows
+@pytest.mark.parametrize("walls", ["periodic", "walls_y", "walls_x"])
+def test_plans_match_twopass(rng, precision, n, tol, walls):
+    """Every form of the step's plan, with the flow-rate controller where there
+    are walls (its sums run over the same tiles), against the two-pass kernels:
+    3 FP64 steps of 1e-13, one FP32 step of 2e-6, on both sides."""
+    kw = dict(RAGGED_WALLS[walls], **({"flow_rate": 0.02} if walls != "periodic" else {}))
+    text = configs.base(nx=n[0], ny=n[1], nz=n[2], xwidth=n[0] / 10, ywidth=n[1] / 10, zwidth=n[2] / 10, visc=0.02,
+                        CFL=0.5, ambient_fz=1e-4, flow_axis=2, **kw)
+    f0 = random_state(n, rng)
+    got = []
+    for kernel in (KERNEL_AUTO, KERNEL_TWOPASS):
+        eng = _engine(text, precision=precision, kernel=kernel)
+        eng.set_f(f0)
+        eng.step(3 if precision == PREC_FP64 else 1)
+        got.append(eng.get_f())
+    assert _relerr(*got) <= tol
