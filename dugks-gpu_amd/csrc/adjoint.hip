@@ -17,8 +17,10 @@
 //      reconstructed values (in the arithmetic type);
 //   3. the gather: S3^T of those values over the faces whose stencil
 //      contains each cell (the wall ghost extrapolation folded in), then S5^T
-//      and S1^T.  k_adj_cells_z (32 x 8 column tiles)
-//      stages each plane of face cotangents in LDS and marches along z;
+//      and S1^T.  k_adj_cells_z
+//      stages each plane of face cotangents in LDS and marches along z (its
+//      faces come from the fused pass as records of A and B alone, and it
+//      forms lam_ft from lam' itself);
 //      k_adj_cells (every other case) runs one thread per cell over face
 //      arrays with periodic ghost copies (k_face_ghosts).
 // Deterministic (no atomics).  At most one wall axis.
@@ -328,27 +330,44 @@ __global__ void __launch_bounds__(256) k_adj_cells(KParams P, const Store* __res
   }
 }
 
-// ---- kernel 3, z-marching form (32 x 8 column tiles) ----
-// A workgroup owns a kGX x kGY tile of cell columns and marches along z over
-// a chunk of planes.  Per plane it stages the x-, y- and z-face cotangents of
-// the tile and a one-deep ring ((kGY+2) x (kGX+2) ghost-inclusive positions,
-// periodic indices wrapped, so no ghost copies are needed) in LDS, with the
-// next plane's loads in flight in registers; each cell then gathers its
-// transposed in-plane lerps from LDS.  The transposed z-lerps are pushed
-// into the f-bar+ cotangents of planes p-1, p and p+1 held in registers:
-// the x- and y-faces of plane p (z-lerped toward p - c_z in the step) and
-// the z-face p+1/2 (normal lerp between p and p+1).  Wall ghosts are folded
-// at the in-plane level: a cell beside a wall adds q (or 1 - q) times the
-// in-plane gather at the ghost position, which takes the same z transposes
-// as its own.  Each face value is read from HBM about 1.3 times (the ring)
-// instead of about 2.5 times.  The centre-stage adjoint needs only rho and j
-// of the state: with the state stored in the arithmetic type it reads them
-// from the face pass (16 or 32 bytes a cell) rather than the 19 values of f.
-constexpr int kGX = 32, kGY = 8;
-constexpr int kGW = kGX + 2;          // staged row length
-constexpr int kGP = (kGY + 2) * kGW;  // staged positions per array and population
-constexpr int kGT = kGX * kGY;        // lanes: one per cell column
-static_assert(kGP <= 2 * kGT, "two staged positions per lane at most");
+// ---- kernel 3, z-marching form ----
+// A workgroup owns a tile of cell columns (32 x 12 with FP32 arithmetic, 16 x
+// 12 with FP64) and marches along z over a chunk of planes.  A lane stages one
+// position of the tile or of its one-deep ring (periodic indices wrapped, so no
+// ghost copies are needed).  Per plane p:
+//   - lam'(p) of every position goes to LDS;
+//   - each position's x- and y-face of plane p and z-face p-1/2 are expanded to
+//     their 19 reconstructed-value cotangents in LDS, from the face's record
+//     (Ac, B) and the lam' on both of its sides;
+//   - each cell gathers its transposed in-plane lerps from LDS.  The transposed
+//     z-lerps are pushed into the f-bar+ cotangents of planes p-1, p and p+1
+//     held in registers: the x- and y-faces of plane p (z-lerped toward p - c_z
+//     in the step) and the z-face p-1/2 (normal lerp between p-1 and p).  Plane
+//     p-1 is then complete and goes through the centre stage's adjoint.
+// Wall ghosts are folded at the in-plane level: a cell beside a wall adds q (or
+// 1 - q) times the in-plane gather at the ghost position, which takes the same
+// z transposes as its own.  The centre stage needs only rho and j of the state:
+// with the state stored in the arithmetic type it reads them from the face pass
+// (16 or 32 bytes a cell) rather than the 19 values of f.
+//
+// What bounds it: HBM.  A cell reads lam' (19 values), three face records (4
+// each, in one 16-byte access with FP32) and rho, j, and writes lam; the records
+// held the ten crossing values as well (13 each) before, so that the two passes
+// moved 174 values a cell, now 120.  The next plane's loads go out during the
+// gather, a plane ahead of their use, without branches (accesses that are not
+// wanted go out of range), so that every wait counts exactly.  Ring lanes run
+// the gather and the centre stage on clamped positions and store nothing: they
+// share SIMDs with one wave of cells where the others hold two.
+// 256x192x256 FP32: 0.98 ms, before 1.23; the face pass 1.09, before 1.41.
+// lanes of a workgroup, and LDS positions (the last ones idle)
+constexpr int gather_lanes(bool fp64, int rows) { return ((rows + 2) * (fp64 ? 18 : 34) + 63) / 64 * 64; }
+template <class Real, int ROWS>
+struct GatherTile {
+  static constexpr int TX = sizeof(Real) == 8 ? 16 : 32, TY = ROWS;
+  static constexpr int AC = TX + 2, NP = (TY + 2) * AC;
+  static constexpr int NT = gather_lanes(sizeof(Real) == 8, ROWS);
+  static_assert(NT > NP, "an idle position, whose face cotangents are zeros");
+};
 
 // mom: the region of rho, j behind the face records that holds fin's
 // (storage in the arithmetic type).  FLOW (such storage, with FP32 lam and
@@ -356,41 +375,62 @@ static_assert(kGP <= 2 * kGT, "two staged positions per lane at most");
 // controller): lam' still lacks the bulk velocity's cotangent ubar (dV/V)
 // (c_ia - u_a)/rho of f(n+1), whose rho, j the previous pass left in the
 // other region; it is added as lam' is used.
-template <class Real, class Store, class Lam, bool FLOW = false>
-__global__ void __launch_bounds__(kGT) k_adj_cells_z(KParams P, const Store* __restrict__ fin,
-                                                     const Lam* __restrict__ lam, const Real* __restrict__ faces,
-                                                     Lam* __restrict__ lam_prev, double* __restrict__ grad, int TZ,
-                                                     int mom, const double* __restrict__ ubar, double inv_vol) {
-  __shared__ Real S[3][Q][kGP];   // face cotangents of plane p: x-faces, y-faces, z-faces p+1/2
-  __shared__ Real WXs[5][kGW];    // per staged column: wR for c = -1, 0, +1, then the shift weights
-  __shared__ Real WYs[5][kGY + 2];  // per staged row
+template <class Real, class Store, class Lam, int ROWS, bool FLOW = false>
+__global__ void __launch_bounds__(gather_lanes(sizeof(Real) == 8, ROWS), sizeof(Real) == 4 ? 2 : 1)
+    k_adj_cells_z(KParams P, const Store* __restrict__ fin, const Lam* __restrict__ lam,
+                  const Real* __restrict__ faces, Lam* __restrict__ lam_prev, double* __restrict__ grad, int nchunk,
+                  int mom, const double* __restrict__ ubar, double inv_vol) {
+  using T = GatherTile<Real, ROWS>;
+  constexpr int TX = T::TX, TY = T::TY, AC = T::AC, NT = T::NT;
+  __shared__ Real S[3][Q][NT];   // face cotangents: x-faces and y-faces of plane p, z-faces p-1/2
+  __shared__ Real L[Q][NT];      // lam'(p) (populations with c_x or c_y)
+  __shared__ Real WXs[6][AC];    // per staged column: wR for c = -1, 0, +1, the shift weights, dt/dx
+  __shared__ Real WYs[6][TY + 2];  // per staged row
 
   const int nx = P.n[0], ny = P.n[1], nz = P.n[2];
   const int t = threadIdx.x;
   // XCD-aware tile order (workgroup b runs on XCD b % 8)
-  const int gxn = nx / kGX, gyn = ny / kGY;
-  const int ntiles = gxn * gyn * (int)gridDim.z;
-  const int b = blockIdx.x + gxn * (blockIdx.y + gyn * blockIdx.z);
-  const int tt = (ntiles % 8 == 0) ? (b % 8) * (ntiles / 8) + b / 8 : b;
+  const int gxn = nx / TX, gyn = (ny + TY - 1) / TY;
+  const int nblocks = gxn * gyn * nchunk, b = blockIdx.x, xcd = b % 8;
+  const int tt = xcd * (nblocks / 8) + min(xcd, nblocks % 8) + b / 8;
   const int bx = tt % gxn, by = (tt / gxn) % gyn, bz = tt / (gxn * gyn);
-  const int i0 = bx * kGX, j0 = by * kGY;
-  const int z0 = bz * TZ, zend = min(z0 + TZ, nz);
+  // the last row of tiles starts early where TY does not divide ny; its first
+  // ry0 rows are the other tile's to store
+  const int th = min(TY, ny);
+  const int i0 = bx * TX, j0 = min(by * TY, ny - th), ry0 = by * TY - j0;
+  const int z0 = (int)((long long)bz * nz / nchunk), zend = (int)((long long)(bz + 1) * nz / nchunk);
   const int ex = P.e[0], ey = P.e[1];
 
-  // the lane's cell, and its staged (ghost-inclusive, tile-local) position
-  const int r = t / kGX, c = t % kGX;
-  const int R = r + 1, Cc = c + 1;
-  const unsigned plane = (unsigned)nx * (unsigned)ny;
-  const unsigned colcell = (unsigned)(j0 + r) * (unsigned)nx + (unsigned)(i0 + c);
+  // the lane's staged position (R, C), ghost-inclusive and tile-local: the
+  // cells first, then the rows above and below, then the columns beside
+  int R, C;
+  if (t < TX * TY) {
+    R = t / TX + 1;
+    C = t % TX + 1;
+  } else if (t < TX * TY + 2 * AC) {
+    const int v = t - TX * TY;
+    R = v < AC ? 0 : th + 1;
+    C = v % AC;
+  } else {
+    const int v = t - TX * TY - 2 * AC;
+    R = v % TY + 1;
+    C = v < TY ? 0 : TX + 1;
+  }
+  const bool staged = t < T::NP && (R <= th || (R == th + 1 && t >= TX * TY));
+  const bool cell_lane = staged && t < TX * TY;
+  const int pos0 = staged ? R * AC + C : T::NP;  // the others: the idle position
+  const bool stored = cell_lane && R > ry0;
+  // where the lane gathers (cells: their own position)
+  const int Rg0 = min(max(R, 1), th), Cg0 = min(max(C, 1), TX);
 
   // weights of the staged columns and rows (table_slot maps the periodic ghosts)
-  for (int u = t; u < 5 * kGW + 5 * (kGY + 2); u += kGT) {
-    const bool isx = u < 5 * kGW;
-    const int v = isx ? u : u - 5 * kGW;
-    const int n = isx ? kGW : kGY + 2;
+  for (int u = t; u < 6 * AC + 6 * (TY + 2); u += NT) {
+    const bool isx = u < 6 * AC;
+    const int v = isx ? u : u - 6 * AC;
+    const int n = isx ? AC : TY + 2;
     const int k = v / n, q = v % n;
     const int a = isx ? 0 : 1;
-    const int slot = table_slot(P, a, (isx ? i0 : j0) + q);
+    const int slot = table_slot(P, a, min((isx ? i0 : j0) + q, (isx ? nx : ny) + 1));
     const Real w = tabv<Real>(P, a, slot * 9 + (k < 3 ? k : k + 3));
     if (isx)
       WXs[k][q] = w;
@@ -398,131 +438,126 @@ __global__ void __launch_bounds__(kGT) k_adj_cells_z(KParams P, const Store* __r
       WYs[k][q] = w;
   }
   // z is periodic and uniform
-  const Real mz6 = tabv<Real>(P, 2, 9 + 6), mz7 = tabv<Real>(P, 2, 9 + 7);
+  const Real mz6 = tabv<Real>(P, 2, 9 + 6), mz7 = tabv<Real>(P, 2, 9 + 7), updz = tabv<Real>(P, 2, 9 + 8);
   const Real wRz[3] = {tabv<Real>(P, 2, 9 + 0), tabv<Real>(P, 2, 9 + 1), tabv<Real>(P, 2, 9 + 2)};
 
   Real Famb[3];
   Famb[0] = (Real)P.famb_dev[0];
   Famb[1] = (Real)P.famb_dev[1];
   Famb[2] = (Real)P.famb_dev[2];
-  const Real hdt = (Real)P.hdt, bw0 = (Real)P.bw0, bw1 = (Real)P.bw1, bw2 = (Real)P.bw2;
+  const Real hdt = (Real)P.hdt, bw0 = (Real)P.bw0, bw1 = (Real)P.bw1, bw2 = (Real)P.bw2, fw1 = (Real)P.fw1;
 
-  // staged positions of this lane: t and t + kGT
-  unsigned exy[2];
-  bool okp[2], okx[2], oky[2];
-  for (int h = 0; h < 2; h++) {
-    const int pp = t + h * kGT;
-    okp[h] = pp < kGP;
-    const int Rs = pp / kGW, Cs = pp % kGW;
-    int x = i0 + Cs, y = j0 + Rs;
-    if (P.periodic[0]) x = x == 0 ? nx : (x == nx + 1 ? 1 : x);
-    if (P.periodic[1]) y = y == 0 ? ny : (y == ny + 1 ? 1 : y);
-    exy[h] = (unsigned)y * (unsigned)ex + (unsigned)x;
-    okx[h] = okp[h] && Cs <= kGX;  // x-face slots i0 .. i0+kGX
-    oky[h] = okp[h] && Rs <= kGY;  // y-face slots j0 .. j0+kGY
-  }
-  // compact face records (launch_adjoint_faces_fused, compact_record)
-  const unsigned pop_bytes = (unsigned)(P.eN * (long long)sizeof(Real));
-  const RawBuf fx(faces, kCompact * pop_bytes), fy(faces + kCompact * P.eN, kCompact * pop_bytes),
-      fz(faces + 2 * kCompact * P.eN, kCompact * pop_bytes);
-  // wall faces among the staged slots: x-face slot 0 / nx, y-face slot 0 / ny
-  bool wlo[2][2], whi[2][2];
-  for (int h = 0; h < 2; h++) {
-    const int pp = t + h * kGT;
-    const int xs = i0 + pp % kGW, ys = j0 + pp / kGW;
-    wlo[h][0] = !P.periodic[0] && xs == 0;
-    whi[h][0] = !P.periodic[0] && xs == nx;
-    wlo[h][1] = !P.periodic[1] && ys == 0;
-    whi[h][1] = !P.periodic[1] && ys == ny;
-  }
-  const Real fw1 = (Real)P.fw1;
-  Real pre[2][3][kCompact];
-  // face records of plane p (ghost-inclusive z slot p + 1) into registers
-  auto stage_load = [&](int p) {
-    int zs = p + 1;
-    zs = zs == 0 ? nz : (zs == nz + 1 ? 1 : zs);
-    const unsigned zoff = (unsigned)zs * (unsigned)ey * (unsigned)ex;
-    for (int h = 0; h < 2; h++) {
-      const unsigned vb = (zoff + exy[h]) * (unsigned)sizeof(Real);
-      const unsigned vx = okx[h] ? vb : kOutOfRange, vy = oky[h] ? vb : kOutOfRange, vz = okp[h] ? vb : kOutOfRange;
-      static_for<kCompact>([&](auto K) {
-        constexpr int k = decltype(K)::value;
-        pre[h][0][k] = fx.ld<Real>(vx, k * pop_bytes);
-        pre[h][1][k] = fy.ld<Real>(vy, k * pop_bytes);
-        pre[h][2][k] = fz.ld<Real>(vz, k * pop_bytes);
-      });
+  // the staged position's face slot and cell, the faces it has, and which are at walls
+  int x = i0 + C, y = j0 + R;
+  const bool wlx = !P.periodic[0] && x == 0, whx = !P.periodic[0] && x == nx;
+  const bool wly = !P.periodic[1] && y == 0, why = !P.periodic[1] && y == ny;
+  if (P.periodic[0]) x = x == 0 ? nx : (x == nx + 1 ? 1 : x);
+  if (P.periodic[1]) y = y == 0 ? ny : (y == ny + 1 ? 1 : y);
+  const unsigned exy = (unsigned)y * (unsigned)ex + (unsigned)x;
+  const bool has_cell = staged && x >= 1 && x <= nx && y >= 1 && y <= ny;
+  const bool okx = staged && C <= TX, oky = staged && R <= th;
+  const unsigned plane = (unsigned)nx * (unsigned)ny;
+  const unsigned column = has_cell ? (unsigned)(y - 1) * (unsigned)nx + (unsigned)(x - 1) : 0u;
+
+  const RawBuf recs[3] = {face_records<Real>(faces, 0, P.eN), face_records<Real>(faces, 1, P.eN),
+                          face_records<Real>(faces, 2, P.eN)};
+  const RawBuf lamb(lam, (unsigned)(Q * P.N * sizeof(Lam))), outb(lam_prev, (unsigned)(Q * P.N * sizeof(Lam)));
+  const unsigned lam_pop = (unsigned)(P.N * sizeof(Lam));
+  // the cell force and the gradient; absent ones read as 0 and take no stores
+  const RawBuf fcb(P.fcell, P.fcell ? (unsigned)(3 * P.N * 8) : 0u), gradb(grad, grad ? (unsigned)(3 * P.N * 8) : 0u);
+  const unsigned vec_pop = (unsigned)(P.N * 8);
+  const StateBuf<Store> bin(fin, Q * (unsigned)(P.N * (long long)sizeof(Store)));
+  constexpr bool kMoments = std::is_same<Store, Real>::value;
+  const RawBuf mb = cell_records<Real>(faces, mom, P.eN, P.N);
+  // FLOW: rho and j_a of f(n+1) at the staged cell, and s0 = ubar dV / V
+  static_assert(!FLOW || kMoments, "the controller term needs the moments of f(n+1)");
+  const RawBuf mbn = cell_records<Real>(faces, 1 - mom, P.eN, P.N);
+  const int fa = P.flow_axis;
+  Real s0 = Real(0), rn = Real(0), jn = Real(0);
+  if constexpr (FLOW)
+    if (has_cell) s0 = (Real)(ubar[0] * P.wd[0][x] * P.wd[1][y] * P.wd[2][1] * inv_vol);
+
+  // lam' of planes p-1 and p at the staged position, and of p+1 as loaded; the
+  // records of the position's faces
+  Real lamP[Q], lamC[Q];
+  Lam lraw[Q];
+  Real rec[3][kCompact];
+  auto load_lam = [&](auto A, auto B, int k, bool want) {
+    const unsigned vb = want && has_cell ? ((unsigned)k * plane + column) * (unsigned)sizeof(Lam) : kOutOfRange;
+    static_for<decltype(B)::value - decltype(A)::value>([&](auto I) {
+      constexpr int ip = decltype(A)::value + decltype(I)::value;
+      lraw[ip] = lamb.ld<Lam>(vb, ip * lam_pop);
+    });
+    if constexpr (FLOW && decltype(A)::value == 0) {
+      const unsigned vm = want && has_cell ? ((unsigned)k * plane + column) * (unsigned)(4 * sizeof(Real)) : kOutOfRange;
+      rn = mbn.ld<Real>(vm, 0);
+      jn = mbn.ld<Real>(vm, (unsigned)(1 + fa) * (unsigned)sizeof(Real));
     }
   };
-  // the 19 reconstructed-value cotangents of each staged face into LDS (a
-  // missing face has an all-zero record and expands to zeros)
-  auto expand_store = [&](auto AI, int h, int pp) {
+  // the x- and y-face records of plane k (0-based; z slot k + 1) and the z-face's of k - 1/2 (z slot kl + 1, kl = k - 1 wrapped)
+  auto load_recs = [&](int k, bool want) {
+    const int kl = k == 0 ? nz - 1 : k - 1;
+    const unsigned ez = (unsigned)ey * (unsigned)ex, size = (unsigned)(kCompact * sizeof(Real));
+    const unsigned v = ((unsigned)(k + 1) * ez + exy) * size, vz = ((unsigned)(kl + 1) * ez + exy) * size;
+    recs[0].ld4(want && okx ? v : kOutOfRange, rec[0]);
+    recs[1].ld4(want && oky ? v : kOutOfRange, rec[1]);
+    recs[2].ld4(want && staged ? vz : kOutOfRange, rec[2]);
+  };
+  using I0 = std::integral_constant<int, 0>;
+  using I10 = std::integral_constant<int, 10>;
+  using IQ = std::integral_constant<int, Q>;
+  auto wrap = [&](int k) { return k < 0 ? k + nz : (k >= nz ? k - nz : k); };
+
+  // the 19 reconstructed-value cotangents of the lane's A-face into LDS, from mu
+  auto expand = [&](auto AI, int pos, const Real (&mu)[10], bool ok, bool lo, bool hi) {
     constexpr int A = decltype(AI)::value;
-    Real rec[kCompact], lamf[Q];
-    static_for<kCompact>([&](auto K) { rec[decltype(K)::value] = pre[h][A][decltype(K)::value]; });
-    const bool lo = A < 2 && wlo[h][A < 2 ? A : 0], hi = A < 2 && whi[h][A < 2 ? A : 0];
-    expand_record<Real, A>(rec, lo, hi, lamf);
+    Real v[Q];
+    const Real B[3] = {rec[A][1], rec[A][2], rec[A][3]};
+    expand_cotangents<Real, A>(mu, rec[A][0], B, fw1, lo, hi, v);
     static_for<Q>([&](auto I) {
       constexpr int ip = decltype(I)::value;
-      S[A][ip][pp] = lamf[ip];
+      S[A][ip][pos] = ok ? v[ip] : Real(0);
     });
   };
-  auto stage_store = [&]() {
-    for (int h = 0; h < 2; h++) {
-      if (!okp[h]) continue;
-      const int pp = t + h * kGT;
-      expand_store(std::integral_constant<int, 0>{}, h, pp);
-      expand_store(std::integral_constant<int, 1>{}, h, pp);
-      expand_store(std::integral_constant<int, 2>{}, h, pp);
-    }
-  };
 
-  // In-plane transposed lerps at staged position (Rp, Cp) for population ip:
-  // the cotangent of Z(p) (x- and y-faces) and of Zn(p+1/2) (z-faces).
-  // GUARD: the position is a wall ghost, whose stencil reaches outside the
-  // staged region (nothing is there: 0).
-  auto sget = [&](int A, int ip, int Rp, int Cp, bool guard) -> Real {
-    if (guard && (Rp < 0 || Rp > kGY + 1 || Cp < 0 || Cp > kGX + 1)) return Real(0);
-    return S[A][ip][Rp * kGW + Cp];
-  };
-  auto inplane = [&](auto I, int Rp, int Cp, bool guard, Real& hz_out) -> Real {
+  // In-plane transposed lerps at a position for population ip: the cotangent
+  // of Z(p) (x- and y-faces) and of Zn (z-faces).  at(A, ip, dr, dc): the A-face
+  // cotangent dr rows and dc columns from the position; WX(k, dc), WY(k, dr):
+  // the weights there.
+  auto inplane = [&](auto I, auto at, auto WX, auto WY, Real& hz_out) -> Real {
     constexpr int ip = decltype(I)::value;
     constexpr int cx = CX[ip], cy = CY[ip];
-    // weights at a guarded position's outside neighbours only multiply 0;
-    // clamp their index so that they stay table values
-    auto WX = [&](int k, int Cq) { return WXs[k][guard ? min(max(Cq, 0), kGW - 1) : Cq]; };
-    auto WY = [&](int k, int Rq) { return WYs[k][guard ? min(max(Rq, 0), kGY + 1) : Rq]; };
     if constexpr (ip == 0) {
-      hz_out = sget(2, 0, Rp, Cp, guard);
-      return Real(0.5) * (sget(0, 0, Rp, Cp, guard) + sget(0, 0, Rp, Cp - 1, guard)) +
-             Real(0.5) * (sget(1, 0, Rp, Cp, guard) + sget(1, 0, Rp - 1, Cp, guard));
+      hz_out = at(2, 0, 0, 0);
+      return Real(0.5) * (at(0, 0, 0, 0) + at(0, 0, 0, -1)) + Real(0.5) * (at(1, 0, 0, 0) + at(1, 0, -1, 0));
     } else {
-      // x-faces: slot Cp (this column is the left cell), Cp-1 (right cell);
-      // rows Rp and Rp+c_y
-      const Real a0 = Real(1) - WX(cx + 1, Cp), a1 = WX(cx + 1, Cp - 1);
-      Real hx = a0 * sget(0, ip, Rp, Cp, guard) + a1 * sget(0, ip, Rp, Cp - 1, guard);
+      // x-faces: this column is the left cell of its own slot, the right cell
+      // of the slot before; rows 0 and c_y
+      const Real a0 = Real(1) - WX(cx + 1, 0), a1 = WX(cx + 1, -1);
+      Real hx = a0 * at(0, ip, 0, 0) + a1 * at(0, ip, 0, -1);
       if constexpr (cy != 0) {
-        const Real m0 = Real(1) - WY(cy < 0 ? 3 : 4, Rp), m1 = WY(cy < 0 ? 3 : 4, Rp + cy);
-        hx = m0 * hx + m1 * (a0 * sget(0, ip, Rp + cy, Cp, guard) + a1 * sget(0, ip, Rp + cy, Cp - 1, guard));
+        const Real m0 = Real(1) - WY(cy < 0 ? 3 : 4, 0), m1 = WY(cy < 0 ? 3 : 4, cy);
+        hx = m0 * hx + m1 * (a0 * at(0, ip, cy, 0) + a1 * at(0, ip, cy, -1));
       }
-      // y-faces: slot Rp (this row is the lower cell), Rp-1 (upper cell);
-      // columns Cp and Cp+c_x
-      const Real b0 = Real(1) - WY(cy + 1, Rp), b1 = WY(cy + 1, Rp - 1);
-      Real hy = b0 * sget(1, ip, Rp, Cp, guard) + b1 * sget(1, ip, Rp - 1, Cp, guard);
+      // y-faces: this row is the lower cell of its own slot, the upper cell of
+      // the slot before; columns 0 and c_x
+      const Real b0 = Real(1) - WY(cy + 1, 0), b1 = WY(cy + 1, -1);
+      Real hy = b0 * at(1, ip, 0, 0) + b1 * at(1, ip, -1, 0);
       if constexpr (cx != 0) {
-        const Real m0 = Real(1) - WX(cx < 0 ? 3 : 4, Cp), m1 = WX(cx < 0 ? 3 : 4, Cp + cx);
-        hy = m0 * hy + m1 * (b0 * sget(1, ip, Rp, Cp + cx, guard) + b1 * sget(1, ip, Rp - 1, Cp + cx, guard));
+        const Real m0 = Real(1) - WX(cx < 0 ? 3 : 4, 0), m1 = WX(cx < 0 ? 3 : 4, cx);
+        hy = m0 * hy + m1 * (b0 * at(1, ip, 0, cx) + b1 * at(1, ip, -1, cx));
       }
-      // z-face p+1/2: columns Cp, Cp+c_x; rows Rp, Rp+c_y
-      Real hz = sget(2, ip, Rp, Cp, guard);
+      // z-face: columns 0, c_x; rows 0, c_y
+      Real hz = at(2, ip, 0, 0);
       Real hz2 = Real(0);
-      if constexpr (cy != 0) hz2 = sget(2, ip, Rp + cy, Cp, guard);
+      if constexpr (cy != 0) hz2 = at(2, ip, cy, 0);
       if constexpr (cx != 0) {
-        const Real m0 = Real(1) - WX(cx < 0 ? 3 : 4, Cp), m1 = WX(cx < 0 ? 3 : 4, Cp + cx);
-        hz = m0 * hz + m1 * sget(2, ip, Rp, Cp + cx, guard);
-        if constexpr (cy != 0) hz2 = m0 * hz2 + m1 * sget(2, ip, Rp + cy, Cp + cx, guard);
+        const Real m0 = Real(1) - WX(cx < 0 ? 3 : 4, 0), m1 = WX(cx < 0 ? 3 : 4, cx);
+        hz = m0 * hz + m1 * at(2, ip, 0, cx);
+        if constexpr (cy != 0) hz2 = m0 * hz2 + m1 * at(2, ip, cy, cx);
       }
       if constexpr (cy != 0) {
-        const Real m0 = Real(1) - WY(cy < 0 ? 3 : 4, Rp), m1 = WY(cy < 0 ? 3 : 4, Rp + cy);
+        const Real m0 = Real(1) - WY(cy < 0 ? 3 : 4, 0), m1 = WY(cy < 0 ? 3 : 4, cy);
         hz = m0 * hz + m1 * hz2;
       }
       hz_out = hz;
@@ -531,104 +566,98 @@ __global__ void __launch_bounds__(kGT) k_adj_cells_z(KParams P, const Store* __r
   };
 
   // wall ghost folded into this cell: position and weight (at most one wall axis)
-  int gR = -1, gC = -1;
+  int gR0 = -1, gC0 = -1;
   Real gq = Real(0);
-  if (!P.periodic[1]) {
+  if (cell_lane && !P.periodic[1]) {
     if (j0 == 0 && R <= 2) {
-      gR = 0, gC = Cc, gq = R == 1 ? (Real)P.qlo[1] : Real(1) - (Real)P.qlo[1];
-    } else if (j0 + kGY == ny && R >= kGY - 1) {
-      gR = kGY + 1, gC = Cc, gq = R == kGY ? (Real)P.qhi[1] : Real(1) - (Real)P.qhi[1];
+      gR0 = 0, gC0 = C, gq = R == 1 ? (Real)P.qlo[1] : Real(1) - (Real)P.qlo[1];
+    } else if (j0 + th == ny && R >= th - 1) {
+      gR0 = th + 1, gC0 = C, gq = R == th ? (Real)P.qhi[1] : Real(1) - (Real)P.qhi[1];
     }
-  } else if (!P.periodic[0]) {
-    if (i0 == 0 && Cc <= 2) {
-      gR = R, gC = 0, gq = Cc == 1 ? (Real)P.qlo[0] : Real(1) - (Real)P.qlo[0];
-    } else if (i0 + kGX == nx && Cc >= kGX - 1) {
-      gR = R, gC = kGX + 1, gq = Cc == kGX ? (Real)P.qhi[0] : Real(1) - (Real)P.qhi[0];
+  } else if (cell_lane && !P.periodic[0]) {
+    if (i0 == 0 && C <= 2) {
+      gR0 = R, gC0 = 0, gq = C == 1 ? (Real)P.qlo[0] : Real(1) - (Real)P.qlo[0];
+    } else if (i0 + TX == nx && C >= TX - 1) {
+      gR0 = R, gC0 = TX + 1, gq = C == TX ? (Real)P.qhi[0] : Real(1) - (Real)P.qhi[0];
     }
   }
-  const bool ghost = gR >= 0;
+  const bool ghost = gR0 >= 0;
 
-  Real accP[Q], accC[Q];
+  Real accP[Q], accC[Q], accN[Q];
   static_for<Q>([&](auto I) {
     constexpr int ip = decltype(I)::value;
     accP[ip] = Real(0);
     accC[ip] = Real(0);
+    lamC[ip] = Real(0);
   });
-  const StateBuf<Store> bin(fin, Q * (unsigned)(P.N * (long long)sizeof(Store)));
-  const unsigned Nb = (unsigned)(P.N * (long long)sizeof(Store));
-  const RawBuf lamb(lam, (unsigned)(Q * P.N * sizeof(Lam)));
-  const unsigned lam_pop = (unsigned)(P.N * sizeof(Lam));
-  // with the state stored in the arithmetic type the face pass has stored
-  // rho and j of every cell behind the records: 4 values read per cell
-  // instead of 19 of f
-  constexpr bool kMoments = std::is_same<Store, Real>::value;
-  const RawBuf mb(faces + 3LL * kCompact * P.eN + mom * 4LL * P.N, (unsigned)(4 * P.N * sizeof(Real)));
-  const unsigned mom_pop = (unsigned)(P.N * sizeof(Real));
-  // FLOW: rho and j_a of f(n+1) at the cell, and s0 = ubar dV / V
-  static_assert(!FLOW || kMoments, "the controller term needs the moments of f(n+1)");
-  const RawBuf mbn(faces + 3LL * kCompact * P.eN + (1 - mom) * 4LL * P.N, (unsigned)(4 * P.N * sizeof(Real)));
-  const int fa = P.flow_axis;
-  Real s0 = Real(0), rn = Real(1), jn = Real(0);
-  if constexpr (FLOW) s0 = (Real)(ubar[0] * P.wd[0][i0 + c + 1] * P.wd[1][j0 + r + 1] * P.wd[2][1] * inv_vol);
-
-  // inputs of the centre stage of one cell: lam', rho and j, the cell force,
-  // the gradient so far
-  Real lp[Q], rho = Real(1), j[3] = {0, 0, 0};
-  double fc[3] = {0, 0, 0}, g0[3] = {0, 0, 0};
-  auto load_centre = [&](unsigned cell) {
-    static_for<Q>([&](auto I) {
-      constexpr int ip = decltype(I)::value;
-      lp[ip] = (Real)lamb.ld<Lam>(cell * (unsigned)sizeof(Lam), ip * lam_pop);
-    });
-    if constexpr (kMoments) {
-      rho = mb.ld<Real>(cell * (unsigned)sizeof(Real), 0);
-      j[0] = mb.ld<Real>(cell * (unsigned)sizeof(Real), mom_pop);
-      j[1] = mb.ld<Real>(cell * (unsigned)sizeof(Real), 2 * mom_pop);
-      j[2] = mb.ld<Real>(cell * (unsigned)sizeof(Real), 3 * mom_pop);
-      if constexpr (FLOW) {
-        rn = mbn.ld<Real>(cell * (unsigned)sizeof(Real), 0);
-        jn = mbn.ld<Real>(cell * (unsigned)sizeof(Real), (unsigned)(1 + fa) * mom_pop);
-      }
-    } else {
-      Real ff[Q];
-      static_for<Q>([&](auto I) {
-        constexpr int ip = decltype(I)::value;
-        ff[ip] = ld_state<Real, Store>(bin, cell * (unsigned)sizeof(Store), ip * Nb, P, ip);
-      });
-      cell_moments<Real>(ff, rho, j);
-    }
-    if (P.fcell)
-      for (int a = 0; a < 3; a++) fc[a] = P.fcell[a * P.N + (long long)cell];
-    if (grad)
-      for (int a = 0; a < 3; a++) g0[a] = grad[a * P.N + (long long)cell];
-  };
-  // With FP32 lam and moments the registers allow these loads to be issued
-  // before the plane's face records, so the staging and the gather hide them.
-  constexpr bool kEarly = kMoments && std::is_same<Lam, float>::value;
+  load_lam(I0{}, IQ{}, wrap(z0 - 1), true);
+  load_recs(wrap(z0 - 1), true);
 
   for (int p = z0 - 1; p <= zend; p++) {
-    if constexpr (kEarly) {
-      if (p - 1 >= z0) load_centre((unsigned)(p - 1) * plane + colcell);
-    }
-    stage_load(p);
-    __syncthreads();  // the previous plane's gather is done with S
-    stage_store();
-    __syncthreads();
-    // transposed reconstruction, merged with the shift of the cotangent
-    // window after the plane p-1 is complete
-    Real accN[Q];
+    const int pos = here(pos0), Rg = here(Rg0), Cg = here(Cg0);  // (addresses formed anew each plane)
+    // lam'(p), complete
     static_for<Q>([&](auto I) {
       constexpr int ip = decltype(I)::value;
+      lamP[ip] = lamC[ip];
+      lamC[ip] = (Real)lraw[ip];
+    });
+    if constexpr (FLOW) {
+      // rn is 0 where nothing was loaded (s0 or lam' is unused there)
+      const Real inv = Real(1) / (rn != Real(0) ? rn : Real(1)), sc = s0 * inv, t0 = -sc * (jn * inv);
+      const Real ax = fa == 0 ? Real(1) : Real(0), ay = fa == 1 ? Real(1) : Real(0), az = fa == 2 ? Real(1) : Real(0);
+      static_for<Q>([&](auto I) {
+        constexpr int ip = decltype(I)::value;
+        lamC[ip] += fma_rn(Real(CX[ip]) * ax + Real(CY[ip]) * ay + Real(CZ[ip]) * az, sc, t0);
+      });
+    }
+    __syncthreads();  // the previous plane's gather is done with S
+    static_for<Q>([&](auto I) {
+      constexpr int ip = decltype(I)::value;
+      if constexpr (CX[ip] != 0 || CY[ip] != 0) L[ip][pos] = lamC[ip];
+    });
+    __syncthreads();
+    {
+      // mu of a face: c_A (dt/dA lam' of the upper cell - dt/dA lam' of the lower)
+      Real mu[10];
+      const int posx = okx ? pos + 1 : pos, posy = oky ? pos + AC : pos;
+      const Real ul = WXs[5][C], ur = WXs[5][min(C + 1, AC - 1)];
+      static_for<10>([&](auto K) {
+        constexpr int ip = XD[decltype(K)::value];
+        mu[decltype(K)::value] = Real(CX[ip]) * (ur * L[ip][posx] - ul * lamC[ip]);
+      });
+      expand(std::integral_constant<int, 0>{}, pos, mu, okx, wlx, whx);
+      const Real vl = WYs[5][R], vr = WYs[5][min(R + 1, TY + 1)];
+      static_for<10>([&](auto K) {
+        constexpr int ip = YD[decltype(K)::value];
+        mu[decltype(K)::value] = Real(CY[ip]) * (vr * L[ip][posy] - vl * lamC[ip]);
+      });
+      expand(std::integral_constant<int, 1>{}, pos, mu, oky, wly, why);
+      static_for<10>([&](auto K) {
+        constexpr int ip = ZD[decltype(K)::value];
+        mu[decltype(K)::value] = Real(CZ[ip]) * updz * (lamC[ip] - lamP[ip]);
+      });
+      expand(std::integral_constant<int, 2>{}, pos, mu, p >= z0, false, false);
+    }
+    // The centre stage's inputs of plane p-1 first, then, in groups, what the
+    // next plane needs
+    const bool centre = stored && p - 1 >= z0, more = p < zend;
+    const unsigned cell = centre ? (unsigned)(p - 1) * plane + column : 0u;
+    const unsigned v8 = centre ? cell * 8u : kOutOfRange;
+    Real m4[4] = {Real(1), Real(0), Real(0), Real(0)};
+    RawCell<Real, Store> fraw;
+    double fc[3], g0[3];
+    if constexpr (kMoments)
+      mb.ld4(centre ? cell * (unsigned)(4 * sizeof(Real)) : kOutOfRange, m4);
+    else
+      fraw.load(bin, cell, (unsigned)P.N);
+    for (int a = 0; a < 3; a++) fc[a] = fcb.ld<double>(v8, a * vec_pop);
+    for (int a = 0; a < 3; a++) g0[a] = gradb.ld<double>(v8, a * vec_pop);
+    __syncthreads();
+    // transposed reconstruction: a position's in-plane lerps through the
+    // transposed z-lerps
+    auto push = [&](auto I, Real hzr, Real hz) {
+      constexpr int ip = decltype(I)::value;
       constexpr int cz = CZ[ip];
-      Real hz;
-      Real hzr = inplane(I, R, Cc, false, hz);
-      if (ghost) {
-        Real gz;
-        const Real g = inplane(I, gR, gC, true, gz);
-        hzr += gq * g;
-        hz += gq * gz;
-      }
-      Real nxt = Real(0);
       if constexpr (cz == 0) {
         accC[ip] += hzr;
       } else if constexpr (cz > 0) {
@@ -636,51 +665,80 @@ __global__ void __launch_bounds__(kGT) k_adj_cells_z(KParams P, const Store* __r
         accP[ip] += mz7 * hzr;
       } else {
         accC[ip] += (Real(1) - mz6) * hzr;
-        nxt = mz6 * hzr;
+        accN[ip] += mz6 * hzr;
       }
       const Real wn = ip == 0 ? Real(0.5) : wRz[cz + 1];
-      accC[ip] += (Real(1) - wn) * hz;
-      accN[ip] = nxt + wn * hz;
+      accP[ip] += (Real(1) - wn) * hz;
+      accC[ip] += wn * hz;
+    };
+    const int gat = Rg * AC + Cg;
+    auto cell_at = [&](int A, int ip, int dr, int dc) -> Real { return S[A][ip][gat + dr * AC + dc]; };
+    auto cell_wx = [&](int k, int dc) -> Real { return WXs[k][Cg + dc]; };
+    auto cell_wy = [&](int k, int dr) -> Real { return WYs[k][Rg + dr]; };
+    static_for<Q>([&](auto I) {
+      constexpr int ip = decltype(I)::value;
+      if constexpr (ip == 1) load_lam(I0{}, I10{}, wrap(p + 1), more);
+      if constexpr (ip == 7) load_lam(I10{}, IQ{}, wrap(p + 1), more);
+      if constexpr (ip == 13) load_recs(wrap(p + 1), more);
+      Real hz;
+      const Real hzr = inplane(I, cell_at, cell_wx, cell_wy, hz);
+      accN[ip] = Real(0);
+      push(I, hzr, hz);
     });
-    // centre-stage adjoint of plane p-1 (as k_adj_cells)
-    if (p - 1 >= z0) {
-      const unsigned cell = (unsigned)(p - 1) * plane + colcell;
-      const long long cl = (long long)cell;
-      if constexpr (!kEarly) load_centre(cell);
-      if constexpr (FLOW) {
-        const Real inv = Real(1) / rn, sc = s0 * inv, t0 = -sc * (jn * inv);
-        const Real ex = fa == 0 ? Real(1) : Real(0), ey = fa == 1 ? Real(1) : Real(0),
-                   ez = fa == 2 ? Real(1) : Real(0);
-        static_for<Q>([&](auto I) {
-          constexpr int ip = decltype(I)::value;
-          lp[ip] += fma_rn(Real(CX[ip]) * ex + Real(CY[ip]) * ey + Real(CZ[ip]) * ez, sc, t0);
-        });
+    if (ghost) {
+      // The same at the ghost position, whose stencil reaches outside the
+      // staged region: nothing is there, and the idle position holds zeros.
+      // (One branch for all populations and no condition per value: with a
+      // branch each, the tiles at a wall took twice the time.)  The weights
+      // there only multiply zeros; their index is clamped.
+      const int gR = here(gR0), gC = here(gC0);
+      int gi[3][3], gx[3], gy[3];
+      for (int q = -1; q <= 1; q++) {
+        gx[q + 1] = min(max(gC + q, 0), AC - 1);
+        gy[q + 1] = min(max(gR + q, 0), TY + 1);
+        for (int v = -1; v <= 1; v++) {
+          const bool in = gR + q >= 0 && gR + q <= th + 1 && gC + v >= 0 && gC + v <= TX + 1;
+          gi[q + 1][v + 1] = in ? (gR + q) * AC + gC + v : T::NP;
+        }
       }
+      auto ghost_at = [&](int A, int ip, int dr, int dc) -> Real { return S[A][ip][gi[dr + 1][dc + 1]]; };
+      auto ghost_wx = [&](int k, int dc) -> Real { return WXs[k][gx[dc + 1]]; };
+      auto ghost_wy = [&](int k, int dr) -> Real { return WYs[k][gy[dr + 1]]; };
       static_for<Q>([&](auto I) {
-        constexpr int ip = decltype(I)::value;
-        accP[ip] += Real(4.0 / 3.0) * lp[ip];
+        Real hz;
+        const Real hzr = inplane(I, ghost_at, ghost_wx, ghost_wy, hz);
+        push(I, gq * hzr, gq * hz);
       });
-      Real F[3], u[3], ut[3];
-      const Real invr = Real(1) / rho;
-      for (int a = 0; a < 3; a++) {
-        F[a] = Famb[a];
-        if (P.fcell) F[a] += (Real)fc[a];
-        ut[a] = j[a] * invr;
-        u[a] = ut[a] + hdt * F[a];
-      }
-      Real g_rho, g_u[3], g_F[3];
-      feq_adjoint<Real>(accP, bw2, bw0, rho, u, F, g_rho, g_u, g_F, AllPops{});
-      const Real Acoef = g_rho - (g_u[0] * ut[0] + g_u[1] * ut[1] + g_u[2] * ut[2]) * invr;
-      static_for<Q>([&](auto I) {
-        constexpr int ip = decltype(I)::value;
-        const Real v = -lp[ip] * Real(1.0 / 3.0) + bw1 * accP[ip] + Acoef +
-                       (g_u[0] * Real(CX[ip]) + g_u[1] * Real(CY[ip]) + g_u[2] * Real(CZ[ip])) * invr;
-        lam_prev[ip * P.N + cl] = (Lam)v;
-      });
-      if (grad) {
-        for (int a = 0; a < 3; a++) grad[a * P.N + cl] = g0[a] + (double)(g_F[a] + hdt * g_u[a]);
-      }
     }
+    // centre-stage adjoint of plane p-1 (as k_adj_cells)
+    Real rho = m4[0], j[3] = {m4[1], m4[2], m4[3]};
+    if constexpr (!kMoments) {
+      Real ff[Q], u0[3];
+      fraw.decode(P, ff, rho, u0);
+      cell_moments<Real>(ff, rho, j);
+    }
+    static_for<Q>([&](auto I) {
+      constexpr int ip = decltype(I)::value;
+      accP[ip] += Real(4.0 / 3.0) * lamP[ip];
+    });
+    Real F[3], u[3], ut[3];
+    const Real invr = Real(1) / rho;
+    for (int a = 0; a < 3; a++) {
+      F[a] = Famb[a] + (Real)fc[a];
+      ut[a] = j[a] * invr;
+      u[a] = ut[a] + hdt * F[a];
+    }
+    Real g_rho, g_u[3], g_F[3];
+    feq_adjoint<Real>(accP, bw2, bw0, rho, u, F, g_rho, g_u, g_F, AllPops{});
+    const Real Acoef = g_rho - (g_u[0] * ut[0] + g_u[1] * ut[1] + g_u[2] * ut[2]) * invr;
+    const unsigned vl = centre ? cell * (unsigned)sizeof(Lam) : kOutOfRange;
+    static_for<Q>([&](auto I) {
+      constexpr int ip = decltype(I)::value;
+      const Real v = -lamP[ip] * Real(1.0 / 3.0) + bw1 * accP[ip] + Acoef +
+                     (g_u[0] * Real(CX[ip]) + g_u[1] * Real(CY[ip]) + g_u[2] * Real(CZ[ip])) * invr;
+      outb.st((Lam)v, vl, ip * lam_pop);
+    });
+    for (int a = 0; a < 3; a++) gradb.st(g0[a] + (double)(g_F[a] + hdt * g_u[a]), v8, a * vec_pop);
     static_for<Q>([&](auto I) {
       constexpr int ip = decltype(I)::value;
       accP[ip] = accC[ip];
@@ -689,13 +747,13 @@ __global__ void __launch_bounds__(kGT) k_adj_cells_z(KParams P, const Store* __r
   }
 }
 
-// The z-marching gather covers FP32 and FP64 arithmetic on 32 x 8 column
-// tiles with z periodic and uniform, at most one wall axis (x or y), and face
-// arrays and lam' that 32-bit buffer offsets reach.
+// The z-marching gather covers FP32 and FP64 arithmetic on grids of whole 32 x
+// 8 columns with z periodic and uniform, at most one wall axis (x or y), and
+// face arrays and lam' that 32-bit buffer offsets reach.
 bool gather_z_supported(const Ctx& c) {
   const Setup& s = c.s;
   if (c.kernel == 0) return false;
-  if (s.n[0] % kGX != 0 || s.n[1] % kGY != 0 || !s.periodic[2] || !s.uniform[2]) return false;
+  if (s.n[0] % 32 != 0 || s.n[1] % 8 != 0 || !s.periodic[2] || !s.uniform[2]) return false;
   if (!s.periodic[0] && !s.periodic[1]) return false;
   if (!s.periodic[0] && s.n[0] < 3) return false;
   if (!s.periodic[1] && s.n[1] < 3) return false;
@@ -704,13 +762,37 @@ bool gather_z_supported(const Ctx& c) {
   return true;
 }
 
-// A chunk gathers the two planes beside it too.  FP32 tiles run two to a CU,
-// FP64 one.  On 64x64x32 FP64 (16 tiles): 46 us with 2-plane chunks, 106 with
-// 8-plane ones.
-int gather_z_chunk(const KParams& P, bool fp64) {
-  const long long cols = (long long)(P.n[0] / kGX) * (P.n[1] / kGY);
-  const int nc = plan_z_chunks(cols, P.n[2], fp64 ? 256 : 512, 2.0);
-  return (P.n[2] + nc - 1) / nc;
+// Tile height (12 or 8 rows) and z-chunks of the gather, one workgroup per CU;
+// a chunk gathers the two planes beside it too.  A plane of an 8-row tile takes
+// 0.8 of the time, so they go where they fill more CUs (64x64x32: FP32 adjoint
+// step 58 us against 62 with 12 rows, FP64 gather 56.5 against 58).
+struct GatherPlan {
+  int rows, nchunk;
+  long long nblocks;
+};
+GatherPlan gather_plan(const KParams& P, bool fp64) {
+  GatherPlan best{};
+  double least = 0;
+  for (const int rows : {12, 8}) {
+    const long long tiles = (long long)(P.n[0] / (fp64 ? 16 : 32)) * ((P.n[1] + rows - 1) / rows);
+    const int nz = P.n[2], nc = plan_z_chunks(tiles, nz, 256, 2.0);
+    const double cost = (rows == 12 ? 1.0 : 0.8) * (double)((tiles * nc + 255) / 256) * ((nz + nc - 1) / nc + 2.0);
+    if (rows == 12 || cost < 0.97 * least) {
+      best = {rows, nc, tiles * nc};
+      least = cost;
+    }
+  }
+  return best;
+}
+
+template <class Real, class Store, class Lam, int ROWS, bool FLOW>
+void launch_gather(const Ctx& cx, const GatherPlan& g, const void* f, const Lam* lam_next, Lam* lam_prev,
+                   double* grad, int mom, const double* ubar) {
+  const double inv_vol = 1.0 / (cx.s.width[0] * cx.s.width[1] * cx.s.width[2]);
+  hipLaunchKernelGGL((k_adj_cells_z<Real, Store, Lam, ROWS, FLOW>), dim3((unsigned)g.nblocks),
+                     dim3(GatherTile<Real, ROWS>::NT), 0, cx.stream, cx.kp, static_cast<const Store*>(f), lam_next,
+                     static_cast<const Real*>(cx.adj_faces), lam_prev, grad, g.nchunk, mom, FLOW ? ubar : nullptr,
+                     inv_vol);
 }
 
 // One adjoint step.  Lam = double: every configuration; Lam = float (FP32
@@ -747,20 +829,19 @@ hipError_t run_adjoint(Ctx& cx, const void* f, const Lam* lam_next, Lam* lam_pre
   if (fpart && !handled) return hipErrorNotSupported;
   {
     if (compact) {
-      const int TZ = gather_z_chunk(P, sizeof(Real) == 8);
-      dim3 grid(P.n[0] / kGX, P.n[1] / kGY, (P.n[2] + TZ - 1) / TZ);
-      const double inv_vol = 1.0 / (cx.s.width[0] * cx.s.width[1] * cx.s.width[2]);
+      const GatherPlan g = gather_plan(P, sizeof(Real) == 8);
+      bool flow = false;
       if constexpr (kFuse) {
-        if (ubar) {
-          hipLaunchKernelGGL((k_adj_cells_z<Real, Store, Lam, true>), grid, dim3(kGT), 0, cx.stream, P,
-                             static_cast<const Store*>(f), lam_next, static_cast<const Real*>(cx.adj_faces),
-                             lam_prev, grad, TZ, mom, ubar, inv_vol);
-          return hipGetLastError();
-        }
+        flow = ubar != nullptr;
+        if (flow && g.rows == 12)
+          launch_gather<Real, Store, Lam, 12, true>(cx, g, f, lam_next, lam_prev, grad, mom, ubar);
+        else if (flow)
+          launch_gather<Real, Store, Lam, 8, true>(cx, g, f, lam_next, lam_prev, grad, mom, ubar);
       }
-      hipLaunchKernelGGL((k_adj_cells_z<Real, Store, Lam>), grid, dim3(kGT), 0, cx.stream, P,
-                         static_cast<const Store*>(f), lam_next, static_cast<const Real*>(cx.adj_faces), lam_prev,
-                         grad, TZ, mom, nullptr, inv_vol);
+      if (!flow && g.rows == 12)
+        launch_gather<Real, Store, Lam, 12, false>(cx, g, f, lam_next, lam_prev, grad, mom, ubar);
+      else if (!flow)
+        launch_gather<Real, Store, Lam, 8, false>(cx, g, f, lam_next, lam_prev, grad, mom, ubar);
       return hipGetLastError();
     }
   }

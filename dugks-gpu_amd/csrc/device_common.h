@@ -161,6 +161,29 @@ struct RawBuf {
     typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
     __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, v), r, (int)vb, (int)sb, 0);
   }
+  // four values side by side, in 16-byte accesses
+  typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+  template <class T>
+  __device__ __forceinline__ void ld4(unsigned vb, T (&v)[4]) const {
+    constexpr int VB = 16 / sizeof(T);
+    typedef T vec __attribute__((ext_vector_type(VB)));
+    static_for<4 / VB>([&](auto B) {
+      constexpr int b = decltype(B)::value;
+      const vec x = __builtin_bit_cast(vec, (u32x4)__builtin_amdgcn_raw_buffer_load_b128(r, (int)vb, b * 16, 0));
+      for (int q = 0; q < VB; q++) v[b * VB + q] = x[q];
+    });
+  }
+  template <class T>
+  __device__ __forceinline__ void st4(const T (&v)[4], unsigned vb) const {
+    constexpr int VB = 16 / sizeof(T);
+    typedef T vec __attribute__((ext_vector_type(VB)));
+    static_for<4 / VB>([&](auto B) {
+      constexpr int b = decltype(B)::value;
+      vec x;
+      for (int q = 0; q < VB; q++) x[q] = v[b * VB + q];
+      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, x), r, (int)vb, b * 16, 0);
+    });
+  }
 };
 template <>
 __device__ __forceinline__ float RawBuf::ld<float>(unsigned vb, unsigned sb) const {

@@ -86,15 +86,14 @@ hipError_t launch_step_fused(Ctx& c, const void* fin, void* fout, bool* handled)
 // when the fused kernel does not cover the configuration.  Face record
 // formats: kFacesFull, the 19 reconstructed-value cotangents per face, lam'
 // in FP64; kFacesCompact (the z-marching gather's configurations, FP32 or
-// FP64 arithmetic; adjoint_record_format), kCompact values per face:
-// the reconstructed-value cotangents of the ten populations crossing the face
-// (fw1 mu + Ac + B.c), then Ac and the two tangential components of B, from
-// which the nine others follow; kFacesCompactLam32, the same with lam' in FP32.
+// FP64 arithmetic; adjoint_record_format), kCompact values per face: Ac and B
+// of the cotangents fw1 mu + Ac + B.c, whose mu the gather forms from lam';
+// kFacesCompactLam32, the same with lam' in FP32.
 // With the state stored in the arithmetic type (FP32 or FP64 storage) the
 // compact formats also carry, after the three record arrays (at 3 kCompact eN
-// values), two regions of rho, j_x, j_y, j_z of every cell ([4][N] each),
+// values), two regions of rho, j_x, j_y, j_z of every cell ([N][4] each),
 // which the gather uses instead of reading f.
-constexpr int kCompact = 13;
+constexpr int kCompact = 4;
 constexpr int kFacesFull = 0, kFacesCompact = 1, kFacesCompactLam32 = 2;
 // With fpart set, the pass also writes per block the cotangent of the
 // ambient force along the flow axis through the face collisions (nparts

@@ -16,6 +16,14 @@ __device__ constexpr int dirs(int k) {
   return A == 0 ? XD[k] : (A == 1 ? YD[k] : ZD[k]);
 }
 
+// v, opaque to the optimiser: what is formed from it is formed at its use and
+// does not live in registers across the plane loop.
+template <class T>
+__device__ __forceinline__ T here(T v) {
+  asm volatile("" : "+v"(v));
+  return v;
+}
+
 // (1 - m) a + m b, evaluated as a + m (b - a): a constant stays exactly
 // constant whatever the rounding of m.  In FP32, (1 - m) and m rounded apart
 // do not sum to 1, which on a stretched axis biases every face value by a
@@ -161,47 +169,22 @@ __device__ __forceinline__ void expand_cotangents(const Real (&mu)[10], Real Ac,
   bounce_transpose<Real, A>(post, low_wall, high_wall, lam);
 }
 
-// Compact face record (kCompact values): the cotangents fw1 mu_k + Ac + B.c_p
-// of the ten crossing populations, then Ac and the two components of B
-// tangential to the face.  The nine other populations have c_A = 0, so B_A
-// only enters the crossing ones.
-template <int A>
-__device__ constexpr int tangential(int t) {
-  return t == 0 ? (A == 0 ? 1 : 0) : (A == 2 ? 1 : 2);
+// The compact form of the adjoint's face data.  The cotangent of a
+// reconstructed value of a face is fw1 mu_p + Ac + B.c_p, and mu (of the
+// crossing populations) is a difference of lam' between the two cells beside
+// the face; so a face record is (Ac, B), four values side by side, one array
+// per axis ([3][slot][4]), and the gather forms mu from the lam' it reads
+// anyway.  Behind the records (storage in the arithmetic type) lie two regions
+// of (rho, j) of every cell ([2][N][4]).
+template <class Real>
+__device__ __forceinline__ RawBuf face_records(const void* faces, int axis, long long eN) {
+  return RawBuf(static_cast<const Real*>(faces) + axis * kCompact * eN,
+                (unsigned)(kCompact * eN * (long long)sizeof(Real)));
 }
-template <class Real, int A>
-__device__ __forceinline__ void compact_record(const Real (&mu)[10], Real Ac, const Real (&B)[3], Real fw1,
-                                               Real (&rec)[kCompact]) {
-  static_for<10>([&](auto K) {
-    constexpr int k = decltype(K)::value;
-    constexpr int ip = dirs<A>(k);
-    rec[k] = plus_cdot<ip>(Ac, B[0], B[1], B[2]) + fw1 * mu[k];
-  });
-  rec[10] = Ac;
-  rec[11] = B[tangential<A>(0)];
-  rec[12] = B[tangential<A>(1)];
-}
-
-// The 19 reconstructed-value cotangents of a compact record (as
-// expand_cotangents of the coefficients it was made from).
-template <class Real, int A>
-__device__ __forceinline__ void expand_record(const Real (&rec)[kCompact], bool low_wall, bool high_wall,
-                                              Real (&lam)[Q]) {
-  Real B[3];
-  B[A] = Real(0);
-  B[tangential<A>(0)] = rec[11];
-  B[tangential<A>(1)] = rec[12];
-  const Real Ac = rec[10];
-  Real post[Q];
-  static_for<Q>([&](auto I) {
-    constexpr int ip = decltype(I)::value;
-    constexpr int k = cross_index<A>(ip);
-    if constexpr (k >= 0)
-      post[ip] = rec[k];
-    else
-      post[ip] = plus_cdot<ip>(Ac, B[0], B[1], B[2]);
-  });
-  bounce_transpose<Real, A>(post, low_wall, high_wall, lam);
+template <class Real>
+__device__ __forceinline__ RawBuf cell_records(const void* faces, int region, long long eN, long long N) {
+  return RawBuf(static_cast<const Real*>(faces) + 3 * kCompact * eN + region * 4 * N,
+                (unsigned)(4 * N * (long long)sizeof(Real)));
 }
 
 // First population that does not cross a face normal to axis A and has a

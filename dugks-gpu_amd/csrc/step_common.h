@@ -84,14 +84,6 @@ __device__ __forceinline__ double uniform(double x) {
   const unsigned hi = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)(b >> 32));
   return __builtin_bit_cast(double, (unsigned long long)lo | (unsigned long long)hi << 32);
 }
-// v, opaque to the optimiser: what is formed from it is formed at its use and
-// does not live in registers across the plane loop.
-template <class T>
-__device__ __forceinline__ T here(T v) {
-  asm volatile("" : "+v"(v));
-  return v;
-}
-
 // v as a value of its own: keeps the optimiser from widening the load of an
 // array element that starts a vector into a load of the array's memory, which
 // would put the array into scratch.

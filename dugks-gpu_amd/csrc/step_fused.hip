@@ -73,8 +73,8 @@ struct Tile {
 struct AdjFaceIO {
   const void* lam;    // lam' = dJ/df(n+1), SoA [19][nz][ny][nx], FP64 or (LamT = float) FP32
   void* faces;        // out: [3][19][ghost-inclusive face slot], arithmetic type; COMPACT:
-                      // [3][kCompact][slot], then (storage in the arithmetic type) two
-                      // [4][N] regions of rho, j of every cell
+                      // [3][slot][kCompact], then (storage in the arithmetic type) two
+                      // [N][4] regions of rho, j of every cell
   int mom = 0;        // COMPACT, such storage: the region the pass writes rho, j of fin into
   // sweep through the flow-rate controller: lam' still lacks the bulk
   // velocity's cotangent ubar (dV/V) (c_ia - u_a)/rho of f(n+1), whose rho, j
@@ -275,8 +275,7 @@ __global__ void __launch_bounds__(((TY + 2) * TX + 2 * (TY + 2) + 63) / 64 * 64,
   // lam' is used: lam'_i += s (c_ia - u_a), s = ubar (dV/V) / rho
   constexpr bool kFlowFuse = FADJ && COMPACT && std::is_same<Store, Real>::value;
   const bool fuse = kFlowFuse && adj.ubar != nullptr;
-  const RawBuf momn(static_cast<Real*>(adj.faces) + 3LL * kCompact * P.eN + (1 - adj.mom) * 4LL * P.N,
-                    (unsigned)(4 * P.N * sizeof(Real)));
+  const RawBuf momn = cell_records<Real>(adj.faces, 1 - adj.mom, P.eN, P.N);
   Real s0 = Real(0), ex = Real(0), ey = Real(0), ez = Real(0);
   if constexpr (kFlowFuse) {
     if (fuse && lam_cell)
@@ -287,10 +286,10 @@ __global__ void __launch_bounds__(((TY + 2) * TX + 2 * (TY + 2) + 63) / 64 * 64,
   }
   auto load_flow = [&](int k, Real& rn, Real& jn) {
     if constexpr (kFlowFuse) {
-      const unsigned vb = fuse && lam_cell ? (unsigned)(((long long)k * ny + gj) * nx + gi) * sizeof(Real)
+      const unsigned vb = fuse && lam_cell ? (unsigned)(((long long)k * ny + gj) * nx + gi) * 4u * sizeof(Real)
                                            : kOutOfRange;
       rn = momn.ld<Real>(vb, 0);
-      jn = momn.ld<Real>(vb, (unsigned)((1 + as) * P.N * sizeof(Real)));
+      jn = momn.ld<Real>(vb, (unsigned)(1 + as) * (unsigned)sizeof(Real));
     }
   };
   auto add_flow = [&](Real (&l)[Q], Real rn, Real jn) {
@@ -311,14 +310,10 @@ __global__ void __launch_bounds__(((TY + 2) * TX + 2 * (TY + 2) + 63) / 64 * 64,
     load_flow(z0, rn, jn);
     add_flow(lamc, rn, jn);
   }
-  // compact form (COMPACT): per face the kCompact values of compact_record
-  auto store_compact = [&](int a, long long slot, const Real (&rec)[kCompact]) {
-    const RawBuf fb(static_cast<Real*>(adj.faces) + (long long)a * kCompact * P.eN, kCompact * face_pop);
-    const unsigned vb = (unsigned)slot * (unsigned)sizeof(Real);
-    static_for<kCompact>([&](auto K) {
-      constexpr int k = decltype(K)::value;
-      fb.st(rec[k], vb, k * face_pop);
-    });
+  // compact form (COMPACT): Ac and B of a face
+  auto store_compact = [&](int a, long long slot, Real Ac, const Real (&B)[3]) {
+    const Real rec[kCompact] = {Ac, B[0], B[1], B[2]};
+    face_records<Real>(adj.faces, a, P.eN).st4(rec, (unsigned)slot * (unsigned)(kCompact * sizeof(Real)));
   };
   auto store_face = [&](int a, long long slot, const Real (&lam)[Q]) {
     const RawBuf fb(static_cast<Real*>(adj.faces) + (long long)a * Q * P.eN, Q * face_pop);
@@ -373,14 +368,9 @@ __global__ void __launch_bounds__(((TY + 2) * TX + 2 * (TY + 2) + 63) / 64 * 64,
   // A chunk writes its planes z0+1 .. zend (mod nz), so the chunks cover
   // every plane once.
   auto store_moments = [&](int k, Real rho, const Real (&jm)[3]) {
-    const RawBuf mb(static_cast<Real*>(adj.faces) + 3LL * kCompact * P.eN + adj.mom * 4LL * P.N,
-                    (unsigned)(4 * P.N * sizeof(Real)));
-    const unsigned vb = (((unsigned)k * ny + gj) * nx + gi) * (unsigned)sizeof(Real);
-    const unsigned pop = (unsigned)(P.N * sizeof(Real));
-    mb.st(rho, vb, 0);
-    mb.st(jm[0], vb, pop);
-    mb.st(jm[1], vb, 2 * pop);
-    mb.st(jm[2], vb, 3 * pop);
+    const Real rec[4] = {rho, jm[0], jm[1], jm[2]};
+    cell_records<Real>(adj.faces, adj.mom, P.eN, P.N)
+        .st4(rec, (unsigned)(((long long)k * ny + gj) * nx + gi) * (unsigned)(4 * sizeof(Real)));
   };
   // One plane p: fbc / lamc hold f-bar+ and lam' of plane p, and the plane
   // computes those of p + 1 into fbn / lamn.
@@ -469,10 +459,9 @@ __global__ void __launch_bounds__(((TY + 2) * TX + 2 * (TY + 2) + 63) / 64 * 64,
       const int slot = gi + ((gi == 0 && P.periodic[0]) ? nx : 0);
       const long long fs = ((long long)(p + 1) * e1 + (gj + 1)) * e0 + slot;
       if constexpr (COMPACT) {
-        Real Ac, B[3], rec[kCompact];
+        Real Ac, B[3];
         fc.template adjoint_coeffs<FADJ>(Famb, hdt, fw0, fw2, mu, Ac, B, fsum);
-        compact_record<Real, 0>(mu, Ac, B, fw1, rec);
-        store_compact(0, fs, rec);
+        store_compact(0, fs, Ac, B);
       } else {
         fc.template adjoint<FADJ>(Famb, hdt, fw0, fw1, fw2, mu, lw, hw, lam, fsum);
         store_face(0, fs, lam);
@@ -509,10 +498,9 @@ __global__ void __launch_bounds__(((TY + 2) * TX + 2 * (TY + 2) + 63) / 64 * 64,
       const int slot = gj + ((gj == 0 && P.periodic[1]) ? ny : 0);
       const long long fs = ((long long)(p + 1) * e1 + slot) * e0 + (gi + 1);
       if constexpr (COMPACT) {
-        Real Ac, B[3], rec[kCompact];
+        Real Ac, B[3];
         fc.template adjoint_coeffs<FADJ>(Famb, hdt, fw0, fw2, mu, Ac, B, fsum);
-        compact_record<Real, 1>(mu, Ac, B, fw1, rec);
-        store_compact(1, fs, rec);
+        store_compact(1, fs, Ac, B);
       } else {
         fc.template adjoint<FADJ>(Famb, hdt, fw0, fw1, fw2, mu, lw, hw, lam, fsum);
         store_face(1, fs, lam);
@@ -532,10 +520,9 @@ __global__ void __launch_bounds__(((TY + 2) * TX + 2 * (TY + 2) + 63) / 64 * 64,
       });
       const long long fs = ((long long)(p + 1) * e1 + (gj + 1)) * e0 + (gi + 1);
       if constexpr (COMPACT) {
-        Real Ac, B[3], rec[kCompact];
+        Real Ac, B[3];
         fc.template adjoint_coeffs<FADJ>(Famb, hdt, fw0, fw2, mu, Ac, B, fsum);
-        compact_record<Real, 2>(mu, Ac, B, fw1, rec);
-        store_compact(2, fs, rec);
+        store_compact(2, fs, Ac, B);
       } else {
         fc.template adjoint<FADJ>(Famb, hdt, fw0, fw1, fw2, mu, false, false, lam, fsum);
         store_face(2, fs, lam);

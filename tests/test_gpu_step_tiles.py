@@ -137,16 +137,18 @@ def test_planar_statistics_over_row_counts(rng, nx):
     assert np.abs(diag[8:12] - [a.max() for a in fields]).max() <= 1e-15
 
 
-@pytest.mark.parametrize("nz", [1, 3, 32, 67])
+@pytest.mark.parametrize("n", [(32, 24, 1), (32, 24, 3), (64, 8, 32), (32, 40, 67), (64, 16, 5)], ids=str)
+@pytest.mark.parametrize("walls", ["periodic", "walls_y", "walls_x"])
 @pytest.mark.parametrize("precision", [PREC_FP64, PREC_FP32], ids=["fp64", "fp32"])
-def test_adjoint_step_over_chunk_counts(rng, precision, nz):
+def test_adjoint_step_over_tiles_and_chunks(rng, precision, walls, n):
     """lam.(df) = lam_prev.(df0) for the adjoint step over chunks of one plane,
-    of a few, and of unequal length, against the finite difference of the FP64
+    of a few, and of unequal length, and over tiles that overlap, that fill the
+    grid's height and that exceed it, against the finite difference of the FP64
     step (central, 1e-6 of a unit perturbation: truncation and cancellation
     1e-8 of the sums of 1e4 terms)."""
     torch = pytest.importorskip("torch")
-    text = configs.base(nx=32, ny=24, nz=nz, xwidth=3.2, ywidth=2.4, zwidth=0.1 * nz, visc=0.02, periods_y=0,
-                        ambient_fx=2e-4)
+    text = configs.base(nx=n[0], ny=n[1], nz=n[2], xwidth=n[0] / 10, ywidth=n[1] / 10, zwidth=n[2] / 10, visc=0.02,
+                        CFL=0.5, ambient_fx=2e-4, **RAGGED_WALLS[walls])
     eng = _engine(text, precision=precision, kernel=KERNEL_AUTO)
     ref = _engine(text, precision=PREC_FP64, kernel=KERNEL_AUTO)
     f0 = random_state(eng.shape, rng)
