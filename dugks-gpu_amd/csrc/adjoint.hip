@@ -358,7 +358,8 @@ __global__ void __launch_bounds__(256) k_adj_cells(KParams P, const Store* __res
 // wanted go out of range), so that every wait counts exactly.  Ring lanes run
 // the gather and the centre stage on clamped positions and store nothing: they
 // share SIMDs with one wave of cells where the others hold two.
-// 256x192x256 FP32: 0.98 ms, before 1.23; the face pass 1.09, before 1.41.
+// 256x192x256 FP32: 0.98 ms, before 1.23; the face pass 1.09, before 1.41 (0.86
+// since).
 // lanes of a workgroup, and LDS positions (the last ones idle)
 constexpr int gather_lanes(bool fp64, int rows) { return ((rows + 2) * (fp64 ? 18 : 34) + 63) / 64 * 64; }
 template <class Real, int ROWS>

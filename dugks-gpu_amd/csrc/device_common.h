@@ -714,19 +714,6 @@ struct RawCell {
         v[ip] = b.raw(vb, ip * Nb);
     });
   }
-  // Waits here for the loads of load() (an empty asm that reads and
-  // "writes" each slot): later reads of the slots then wait for nothing.
-  // The vector-memory counter counts loads and stores together, in issue
-  // order, so a wait for a load issued before a run of stores that the
-  // compiler cannot see on every path (stores under a branch) is compiled as
-  // a wait for those stores too; settling the slots before such stores
-  // avoids it.
-  __device__ __forceinline__ void settle() {
-    static_for<Q>([&](auto I) {
-      constexpr int ip = decltype(I)::value;
-      asm volatile("" : "+v"(v[ip]));
-    });
-  }
   // f, rho and the momentum velocity u0 = j/rho
   __device__ __forceinline__ void decode(const KParams& P, Real (&ff)[Q], Real& rho, Real (&u0)[3]) const {
     static_for<Q>([&](auto I) {
@@ -737,10 +724,6 @@ struct RawCell {
         ff[ip] = (Real)v[ip];
     });
     cell_rho_u<Real>(ff, rho, u0);
-  }
-  // the rho and j only (FP32 storage path of the adjoint-face pass)
-  __device__ __forceinline__ void moments(const Real (&ff)[Q], Real& rho, Real (&j)[3]) const {
-    cell_moments<Real>(ff, rho, j);
   }
 };
 // Adjoint of the equilibrium-with-force term (used by the adjoint of the

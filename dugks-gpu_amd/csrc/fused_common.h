@@ -1,6 +1,5 @@
-// Building blocks of the fused step kernel and the adjoint-face pass:
-// per-axis direction sets, f-bar+ of a (possibly wall-ghost) column, and the
-// face reconstruction record with its collision and the transpose of that
+// Building blocks of the fused step kernel and the adjoint passes: per-axis
+// direction sets, and a face's reconstruction record with the transpose of its
 // collision.  Included inside namespace dugks { namespace { ... } } of the
 // kernel files.
 #pragma once
@@ -40,89 +39,6 @@ __device__ __forceinline__ void ambient_force(const KParams& P, Real F[3]) {
   F[0] = (Real)P.famb_dev[0];
   F[1] = (Real)P.famb_dev[1];
   F[2] = (Real)P.famb_dev[2];
-}
-
-// f-bar+ of interior cell (i, j, k) (0-based).
-template <class Real, class Store>
-__device__ __forceinline__ void fbar_cell(const KParams& P, const StateBuf<Store>& f, unsigned Nb, int i, int j,
-                                          int k, const Real Famb[3], Real (&fb)[Q]) {
-  const unsigned c = ((unsigned)k * P.n[1] + j) * P.n[0] + i;
-  RawCell<Real, Store> raw;
-  raw.load(f, c, (unsigned)P.N);
-  Real ff[Q], rho, u0[3];
-  raw.decode(P, ff, rho, u0);
-  Real F[3] = {Famb[0], Famb[1], Famb[2]};
-  if (P.fcell) {
-    F[0] += (Real)P.fcell[c];
-    F[1] += (Real)P.fcell[P.N + c];
-    F[2] += (Real)P.fcell[2 * P.N + c];
-  }
-  centre_fbar<Real>(ff, rho, u0, F, (Real)P.hdt, (Real)P.bw0, (Real)P.bw2, fb);
-}
-
-// f-bar+ of a column that may be a wall ghost in x and/or y: the ghost value
-// is the linear extrapolation q f(1) + (1-q) f(2) from the wall side.
-// gi, gj are 0-based; a wall ghost is -1 or n; periodic indices are wrapped
-// by the caller.
-template <class Real, class Store>
-__device__ void fbar_column(const KParams& P, const StateBuf<Store>& f, unsigned Nb, int gi, int gj, int kz,
-                            const Real Famb[3], Real (&fb)[Q]) {
-  const bool gx = gi < 0 || gi >= P.n[0];
-  const bool gy = gj < 0 || gj >= P.n[1];
-  if (!gx && !gy) {
-    fbar_cell<Real, Store>(P, f, Nb, gi, gj, kz, Famb, fb);
-    return;
-  }
-  // the two columns (and weights) of the extrapolation along each ghost axis;
-  // a non-ghost axis uses the column itself with weight 1
-  int x0 = gi, x1 = gi, y0 = gj, y1 = gj;
-  Real qx = Real(1), qy = Real(1);
-  if (gx) {
-    const bool lo = gi < 0;
-    qx = (Real)(lo ? P.qlo[0] : P.qhi[0]);
-    x0 = lo ? 0 : P.n[0] - 1;
-    x1 = lo ? 1 : P.n[0] - 2;
-  }
-  if (gy) {
-    const bool lo = gj < 0;
-    qy = (Real)(lo ? P.qlo[1] : P.qhi[1]);
-    y0 = lo ? 0 : P.n[1] - 1;
-    y1 = lo ? 1 : P.n[1] - 2;
-  }
-  // The extrapolation q f(1) + (1 - q) f(2) along a ghost axis is taken as
-  // f(2) + q (f(1) - f(2)) (exact for constants, see lerp_); a corner ghost
-  // of two wall axes takes the tensor product of the two (the x -> y ghost
-  // fill of the reference gives the same linear combination).  f-bar+ has
-  // one code copy per case in a rolled loop, and no indexed local arrays
-  // (those would live in scratch memory): these lanes are few.
-  if (!(gx && gy)) {
-    const Real q = gx ? qx : qy;
-#pragma unroll 1
-    for (int k = 0; k < 2; k++) {
-      // k = 0: the second column (x1 or y1), k = 1: the first
-      const int ci = gx ? (k ? x0 : x1) : gi, cj = gy ? (k ? y0 : y1) : gj;
-      Real t[Q];
-      fbar_cell<Real, Store>(P, f, Nb, ci, cj, kz, Famb, t);
-      static_for<Q>([&](auto I) {
-        constexpr int ip = decltype(I)::value;
-        fb[ip] = k ? fma_rn(q, t[ip] - fb[ip], fb[ip]) : t[ip];
-      });
-    }
-    return;
-  }
-  bool first = true;
-#pragma unroll 1
-  for (int k = 0; k < 4; k++) {
-    const int a = k & 1, b = k >> 1;
-    const Real w = (a ? Real(1) - qx : qx) * (b ? Real(1) - qy : qy);
-    Real t[Q];
-    fbar_cell<Real, Store>(P, f, Nb, a ? x1 : x0, b ? y1 : y0, kz, Famb, t);
-    static_for<Q>([&](auto I) {
-      constexpr int ip = decltype(I)::value;
-      fb[ip] = first ? w * t[ip] : fb[ip] + w * t[ip];
-    });
-    first = false;
-  }
 }
 
 // Index of population ip in the crossing set of axis A (-1 if it does not

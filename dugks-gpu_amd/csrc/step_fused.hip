@@ -54,6 +54,7 @@ namespace dugks {
 namespace {
 
 #include "fused_common.h"
+#include "step_common.h"
 
 constexpr int kXcds = 8;  // accelerator complex dies of an MI355X
 
@@ -111,6 +112,13 @@ __device__ __forceinline__ Real grad_foot(Real m, Real h, Real gx, Real gy, Real
 // by lam' (adj.lam), are written to adj.faces; nothing else is written.  FADJ:
 // also the cotangent of the ambient force along the flow axis through the
 // face collisions, summed per block into partial[tile] (fixed order).
+//
+// What bounds it: with compact records the 38 loads and 4 wide stores of a
+// plane at issue, then the faces' arithmetic.  So the loads go out in three
+// groups (lam' after f-bar+, f of the plane after next between the faces), and
+// wall ghosts are extrapolated in LDS (the lanes of a ghost column formed f-bar+
+// of two columns from memory before, alone and waiting).  256x192x256 channel,
+// FP32: 0.86 ms, before 1.09; 64x64x32 FP64: 35 us, before 47.
 template <class Real, class Store, int TX, int TY, bool COMPACT = false, class LamT = double, bool FADJ = false>
 // FP32 arithmetic: two blocks per CU (at most 256 registers per lane)
 __global__ void __launch_bounds__(((TY + 2) * TX + 2 * (TY + 2) + 63) / 64 * 64, sizeof(Real) == 4 ? 2 : 1)
@@ -144,7 +152,6 @@ __global__ void __launch_bounds__(((TY + 2) * TX + 2 * (TY + 2) + 63) / 64 * 64,
   const int i0 = bx * TX, j0 = by * TY;
   const int z0 = bz * TZ;
   const int zend = min(z0 + TZ, nz);
-  const unsigned Nb = (unsigned)(P.N * (long long)sizeof(Store));  // bytes per population
   const unsigned span = (unsigned)state_bytes<Store>((unsigned long long)P.N);
   const StateBuf<Store> bin(fin, span);
 
@@ -217,17 +224,6 @@ __global__ void __launch_bounds__(((TY + 2) * TX + 2 * (TY + 2) + 63) / 64 * 64,
   // FADJ: the face collisions' force cotangents of this thread's faces
   double fsum[3] = {0, 0, 0};
 
-  // Zn(p+1/2) of this column into An: z-normal lerp between fb(p) and fb(p+1)
-  auto store_zn = [&](const Real (&lo)[Q], const Real (&hi)[Q]) {
-    if (!active) return;
-    static_for<Q>([&](auto I) {
-      constexpr int ip = decltype(I)::value;
-      if constexpr (ip == 0)
-        An[0][ia(r, c + 1)] = Real(0.5) * (lo[0] + hi[0]);
-      else
-        An[ip][ia(r, c + 1)] = lerp_(lo[ip], hi[ip], wzn[CZ[ip] + 1]);
-    });
-  };
   // +z face of an interior column from Zn in A: bilinear over the upwind
   // tangential neighbours, then collision; out = crossing populations
   auto zface_rec = [&](Face<Real, 2>& fc) {
@@ -311,9 +307,10 @@ __global__ void __launch_bounds__(((TY + 2) * TX + 2 * (TY + 2) + 63) / 64 * 64,
     add_flow(lamc, rn, jn);
   }
   // compact form (COMPACT): Ac and B of a face
-  auto store_compact = [&](int a, long long slot, Real Ac, const Real (&B)[3]) {
+  auto store_compact = [&](int a, long long slot, Real Ac, const Real (&B)[3], bool ok = true) {
     const Real rec[kCompact] = {Ac, B[0], B[1], B[2]};
-    face_records<Real>(adj.faces, a, P.eN).st4(rec, (unsigned)slot * (unsigned)(kCompact * sizeof(Real)));
+    face_records<Real>(adj.faces, a, P.eN)
+        .st4(rec, ok ? (unsigned)slot * (unsigned)(kCompact * sizeof(Real)) : kOutOfRange);
   };
   auto store_face = [&](int a, long long slot, const Real (&lam)[Q]) {
     const RawBuf fb(static_cast<Real*>(adj.faces) + (long long)a * Q * P.eN, Q * face_pop);
@@ -326,42 +323,67 @@ __global__ void __launch_bounds__(((TY + 2) * TX + 2 * (TY + 2) + 63) / 64 * 64,
   const long long e0 = P.e[0], e1 = P.e[1];
 
   // Columns inside the domain (tile and periodic halo) compute f-bar+ from f
-  // of their own column; wall ghost columns extrapolate it (fbar_column).
+  // of their own column; wall ghost columns are extrapolated in LDS.
   const bool own = active && gi >= 0 && gi < nx && gj >= 0 && gj < ny;
-  // stored f of the own column at plane k (decoded at use)
-  auto load_own = [&](int k, RawCell<Real, Store>& raw) { raw.load(bin, ((unsigned)k * ny + gj) * nx + gi, (unsigned)P.N); };
   // body force at plane k of the own column
   auto force_own = [&](int k, Real (&F)[3]) {
     F[0] = Famb[0];
     F[1] = Famb[1];
     F[2] = Famb[2];
-    if (P.fcell) {
+    if (P.fcell && own) {
       const unsigned cc = ((unsigned)k * ny + gj) * nx + gi;
       F[0] += (Real)P.fcell[cc];
       F[1] += (Real)P.fcell[P.N + cc];
       F[2] += (Real)P.fcell[2 * P.N + cc];
     }
   };
-  // f of the own column one plane ahead of its f-bar: the loads are issued
-  // one iteration before their f-bar needs them.  The first (plane z0+1) is
-  // issued ahead of the pre-loop's loads, so it arrives with them.
-  RawCell<Real, Store> fpre;
-  if (own) load_own((z0 + 1) % nz, fpre);
+  // f of the own column (other lanes load zeros) one plane ahead of its f-bar.
+  // The loads go out in two groups between the faces: in one burst with those
+  // of lam' they fill the memory pipeline and the wave stalls at issue.
+  using Raw = RawLane<false, Real, Store>;
+  const unsigned column = (unsigned)(gj * nx + gi), nxy = (unsigned)nx * (unsigned)ny;
+  auto load_part = [&](auto X, auto Y, int k, Raw& raw) {
+    raw.template load<decltype(X)::value, decltype(Y)::value>(
+        bin, LaneOffsets<false, Store>(column, (unsigned)P.N, 0).where(own, true, span), (unsigned)k * nxy,
+        (unsigned)P.N);
+  };
+  using L0 = std::integral_constant<int, 0>;
+  using L1 = std::integral_constant<int, 10>;
+  using L2 = std::integral_constant<int, Q>;
+  Raw fpre;
+  load_part(L0{}, L2{}, (z0 + 1) % nz, fpre);
 
   // ---- pre-loop: f-bar at z0-1 and z0 ----
   {
+    Raw lo, hi;
     const int km = (z0 - 1 + nz) % nz;
-    if (active) {
-      fbar_column<Real, Store>(P, bin, Nb, gi, gj, km, Famb, fbn);
-      fbar_column<Real, Store>(P, bin, Nb, gi, gj, z0, Famb, fbc);
-      static_for<5>([&](auto K) {
-        constexpr int k = decltype(K)::value;
-        fbm[k] = fbn[ZP[k]];
-      });
-    }
+    load_part(L0{}, L2{}, km, lo);
+    load_part(L0{}, L2{}, z0, hi);
+    Real F[3], ff[Q], rho, u0[3];
+    force_own(km, F);
+    lo.template decode<false>(P, Real(1), ff, rho, u0);
+    centre_fbar<Real>(ff, rho, u0, F, hdt, (Real)P.bw0, (Real)P.bw2, fbn);
+    force_own(z0, F);
+    hi.template decode<false>(P, Real(1), ff, rho, u0);
+    centre_fbar<Real>(ff, rho, u0, F, hdt, (Real)P.bw0, (Real)P.bw2, fbc);
+    static_for<5>([&](auto K) {
+      constexpr int k = decltype(K)::value;
+      fbm[k] = fbn[ZP[k]];
+    });
   }
 
-  fpre.settle();
+  // The wall ghost that the lane's column extrapolates (the column at the wall
+  // does, from itself and the next one, which is in the same wave: rows in
+  // pairs, halo columns in one wave), as q f(1) + (1 - q) f(2) taken as f(2) +
+  // q (f(1) - f(2)).  Z and Zn are linear in f-bar+ with weights shared by the
+  // columns, so their ghosts extrapolate as f-bar+ does.  At most one wall axis.
+  static_assert(TX * TY % 64 == 0 && 64 / TX % 2 == 0 && T::NROW % 64 + T::NHALO <= 64, "columns of a wave");
+  const bool xin = own && !P.periodic[0] && c >= 0 && c < TX, yin = own && !P.periodic[1] && r >= 1 && r <= TY;
+  const int gdx = !xin ? 0 : (gi == 0 ? -1 : (gi == nx - 1 ? 1 : 0));
+  const int gdy = !yin ? 0 : (gj == 0 ? -1 : (gj == ny - 1 ? 1 : 0));
+  const Real gqx = gdx < 0 ? uniform((Real)P.qlo[0]) : uniform((Real)P.qhi[0]);
+  const Real gqy = gdy < 0 ? uniform((Real)P.qlo[1]) : uniform((Real)P.qhi[1]);
+
   // compact adjoint-face records with the state stored in the arithmetic
   // type (FP32 or FP64): rho and j of every cell
   // for the gather, written by the interior lanes from the prefetched f.
@@ -378,13 +400,11 @@ __global__ void __launch_bounds__(((TY + 2) * TX + 2 * (TY + 2) + 63) / 64 * 64,
   // in scratch memory, 3.8 against 2.7 ms an adjoint step on 256x192x256.)
   auto plane = [&](int p, Real (&fbc)[Q], Real (&fbn)[Q], Real (&lamc)[Q], Real (&lamn)[Q]) {
     const int kn = (p + 1) % nz;
-    load_lam(kn, lamn);
-    load_flow(kn, rnn, jnn);
-    if (own) {
+    {
       Real F[3];
       force_own(kn, F);
       Real ff[Q], rho, u0[3];
-      fpre.decode(P, ff, rho, u0);
+      fpre.template decode<false>(P, Real(1), ff, rho, u0);
       if constexpr (COMPACT && std::is_same<Store, Real>::value) {
         if (interior) {
           Real jm[3];
@@ -393,26 +413,46 @@ __global__ void __launch_bounds__(((TY + 2) * TX + 2 * (TY + 2) + 63) / 64 * 64,
         }
       }
       centre_fbar<Real>(ff, rho, u0, F, hdt, (Real)P.bw0, (Real)P.bw2, fbn);
-      if (p + 1 < zend) load_own((p + 2) % nz, fpre);
-    } else if (active) {
-      fbar_column<Real, Store>(P, bin, Nb, gi, gj, kn, Famb, fbn);
     }
+    load_lam(kn, lamn);
+    load_flow(kn, rnn, jnn);
     // ---- phase 1: Z(p) (tangential z-lerp of f-bar(p)) and Zn(p+1/2) ----
-    if (active) {
+    Real zt[Q], zn[Q];
+    static_for<Q>([&](auto I) {
+      constexpr int ip = decltype(I)::value;
+      constexpr int cz = CZ[ip];
+      if constexpr (cz == 0) {
+        zt[ip] = fbc[ip];
+      } else if constexpr (cz > 0) {
+        constexpr int zk = ip == 5 ? 0 : (ip == 11 ? 1 : (ip == 12 ? 2 : (ip == 15 ? 3 : 4)));
+        zt[ip] = lerp_(fbc[ip], fbm[zk], wzt_p);
+      } else {
+        zt[ip] = lerp_(fbc[ip], fbn[ip], wzt_m);
+      }
+      if constexpr (ip == 0)
+        zn[0] = Real(0.5) * (fbc[0] + fbn[0]);
+      else
+        zn[ip] = lerp_(fbc[ip], fbn[ip], wzn[cz + 1]);
+    });
+    if (own) {
       static_for<Q>([&](auto I) {
         constexpr int ip = decltype(I)::value;
-        constexpr int cz = CZ[ip];
-        if constexpr (cz == 0) {
-          A[ip][ia(r, c + 1)] = fbc[ip];
-        } else if constexpr (cz > 0) {
-          constexpr int zk = ip == 5 ? 0 : (ip == 11 ? 1 : (ip == 12 ? 2 : (ip == 15 ? 3 : 4)));
-          A[ip][ia(r, c + 1)] = lerp_(fbc[ip], fbm[zk], wzt_p);
-        } else {
-          A[ip][ia(r, c + 1)] = lerp_(fbc[ip], fbn[ip], wzt_m);
-        }
+        A[ip][ia(r, c + 1)] = zt[ip];
+        An[ip][ia(r, c + 1)] = zn[ip];
       });
     }
-    store_zn(fbc, fbn);
+    if (gdx != 0 || gdy != 0) {
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      const int g = ia(r + gdy, c + 1 + gdx), i2 = ia(r - gdy, c + 1 - gdx);
+      const Real q = gdx != 0 ? gqx : gqy;
+      static_for<Q>([&](auto I) {
+        constexpr int ip = decltype(I)::value;
+        const Real a2 = A[ip][i2], n2 = An[ip][i2];
+        A[ip][g] = fma_rn(q, zt[ip] - a2, a2);
+        An[ip][g] = fma_rn(q, zn[ip] - n2, n2);
+      });
+    }
     if (active) {
       static_for<Q>([&](auto I) {
         constexpr int ip = decltype(I)::value;
@@ -467,6 +507,8 @@ __global__ void __launch_bounds__(((TY + 2) * TX + 2 * (TY + 2) + 63) / 64 * 64,
         store_face(0, fs, lam);
       }
     }
+    const int kp = (p + 2) % nz;
+    load_part(L0{}, L1{}, kp, fpre);
     if (do_y) {
       // face between y-rows gj-1 (below) and gj
       Face<Real, 1> fc;
@@ -506,8 +548,11 @@ __global__ void __launch_bounds__(((TY + 2) * TX + 2 * (TY + 2) + 63) / 64 * 64,
         store_face(1, fs, lam);
       }
     }
-    // lam' of plane p+1 complete (its loads were issued at the top of the plane)
+    load_part(L1{}, L2{}, kp, fpre);
+    // lam' of plane p+1 complete (its loads were issued in phase 1)
     if constexpr (kFlowFuse) add_flow(lamn, rnn, jnn);
+    Real zA = Real(0), zB[3] = {Real(0), Real(0), Real(0)};
+    const long long zs = ((long long)(p + 1) * e1 + (gj + 1)) * e0 + (gi + 1);
     if (interior) {
       // +z face of the cell: between planes p and p+1 (z is periodic)
       Face<Real, 2> fc;
@@ -518,33 +563,28 @@ __global__ void __launch_bounds__(((TY + 2) * TX + 2 * (TY + 2) + 63) / 64 * 64,
         constexpr int ip = ZD[k];
         mu[k] = Real(CZ[ip]) * updz * (lamn[ip] - lamc[ip]);
       });
-      const long long fs = ((long long)(p + 1) * e1 + (gj + 1)) * e0 + (gi + 1);
       if constexpr (COMPACT) {
-        Real Ac, B[3];
-        fc.template adjoint_coeffs<FADJ>(Famb, hdt, fw0, fw2, mu, Ac, B, fsum);
-        store_compact(2, fs, Ac, B);
+        fc.template adjoint_coeffs<FADJ>(Famb, hdt, fw0, fw2, mu, zA, zB, fsum);
       } else {
         fc.template adjoint<FADJ>(Famb, hdt, fw0, fw1, fw2, mu, false, false, lam, fsum);
-        store_face(2, fs, lam);
+        store_face(2, zs, lam);
       }
     }
+    // without a branch: the next plane's wait for the loads above does not cover it
+    if constexpr (COMPACT) store_compact(2, zs, zA, zB, interior);
     __syncthreads();
-    if (active) {
-      static_for<5>([&](auto K) {
-        constexpr int k = decltype(K)::value;
-        fbm[k] = fbc[ZP[k]];
-      });
-    }
+    static_for<5>([&](auto K) {
+      constexpr int k = decltype(K)::value;
+      fbm[k] = fbc[ZP[k]];
+    });
   };
   for (int p = z0; p < zend; p++) {
     plane(p, fbc, fbn, lamc, lamn);
-    if (active) {
-      static_for<Q>([&](auto I) {
-        constexpr int ip = decltype(I)::value;
-        fbc[ip] = fbn[ip];
-        if constexpr (ip != 0) lamc[ip] = lamn[ip];
-      });
-    }
+    static_for<Q>([&](auto I) {
+      constexpr int ip = decltype(I)::value;
+      fbc[ip] = fbn[ip];
+      if constexpr (ip != 0) lamc[ip] = lamn[ip];
+    });
   }
 
   if constexpr (FADJ) {
@@ -559,7 +599,6 @@ __global__ void __launch_bounds__(((TY + 2) * TX + 2 * (TY + 2) + 63) / 64 * 64,
   }
 }
 
-#include "step_common.h"
 #include "step_kernel.h"
 
 // Final reduction of the per-block flow sums <j/rho> dV and the flow-rate
@@ -584,8 +623,8 @@ __global__ void __launch_bounds__(256) k_flow_finish(const double* partial, int 
 // z-chunk length of the adjoint-face pass (plan_z_chunks; a chunk recomputes
 // f-bar+ of the two planes before it, about as long as one plane).  At most
 // 32 planes: several rounds even out the finish (256x192x256 FP32: 128 planes
-// 0.3 % slower).  On 64x64x32 FP64 (32 tiles, one workgroup per CU): 51 us
-// with 4-plane chunks, 86 with 8.
+// 0.3 % slower).  On 64x64x32 FP64 (32 tiles, one workgroup per CU) 4-plane
+// chunks took 51 us where 8-plane ones took 86.
 int blocks_per_cu(bool fp64, int TX, int TY) { return fp64 || Tile_nt(TX, TY) > 256 ? 1 : 2; }
 int z_chunk(const Ctx& cx, int TX, int TY) {
   const long long cols = (long long)(cx.kp.n[0] / TX) * (cx.kp.n[1] / TY);
