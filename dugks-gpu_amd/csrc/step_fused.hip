@@ -601,25 +601,6 @@ __global__ void __launch_bounds__(((TY + 2) * TX + 2 * (TY + 2) + 63) / 64 * 64,
 
 #include "step_kernel.h"
 
-// Final reduction of the per-block flow sums <j/rho> dV and the flow-rate
-// controller update (the law of k_flow_control).
-__global__ void __launch_bounds__(256) k_flow_finish(const double* partial, int nparts, double* famb, int axis,
-                                                     double volume, double target, double gain, double dt) {
-  double s[1] = {0};
-  for (int b = threadIdx.x; b < nparts; b += 256) s[0] += partial[b];
-  constexpr int kSum[1] = {0};
-  block_reduce<1, 256>(s, kSum);
-  if (threadIdx.x == 0) {
-    const double Ub = s[0] / volume;
-    const double Fprev = famb[axis];
-    double drag = Fprev;
-    if (famb[4] != 0) drag = Fprev - (Ub - famb[3]) / dt;
-    famb[axis] = drag + gain * (target - Ub) / dt;
-    famb[3] = Ub;
-    famb[4] = 1;
-  }
-}
-
 // z-chunk length of the adjoint-face pass (plan_z_chunks; a chunk recomputes
 // f-bar+ of the two planes before it, about as long as one plane).  At most
 // 32 planes: several rounds even out the finish (256x192x256 FP32: 128 planes
@@ -700,24 +681,18 @@ namespace {
 template <class Real, class Store, int TX, int TY, bool GRAD, bool RUNS>
 hipError_t run_step(Ctx& cx, const void* fin, void* fout, const StepPlan& plan) {
   using T = StepTile<Real, TX, TY, GRAD>;
-  double* partial = nullptr;
-  const bool flow = cx.s.flow_rate != 0 && !cx.flow_frozen;
-  if (flow) {
+  FlowLaw law{};
+  if (cx.s.flow_rate != 0 && !cx.flow_frozen) {
+    const Setup& s = cx.s;
     if ((size_t)plan.nblocks > cx.flow_partial_len) return hipErrorInvalidValue;
-    partial = cx.flow_partial;
+    law = {cx.flow_partial, reinterpret_cast<unsigned*>(cx.famb_dev + kFambArrived), cx.famb_dev,
+           s.width[0] * s.width[1] * s.width[2], s.flow_rate, s.flow_gain, s.dt};
   }
   if (cx.timing) hipEventRecord(cx.tev[0], cx.stream);
   hipLaunchKernelGGL((k_step<Real, Store, TX, TY, GRAD, RUNS>), dim3((unsigned)plan.nblocks), dim3(T::NT), 0, cx.stream,
-                     cx.kp, static_cast<const Store*>(fin), static_cast<Store*>(fout), plan.nchunk, plan.len,
-                     partial);
+                     cx.kp, static_cast<const Store*>(fin), static_cast<Store*>(fout), plan.nchunk, plan.len, law);
   if (cx.timing) hipEventRecord(cx.tev[1], cx.stream);
-  if (flow) {
-    const Setup& s = cx.s;
-    const double vol = s.width[0] * s.width[1] * s.width[2];
-    hipLaunchKernelGGL(k_flow_finish, dim3(1), dim3(256), 0, cx.stream, partial, (int)plan.nblocks, cx.famb_dev,
-                       s.stream_axis(), vol, s.flow_rate, s.flow_gain, s.dt);
-  }
-  cx.launches_per_step = flow ? 2 : 1;
+  cx.launches_per_step = 1;
   return hipGetLastError();
 }
 

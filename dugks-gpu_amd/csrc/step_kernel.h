@@ -8,6 +8,26 @@ constexpr int step_nw(bool pair, int TX, int TY) {
   return ((TY + 2) * (TX + 2) + step_unit(pair) - 1) / step_unit(pair);
 }
 
+// The flow-rate controller: where the workgroups leave their parts of the sum
+// over cells of u dV of the new state (nullptr: no controller), and how many
+// have; the force and the controller's state (flow_law), and its constants.
+struct FlowLaw {
+  double* partial;
+  unsigned* arrived;
+  double* famb;
+  double volume, target, gain, dt;
+};
+// One step of the controller on bulk velocity Ub (the law of k_flow_control;
+// famb: the force, then the previous bulk velocity and whether there is one).
+__device__ __forceinline__ void flow_law(double* famb, int axis, double Ub, double target, double gain, double dt) {
+  const double Fprev = famb[axis];
+  double drag = Fprev;
+  if (famb[4] != 0) drag = Fprev - (Ub - famb[3]) / dt;
+  famb[axis] = drag + gain * (target - Ub) / dt;
+  famb[3] = Ub;
+  famb[4] = 1;
+}
+
 template <class Real, int TX, int TY, bool GRAD>
 struct StepTile {
   static constexpr bool PAIR = sizeof(Real) == 8;
@@ -42,7 +62,7 @@ struct StepTile {
 template <class Real, class Store, int TX, int TY, bool GRAD, bool RUNS>
 __global__ void __launch_bounds__(step_nw(sizeof(Real) == 8, TX, TY) * 64, 2)
     k_step(KParams P, const Store* __restrict__ fin, Store* __restrict__ fout, int nchunk,
-           int len, double* __restrict__ partial) {
+           int len, FlowLaw law) {
   using T = StepTile<Real, TX, TY, GRAD>;
   constexpr bool PAIR = T::PAIR;
   constexpr int NQ = T::NQ, NX = T::NX, AC = T::AC, STR = T::STR, FS = T::FS, UNIT = T::UNIT;
@@ -592,7 +612,7 @@ __global__ void __launch_bounds__(step_nw(sizeof(Real) == 8, TX, TY) * 64, 2)
       });
       if constexpr (kNeq) {
         lane_rho_u<PAIR, Real>(fnew, rr, un, true);
-      } else if (partial) {
+      } else if (law.partial) {
         // the controller's reading only: sums in the arithmetic type suffice
         // (the moments that feed the step are summed in FP64, lane_rho_u)
         Real jn[3];
@@ -601,7 +621,7 @@ __global__ void __launch_bounds__(step_nw(sizeof(Real) == 8, TX, TY) * 64, 2)
         un[0] = cell_diff<PAIR>(as == 0 ? jn[0] : (as == 1 ? jn[1] : jn[2])) * rcp_real(rr);
       }
       // bulk velocity of the new state for the flow-rate controller
-      if (partial && stored) run_flow += (double)(!kNeq || as == 0 ? un[0] : (as == 1 ? un[1] : un[2]));
+      if (law.partial && stored) run_flow += (double)(!kNeq || as == 0 ? un[0] : (as == 1 ? un[1] : un[2]));
     }
     // Stores without a branch (lanes that store nothing address the end of
     // the array): the compiler then knows how many stores follow the loads
@@ -655,7 +675,7 @@ __global__ void __launch_bounds__(step_nw(sizeof(Real) == 8, TX, TY) * 64, 2)
     }
   }
 
-  if (partial) {
+  if (law.partial) {
     // every column of the tile has the same z width (z is uniform here)
     const Place w = place();
     if (stored && !w.half) flow += run_flow * (P.wd[0][i0 + w.c + 1] * P.wd[1][j0 + w.r] * P.wd[2][1]);
@@ -663,11 +683,28 @@ __global__ void __launch_bounds__(step_nw(sizeof(Real) == 8, TX, TY) * 64, 2)
   if constexpr (!RUNS) break;
   }
 
-  if (partial) {
-    // fixed-order block reduction of the flow sums
+  if (law.partial) {
+    // fixed-order block reduction of the flow sums; the last workgroup to get
+    // here adds them all up, in order, and moves the force (every workgroup
+    // read it at its start).  A launch of its own for that took 8 us a step.
     double v[1] = {flow};
     constexpr int kSum[1] = {0};
     block_reduce<1, T::NT>(v, kSum);
-    if (t == 0) partial[tt] = v[0];
+    __shared__ unsigned arrived;
+    if (t == 0) {
+      __hip_atomic_store(&law.partial[tt], v[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      arrived = __hip_atomic_fetch_add(law.arrived, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __syncthreads();
+    if (arrived == gridDim.x - 1) {
+      double sum[1] = {0.0};
+      for (int k = t; k < (int)gridDim.x; k += T::NT)
+        sum[0] += __hip_atomic_load(&law.partial[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      block_reduce<1, T::NT>(sum, kSum);
+      if (t == 0) {
+        flow_law(law.famb, as, sum[0] / law.volume, law.target, law.gain, law.dt);
+        *law.arrived = 0;  // for the next launch
+      }
+    }
   }
 }

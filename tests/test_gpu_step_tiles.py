@@ -97,7 +97,7 @@ def test_automatic_choice_of_ragged_grids():
         base = dict(nx=20, ny=17, nz=5, xwidth=2.0, ywidth=1.7, zwidth=0.5, visc=0.02)
         return _engine(configs.base(**{**base, **kw}), kernel=KERNEL_AUTO).time_steps(1)["launches_per_step"]
     assert launches() == 1
-    assert launches(periods_y=0, flow_rate=0.01, ambient_fx=1e-4) == 2
+    assert launches(periods_y=0, flow_rate=0.01, ambient_fx=1e-4) == 1  # the controller runs in the step
     assert launches(nz=1) == 5       # fewer than 512 cells
     assert launches(periods_z=0) == 5
 
