@@ -51,9 +51,9 @@ struct KParams {
 struct Ctx;
 
 // Ctx::famb_dev: the ambient force, the controller's previous bulk velocity and
-// whether there is one, then the count of the step's workgroups that are done
-// (0 between launches).
-constexpr int kFambArrived = 5;
+// whether there is one, then the counts of the step's and of the loss's
+// workgroups that are done (0 between launches).
+constexpr int kFambArrived = 5, kFambLossArrived = 6;
 
 // The number of z-chunks for `tiles` columns of nz planes, `slots` workgroups
 // resident at once and a prologue that costs as much as `prologue` planes: the
@@ -243,7 +243,7 @@ struct Ctx {
   double* tab[3] = {nullptr, nullptr, nullptr};
   double* wd[3] = {nullptr, nullptr, nullptr};
   float* tabf[3] = {nullptr, nullptr, nullptr};
-  double* famb_dev = nullptr; // 3 doubles + controller state + the step's arrival counter (kFambArrived)
+  double* famb_dev = nullptr; // 3 doubles + controller state + arrival counters (kFambArrived)
   double* fcell = nullptr;    // [3][N] additive centre force
   double* red = nullptr;      // reduction scratch
   size_t red_len = 0;

@@ -3,6 +3,7 @@
 #include <map>
 #include <mutex>
 
+#include <algorithm>
 #include "device_common.h"
 
 namespace dugks {
@@ -190,23 +191,32 @@ __global__ void __launch_bounds__(256) k_perturb(KParams P, int step, double xwi
 // planes only (2 nx nz of the N cells on a y-wall channel).
 // NV = 2: the second sum is dJ/dF_fa, the derivative with respect to the
 // ambient force component fa (both losses read h F).
+// A sweep takes the loss in every step, forward and back; on small grids its
+// cost is that of its launches, so a call is one launch with as many blocks as
+// have cells (up to kRedBlocks: the order of the sums is fixed by the grid).
+// Wall shear on 64x64x32 FP64: 9.2 us, before 7.8 and 4.5 for two launches of
+// 1024 blocks and of one.
+__host__ __device__ constexpr bool loss_wall_only(int kind, bool grad, double gacc) {
+  return kind == 0 && !(grad && gacc == 0.0);
+}
 template <class Store, class G, int NV = 1>
 __global__ void __launch_bounds__(kRedThreads) k_loss(KParams P, const Store* __restrict__ f, int kind,
                                                       int aw, int as, double visc, double vol,
                                                       double nplane, G* grad, double gacc,
-                                                      double* partial, int fa = 0) {
+                                                      double* partial, unsigned* arrived, double* out,
+                                                      int accumulate, int fa = 0) {
   double acc[NV];
   for (int q = 0; q < NV; q++) acc[q] = 0;
   double F[3];
   ambient_d(P, F);
-  const bool wall_only = kind == 0 && !(grad && gacc == 0.0);
+  const bool wall_only = loss_wall_only(kind, grad != nullptr, gacc);
   // in-plane axes of the wall planes, the faster-varying first, so that
   // consecutive threads read consecutive cells
   const int b1 = aw == 0 ? 1 : 0, b2 = aw == 2 ? 1 : 2;
   const long long npl = (long long)P.n[b1] * P.n[b2];
   const long long count = wall_only ? (P.n[aw] > 1 ? 2 : 1) * npl : P.N;
   for (long long w = (long long)blockIdx.x * kRedThreads + threadIdx.x; w < count;
-       w += (long long)kRedBlocks * kRedThreads) {
+       w += (long long)gridDim.x * kRedThreads) {
     int idx[3];
     long long c = w;
     if (wall_only) {
@@ -276,7 +286,26 @@ __global__ void __launch_bounds__(kRedThreads) k_loss(KParams P, const Store* __
       }
     }
   }
-  block_reduce_store<NV>(acc, partial);
+  // the last block to get here adds all blocks' sums up, in order
+  constexpr AllSums<NV> sums;
+  block_reduce<NV, kRedThreads>(acc, sums.op);
+  __shared__ unsigned before;
+  if (threadIdx.x == 0) {
+    for (int q = 0; q < NV; q++)
+      __hip_atomic_store(&partial[blockIdx.x * NV + q], acc[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    before = __hip_atomic_fetch_add(arrived, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  __syncthreads();
+  if (before != gridDim.x - 1) return;
+  for (int q = 0; q < NV; q++) acc[q] = 0;
+  for (int b = threadIdx.x; b < (int)gridDim.x; b += kRedThreads)
+    for (int q = 0; q < NV; q++)
+      acc[q] += __hip_atomic_load(&partial[b * NV + q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  block_reduce<NV, kRedThreads>(acc, sums.op);
+  if (threadIdx.x == 0) {
+    for (int q = 0; q < NV; q++) out[q] = (accumulate ? out[q] : 0.0) + acc[q];
+    *arrived = 0;  // for the next launch
+  }
 }
 
 __global__ void __launch_bounds__(256) k_axpy(double a, const double* __restrict__ x, double* y, long long n) {
@@ -446,19 +475,19 @@ hipError_t loss_t(Ctx& c, const void* f, int kind, double* value, G* grad, doubl
   if (fa > 2) return hipErrorInvalidValue;
   double vol = s.width[0] * s.width[1] * s.width[2];
   double nplane = aw >= 0 ? (double)s.ncell() / s.n[aw] : 1.0;
-  if (fa < 0) {
-    hipLaunchKernelGGL((k_loss<Store, G>), dim3(kRedBlocks), dim3(kRedThreads), 0, c.stream, c.kp,
-                       static_cast<const Store*>(f), kind, aw < 0 ? 0 : aw, as, s.visc, vol, nplane, grad,
-                       gacc, c.red, 0);
-    hipLaunchKernelGGL((k_reduce_final<1>), dim3(1), dim3(kRedThreads), 0, c.stream, c.red, kRedBlocks,
-                       value, vacc ? 1 : 0);
-  } else {
-    hipLaunchKernelGGL((k_loss<Store, G, 2>), dim3(kRedBlocks), dim3(kRedThreads), 0, c.stream, c.kp,
-                       static_cast<const Store*>(f), kind, aw < 0 ? 0 : aw, as, s.visc, vol, nplane, grad,
-                       gacc, c.red, fa);
-    hipLaunchKernelGGL((k_reduce_final<2>), dim3(1), dim3(kRedThreads), 0, c.stream, c.red, kRedBlocks,
-                       value, vacc ? 1 : 0);
-  }
+  const int axis = aw < 0 ? 0 : aw;
+  const long long count = loss_wall_only(kind, grad != nullptr, gacc)
+                              ? (s.n[axis] > 1 ? 2 : 1) * ((long long)s.ncell() / s.n[axis])
+                              : (long long)s.ncell();
+  const dim3 grid((unsigned)std::min<long long>(kRedBlocks, (count + kRedThreads - 1) / kRedThreads));
+  unsigned* arrived = reinterpret_cast<unsigned*>(c.famb_dev + kFambLossArrived);
+  if (fa < 0)
+    hipLaunchKernelGGL((k_loss<Store, G>), grid, dim3(kRedThreads), 0, c.stream, c.kp, static_cast<const Store*>(f),
+                       kind, axis, as, s.visc, vol, nplane, grad, gacc, c.red, arrived, value, vacc ? 1 : 0, 0);
+  else
+    hipLaunchKernelGGL((k_loss<Store, G, 2>), grid, dim3(kRedThreads), 0, c.stream, c.kp,
+                       static_cast<const Store*>(f), kind, axis, as, s.visc, vol, nplane, grad, gacc, c.red, arrived,
+                       value, vacc ? 1 : 0, fa);
   return hipGetLastError();
 }
 

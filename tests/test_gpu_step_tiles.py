@@ -10,8 +10,8 @@ import numpy as np
 import pytest
 
 from conftest import W, feq, moments, random_state
-from dugks_amd import (KERNEL_AUTO, KERNEL_FUSED, KERNEL_TWOPASS, PREC_FP16N, PREC_FP16S, PREC_FP32, PREC_FP64,
-                       configs)
+from dugks_amd import (KERNEL_AUTO, KERNEL_FUSED, KERNEL_TWOPASS, LOSS_KINETIC_ENERGY, PREC_FP16N, PREC_FP16S,
+                       PREC_FP32, PREC_FP64, configs)
 from test_gpu_step import _engine, _oracle_for, _relerr
 
 pytestmark = pytest.mark.gpu
@@ -191,3 +191,18 @@ def test_plans_match_twopass(rng, precision, n, tol, walls):
         eng.step(3 if precision == PREC_FP64 else 1)
         got.append(eng.get_f())
     assert _relerr(*got) <= tol
+
+
+@pytest.mark.parametrize("n", [(3, 4, 2), (16, 16, 1), (257, 1, 1), (64, 64, 65)], ids=str)
+def test_loss_over_grid_sizes(rng, n):
+    """The kinetic-energy loss on fewer cells than a block has threads, exactly
+    one block, one more, and more than the largest grid of blocks, against the
+    fields; the same bits on a second call.  FP64 sums of like terms: 1e-13."""
+    eng = _engine(configs.base(nx=n[0], ny=n[1], nz=n[2], xwidth=n[0] / 10, ywidth=n[1] / 10, zwidth=n[2] / 10,
+                               visc=0.02, ambient_fx=2e-4))
+    eng.set_f(random_state(n, rng))
+    rho, ux, uy, uz = eng.macro()
+    want = (0.5 * rho * (ux ** 2 + uy ** 2 + uz ** 2)).mean()
+    got = eng.loss(LOSS_KINETIC_ENERGY)
+    assert abs(got - want) <= 1e-13 * want
+    assert eng.loss(LOSS_KINETIC_ENERGY) == got
