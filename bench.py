@@ -50,7 +50,7 @@ def measured_traffic(precision):
     with the source hash it was measured on: (bytes, hash, current).  bytes
     is None when no summary for this precision exists or when it was measured
     on other kernel sources than the current ones (current False)."""
-    path = os.path.join(ROOT, "profiles", "k_fused_traffic_256x192x256.txt")
+    path = os.path.join(ROOT, "profiles", "k_step_traffic_256x192x256.txt")
     if not os.path.exists(path):
         return None, None, False
     value, stamp = None, None
@@ -176,7 +176,7 @@ def adjoint_leg(dugks_amd, configs, torch, T, precision="fp32"):
     lam_type = "float32" if "float32" in t_adj else "float64"
     S = {"fp64": 8, "fp32": 4}[precision]
     lb = 4 if lam_type == "float32" else 8
-    rec = 2 * 3 * 13 * S  # compact records (the z-marching gather's configurations)
+    rec = 2 * 3 * 4 * S  # compact records (the z-marching gather's configurations)
     # storage in the arithmetic type: the face pass hands rho and j (4 values)
     # to the gather, which then does not read f
     state = 19 * S + 2 * 4 * S
@@ -202,7 +202,7 @@ def adjoint_leg(dugks_amd, configs, torch, T, precision="fp32"):
                adjoint_over_forward_step=round(t_adj[lam_type] / fwd_step, 3),
                adjoint_step_ms_fp64_lambda=round(t_adj["float64"] * 1e3, 4),
                # algorithmic bytes of one adjoint step (per cell: lam' read twice and lam
-               # written, f read once and rho, j written and read, 13-value face records
+               # written, f read once and rho, j written and read, 4-value face records
                # of 3 axes written and read, the FP64 force gradient read and written)
                adjoint_alg_bytes_per_step=adj_bytes,
                adjoint_achieved_gbs=round(adj_bytes / t_adj[lam_type] / 1e9, 1),
