@@ -88,22 +88,14 @@ struct AdjFaceIO {
 // Gradient reconstruction of one population at a face's foot point: the
 // mean m of the two cells beside the face less h c.g (calc_fx,
 // src/dugks.cu:421-583); the terms of the components c_a = 0 are left out
-// (they add zero).
+// (they add zero).  dx, dy, dz are differences of values, kx, ky, kz what turns
+// them into h times the derivative.
 template <int cx, int cy, int cz, class Real>
-__device__ __forceinline__ Real grad_foot(Real m, Real h, Real gx, Real gy, Real gz) {
-  if constexpr (cx == 0 && cy == 0 && cz == 0) {
-    return m;
-  } else {
-    Real s;
-    if constexpr (cx != 0) s = Real(cx) * gx;
-    if constexpr (cy != 0) {
-      if constexpr (cx != 0) s += Real(cy) * gy; else s = Real(cy) * gy;
-    }
-    if constexpr (cz != 0) {
-      if constexpr (cx != 0 || cy != 0) s += Real(cz) * gz; else s = Real(cz) * gz;
-    }
-    return m - h * s;
-  }
+__device__ __forceinline__ Real grad_foot(Real m, Real kx, Real dx, Real ky, Real dy, Real kz, Real dz) {
+  if constexpr (cx != 0) m = fma_rn(Real(-cx) * kx, dx, m);
+  if constexpr (cy != 0) m = fma_rn(Real(-cy) * ky, dy, m);
+  if constexpr (cz != 0) m = fma_rn(Real(-cz) * kz, dz, m);
+  return m;
 }
 
 // The adjoint-face pass of the step taken from fin: every face is

@@ -139,11 +139,13 @@ __global__ void __launch_bounds__(step_nw(sizeof(Real) == 8, TX, TY) * 64, 2)
   // c_z < 0: the same), normal toward p+1 for c_z = 0, +1, -1
   const Real wzt = uniform(tz(9 + 6)), wzn0 = uniform(tz(9 + 1));
   const Real wznp = uniform(tz(9 + 2)), wznm = uniform(tz(9 + 0)), updz = uniform(tz(9 + 8));
+  // GRAD: h / d of the difference across a face, h / 4d of the difference of
+  // the two-cell sums two rows apart
   Real gin[3] = {Real(0), Real(0), Real(0)}, gtn[3] = {Real(0), Real(0), Real(0)};
   if constexpr (GRAD) {
     for (int a = 0; a < 3; a++) {
-      gin[a] = uniform((Real)(1.0 / P.du[a]));
-      gtn[a] = uniform((Real)(0.5 / P.du[a]));
+      gin[a] = uniform((Real)(P.hdt / P.du[a]));
+      gtn[a] = uniform((Real)(0.25 * P.hdt / P.du[a]));
     }
   }
   double flow = 0;
@@ -289,7 +291,7 @@ __global__ void __launch_bounds__(step_nw(sizeof(Real) == 8, TX, TY) * 64, 2)
     const Real sh = sign(w.half);
     if constexpr (GRAD) {
       const Real *a = S + q0 + w.at, *d = a + (qp - q0);
-      Real fl[NQ], fr[NQ], gx[NQ], gy[NQ];
+      Real fl[NQ], fr[NQ], gx[NQ] = {}, gy[NQ] = {};
       lds_diff<PAIR, kX>(a + STR, d + STR, a - STR, d - STR, gx);
       lds_diff<PAIR, kY>(a + AC * STR, d + AC * STR, a - AC * STR, d - AC * STR, gy);
       lds_get<PAIR, kAll>(a, fl);
@@ -297,11 +299,8 @@ __global__ void __launch_bounds__(step_nw(sizeof(Real) == 8, TX, TY) * 64, 2)
       static_for<NQ>([&](auto K) {
         constexpr int k = decltype(K)::value;
         constexpr int ip = slot_pop(PAIR, k), cx = CX[ip], cy = CY[ip], cz = CZ[ip];
-        Real gxv = Real(0), gyv = Real(0);
-        if constexpr (cx != 0) gxv = gx[k] * gtn[0];
-        if constexpr (cy != 0) gyv = gy[k] * gtn[1];
-        fc.template put<k>(
-            grad_foot<cx, cy, cz>(Real(0.5) * (fr[k] + fl[k]), sh * hdt, gxv, gyv, (fr[k] - fl[k]) * gin[2]));
+        fc.template put<k>(grad_foot<cx, cy, cz>(Real(0.5) * (fr[k] + fl[k]), sh * gtn[0], gx[k], sh * gtn[1], gy[k],
+                                                 sh * gin[2], fr[k] - fl[k]));
       });
     } else {
       const Real* a = S + AN + w.at;
@@ -337,7 +336,7 @@ __global__ void __launch_bounds__(step_nw(sizeof(Real) == 8, TX, TY) * 64, 2)
     const int pos = r * AC + c + 1;
     if constexpr (GRAD) {
       const Real *a = S + q0 + at(half, pos), *m = a + (qm - q0), *d = a + (qp - q0);
-      Real fl[NQ], fr[NQ], gy[NQ], gz[NQ];
+      Real fl[NQ], fr[NQ], gy[NQ] = {}, gz[NQ] = {};
       lds_diff<PAIR, kY>(a + AC * STR - STR, a + AC * STR, a - AC * STR - STR, a - AC * STR, gy);
       lds_diff<PAIR, kZ>(d - STR, d, m - STR, m, gz);
       lds_get<PAIR, kAll>(a - STR, fl);
@@ -345,11 +344,8 @@ __global__ void __launch_bounds__(step_nw(sizeof(Real) == 8, TX, TY) * 64, 2)
       static_for<NQ>([&](auto K) {
         constexpr int k = decltype(K)::value;
         constexpr int ip = slot_pop(PAIR, k), cx = CX[ip], cy = CY[ip], cz = CZ[ip];
-        Real gyv = Real(0), gzv = Real(0);
-        if constexpr (cy != 0) gyv = gy[k] * gtn[1];
-        if constexpr (cz != 0) gzv = gz[k] * gtn[2];
-        fc.template put<k>(
-            grad_foot<cx, cy, cz>(Real(0.5) * (fr[k] + fl[k]), sh * hdt, (fr[k] - fl[k]) * gin[0], gyv, gzv));
+        fc.template put<k>(grad_foot<cx, cy, cz>(Real(0.5) * (fr[k] + fl[k]), sh * gin[0], fr[k] - fl[k], sh * gtn[1],
+                                                 gy[k], sh * gtn[2], gz[k]));
       });
     } else {
       const Real* a = S + at(half, pos);
@@ -384,7 +380,7 @@ __global__ void __launch_bounds__(step_nw(sizeof(Real) == 8, TX, TY) * 64, 2)
     const int pos = r * AC + c + 1;
     if constexpr (GRAD) {
       const Real *a = S + q0 + at(half, pos), *m = a + (qm - q0), *d = a + (qp - q0);
-      Real fl[NQ], fr[NQ], gx[NQ], gz[NQ];
+      Real fl[NQ], fr[NQ], gx[NQ] = {}, gz[NQ] = {};
       lds_diff<PAIR, kX>(a - AC * STR + STR, a + STR, a - AC * STR - STR, a - STR, gx);
       lds_diff<PAIR, kZ>(d - AC * STR, d, m - AC * STR, m, gz);
       lds_get<PAIR, kAll>(a - AC * STR, fl);
@@ -392,11 +388,8 @@ __global__ void __launch_bounds__(step_nw(sizeof(Real) == 8, TX, TY) * 64, 2)
       static_for<NQ>([&](auto K) {
         constexpr int k = decltype(K)::value;
         constexpr int ip = slot_pop(PAIR, k), cx = CX[ip], cy = CY[ip], cz = CZ[ip];
-        Real gxv = Real(0), gzv = Real(0);
-        if constexpr (cx != 0) gxv = gx[k] * gtn[0];
-        if constexpr (cz != 0) gzv = gz[k] * gtn[2];
-        fc.template put<k>(
-            grad_foot<cx, cy, cz>(Real(0.5) * (fr[k] + fl[k]), sh * hdt, gxv, (fr[k] - fl[k]) * gin[1], gzv));
+        fc.template put<k>(grad_foot<cx, cy, cz>(Real(0.5) * (fr[k] + fl[k]), sh * gtn[0], gx[k], sh * gin[1],
+                                                 fr[k] - fl[k], sh * gtn[2], gz[k]));
       });
     } else {
       const Real* a = S + at(half, pos);
