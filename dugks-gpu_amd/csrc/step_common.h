@@ -136,6 +136,29 @@ __device__ __forceinline__ void lane_rho_u(const Real (&v)[lane_slots(PAIR)], Re
   }
 }
 
+// s u_axis of the cell for the flow-rate controller, summed in FP64 whatever the
+// arithmetic.  The controller divides the change of the bulk velocity by dt, so
+// it reads what the state holds, as the two-pass kernels' reduction over the
+// state does (FP32 sums left the reading of a 16x12x1 channel 8e-12 off, these
+// leave it within 5e-15).  128^3 channel with FP16 deviations 168 us a step, with
+// FP32 sums 166; FP32 channels 150x97x83 and 256x192x256 the same.
+template <bool PAIR, class Real>
+__device__ __forceinline__ double lane_velocity(const Real (&v)[lane_slots(PAIR)], int axis) {
+  double r, j[3];
+  lane_moments<PAIR, double>(v, r, j);
+  r = cell_sum<PAIR>(r) + (double)v[0];
+  const double ja = cell_diff<PAIR>(axis == 0 ? j[0] : (axis == 1 ? j[1] : j[2]));
+  if constexpr (sizeof(Real) == 8) {
+    return ja * rcp_real(r);
+  } else {
+    // 1/rho: the hardware reciprocal and two Newton steps
+    double x = __builtin_amdgcn_rcp(r);
+    x = __builtin_fma(x, __builtin_fma(-r, x, 1.0), x);
+    x = __builtin_fma(x, __builtin_fma(-r, x, 1.0), x);
+    return ja * x;
+  }
+}
+
 // centre_fbar of the lane's slots (SHIFT: in shifted populations, hb = f-bar+
 // - w from h, drho and u0; see EqShift).  shdt = s h and
 // sbw0 = s bw0 carry the mirrored frame's sign of the force terms: h F enters

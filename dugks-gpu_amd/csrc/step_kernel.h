@@ -579,7 +579,7 @@ __global__ void __launch_bounds__(step_nw(sizeof(Real) == 8, TX, TY) * 64, 2)
     if (interior) zface(zp, q0, qp);
     __syncthreads();
     // ---- phase 3: update of plane p ----
-    Real fnew[NQ], rr = Real(0), un[3] = {Real(0), Real(0), Real(0)};  // un: s u of the new state
+    Real fnew[NQ], rr = Real(0), un[3] = {Real(0), Real(0), Real(0)};  // kNeq: drho and u of the new state
     if (interior) {
       const Place w = place();
       const Real updx = xw(w.half, 5, w.c), updy = yw(w.half, 5, w.r), uz = sign(w.half) * updz;
@@ -605,16 +605,13 @@ __global__ void __launch_bounds__(step_nw(sizeof(Real) == 8, TX, TY) * 64, 2)
       });
       if constexpr (kNeq) {
         lane_rho_u<PAIR, Real>(fnew, rr, un, true);
+        // (the velocity as it is stored)
+        if (law.partial && stored) run_flow += (double)(as == 0 ? un[0] : (as == 1 ? un[1] : un[2]));
       } else if (law.partial) {
-        // the controller's reading only: sums in the arithmetic type suffice
-        // (the moments that feed the step are summed in FP64, lane_rho_u)
-        Real jn[3];
-        lane_moments<PAIR, Real>(fnew, rr, jn);
-        rr = cell_sum<PAIR>(rr) + fnew[0];
-        un[0] = cell_diff<PAIR>(as == 0 ? jn[0] : (as == 1 ? jn[1] : jn[2])) * rcp_real(rr);
+        // bulk velocity of the new state for the flow-rate controller
+        const double u = lane_velocity<PAIR, Real>(fnew, as);
+        if (stored) run_flow += u;
       }
-      // bulk velocity of the new state for the flow-rate controller
-      if (law.partial && stored) run_flow += (double)(!kNeq || as == 0 ? un[0] : (as == 1 ? un[1] : un[2]));
     }
     // Stores without a branch (lanes that store nothing address the end of
     // the array): the compiler then knows how many stores follow the loads
