@@ -191,11 +191,15 @@ __global__ void __launch_bounds__(256) k_perturb(KParams P, int step, double xwi
 // planes only (2 nx nz of the N cells on a y-wall channel).
 // NV = 2: the second sum is dJ/dF_fa, the derivative with respect to the
 // ambient force component fa (both losses read h F).
-// A sweep takes the loss in every step, forward and back; on small grids its
-// cost is that of its launches, so a call is one launch with as many blocks as
-// have cells (up to kRedBlocks: the order of the sums is fixed by the grid).
-// Wall shear on 64x64x32 FP64: 9.2 us, before 7.8 and 4.5 for two launches of
-// 1024 blocks and of one.
+// The grid has as many blocks as have cells (up to kRedBlocks; it fixes the order
+// of the sums).  A sweep takes the loss in every step, forward and back; up to
+// kLossOneLaunch blocks the last one to end adds all sums up, above that a second
+// launch does (arrived nullptr): the blocks' arrivals are releases at agent scope,
+// one after the other, and cost more than a launch from about 64 blocks on.  20
+// steps of a wall-shear sweep, FP32, one launch / two: 32 blocks 1584 / 1619 us,
+// 64 blocks 2034 / 2024, 128 blocks 2834 / 2806, 512 blocks 7992 / 7642; a
+// kinetic-energy call on 64^3 (1024 blocks) 67 / 31 us.
+constexpr int kLossOneLaunch = 32;
 __host__ __device__ constexpr bool loss_wall_only(int kind, bool grad, double gacc) {
   return kind == 0 && !(grad && gacc == 0.0);
 }
@@ -286,9 +290,14 @@ __global__ void __launch_bounds__(kRedThreads) k_loss(KParams P, const Store* __
       }
     }
   }
-  // the last block to get here adds all blocks' sums up, in order
   constexpr AllSums<NV> sums;
   block_reduce<NV, kRedThreads>(acc, sums.op);
+  if (!arrived) {  // k_reduce_final adds the blocks' sums up
+    if (threadIdx.x == 0)
+      for (int q = 0; q < NV; q++) partial[blockIdx.x * NV + q] = acc[q];
+    return;
+  }
+  // the last block to get here does, in the same order
   __shared__ unsigned before;
   if (threadIdx.x == 0) {
     for (int q = 0; q < NV; q++)
@@ -479,15 +488,21 @@ hipError_t loss_t(Ctx& c, const void* f, int kind, double* value, G* grad, doubl
   const long long count = loss_wall_only(kind, grad != nullptr, gacc)
                               ? (s.n[axis] > 1 ? 2 : 1) * ((long long)s.ncell() / s.n[axis])
                               : (long long)s.ncell();
-  const dim3 grid((unsigned)std::min<long long>(kRedBlocks, (count + kRedThreads - 1) / kRedThreads));
-  unsigned* arrived = reinterpret_cast<unsigned*>(c.famb_dev + kFambLossArrived);
+  const int nblocks = (int)std::min<long long>(kRedBlocks, (count + kRedThreads - 1) / kRedThreads);
+  const dim3 grid((unsigned)nblocks), threads(kRedThreads);
+  const bool one = nblocks <= kLossOneLaunch;
+  unsigned* arrived = one ? reinterpret_cast<unsigned*>(c.famb_dev + kFambLossArrived) : nullptr;
+  const int acc = vacc ? 1 : 0;
   if (fa < 0)
-    hipLaunchKernelGGL((k_loss<Store, G>), grid, dim3(kRedThreads), 0, c.stream, c.kp, static_cast<const Store*>(f),
-                       kind, axis, as, s.visc, vol, nplane, grad, gacc, c.red, arrived, value, vacc ? 1 : 0, 0);
+    hipLaunchKernelGGL((k_loss<Store, G>), grid, threads, 0, c.stream, c.kp, static_cast<const Store*>(f), kind, axis,
+                       as, s.visc, vol, nplane, grad, gacc, c.red, arrived, value, acc, 0);
   else
-    hipLaunchKernelGGL((k_loss<Store, G, 2>), grid, dim3(kRedThreads), 0, c.stream, c.kp,
-                       static_cast<const Store*>(f), kind, axis, as, s.visc, vol, nplane, grad, gacc, c.red, arrived,
-                       value, vacc ? 1 : 0, fa);
+    hipLaunchKernelGGL((k_loss<Store, G, 2>), grid, threads, 0, c.stream, c.kp, static_cast<const Store*>(f), kind,
+                       axis, as, s.visc, vol, nplane, grad, gacc, c.red, arrived, value, acc, fa);
+  if (!one && fa < 0)
+    hipLaunchKernelGGL((k_reduce_final<1>), dim3(1), threads, 0, c.stream, c.red, nblocks, value, acc);
+  else if (!one)
+    hipLaunchKernelGGL((k_reduce_final<2>), dim3(1), threads, 0, c.stream, c.red, nblocks, value, acc);
   return hipGetLastError();
 }
 
