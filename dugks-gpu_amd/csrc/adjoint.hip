@@ -763,20 +763,18 @@ bool gather_z_supported(const Ctx& c) {
   return true;
 }
 
+}  // namespace
+
 // Tile height (12 or 8 rows) and z-chunks of the gather, one workgroup per CU;
 // a chunk gathers the two planes beside it too.  A plane of an 8-row tile takes
 // 0.8 of the time, so they go where they fill more CUs (64x64x32: FP32 adjoint
 // step 58 us against 62 with 12 rows, FP64 gather 56.5 against 58).
-struct GatherPlan {
-  int rows, nchunk;
-  long long nblocks;
-};
-GatherPlan gather_plan(const KParams& P, bool fp64) {
+GatherPlan gather_plan(const Setup& s, bool fp64) {
   GatherPlan best{};
   double least = 0;
   for (const int rows : {12, 8}) {
-    const long long tiles = (long long)(P.n[0] / (fp64 ? 16 : 32)) * ((P.n[1] + rows - 1) / rows);
-    const int nz = P.n[2], nc = plan_z_chunks(tiles, nz, 256, 2.0);
+    const long long tiles = (long long)(s.n[0] / (fp64 ? 16 : 32)) * ((s.n[1] + rows - 1) / rows);
+    const int nz = s.n[2], nc = plan_z_chunks(tiles, nz, 256, 2.0);
     const double cost = (rows == 12 ? 1.0 : 0.8) * (double)((tiles * nc + 255) / 256) * ((nz + nc - 1) / nc + 2.0);
     if (rows == 12 || cost < 0.97 * least) {
       best = {rows, nc, tiles * nc};
@@ -785,6 +783,8 @@ GatherPlan gather_plan(const KParams& P, bool fp64) {
   }
   return best;
 }
+
+namespace {
 
 template <class Real, class Store, class Lam, int ROWS, bool FLOW>
 void launch_gather(const Ctx& cx, const GatherPlan& g, const void* f, const Lam* lam_next, Lam* lam_prev,
@@ -830,7 +830,7 @@ hipError_t run_adjoint(Ctx& cx, const void* f, const Lam* lam_next, Lam* lam_pre
   if (fpart && !handled) return hipErrorNotSupported;
   {
     if (compact) {
-      const GatherPlan g = gather_plan(P, sizeof(Real) == 8);
+      const GatherPlan g = gather_plan(cx.s, sizeof(Real) == 8);
       bool flow = false;
       if constexpr (kFuse) {
         flow = ubar != nullptr;

@@ -1212,6 +1212,19 @@ int dugks_config_initial_state(const char* text, const char* base_dir, double* h
   });
 }
 
+int dugks_config_plan(const char* text, const char* base_dir, int precision, int plan[6]) {
+  if (!text || !plan || precision > DUGKS_PREC_FP16N) return DUGKS_EARG;
+  return host_guard([&]() {
+    Setup s = make_setup(Config::from_text(text), base_dir ? base_dir : "");
+    const int prec = precision >= 0 ? precision : s.precision;
+    const StepPlan p = step_plan(s, prec);
+    const GatherPlan g = gather_plan(s, prec == DUGKS_PREC_FP64);
+    const int v[6] = {p.rows, p.nchunk, p.len, (int)p.nblocks, g.rows, g.nchunk};
+    std::memcpy(plan, v, sizeof v);
+    return DUGKS_OK;
+  });
+}
+
 int dugks_mesh_tanh(int n, double alpha, double width, double* faces) {
   if (n < 1 || !(alpha > 0 && alpha < 1) || !(width > 0) || !faces) return DUGKS_EARG;
   std::vector<double> z = tanh_faces(n, alpha, width);

@@ -82,6 +82,13 @@ struct StepPlan {
   long long nblocks = 0;  // workgroups (each leaves one bulk-velocity partial)
 };
 StepPlan step_plan(const Setup& s, int precision);
+// The same of the adjoint's z-marching gather.
+struct GatherPlan {
+  int rows = 0;           // 12 or 8
+  int nchunk = 0;
+  long long nblocks = 0;
+};
+GatherPlan gather_plan(const Setup& s, bool fp64);
 
 // Launchers (implemented in the .hip files; all stream-ordered).
 hipError_t launch_step_twopass(Ctx& c, const void* fin, void* fout);

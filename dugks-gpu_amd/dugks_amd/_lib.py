@@ -82,6 +82,7 @@ PROTOTYPES = {
     "dugks_sweep_bytes": (_i, [_ctxp, _dp]),
     # host-only helpers (no device needed)
     "dugks_config_derive": (_i, [_cp, _cp, _ip, _dp]),
+    "dugks_config_plan": (_i, [_cp, _cp, _i, _ip]),
     "dugks_config_spacing": (_i, [_cp, _cp, _i, _dp]),
     "dugks_config_initial_state": (_i, [_cp, _cp, _dp]),
     "dugks_mesh_tanh": (_i, [_i, _d, _d, _dp]),

@@ -322,6 +322,15 @@ def config_spacing(config_text, axis, base_dir=None):
     return out
 
 
+def config_plan(config_text, precision=_lib.PREC_CONFIG, base_dir=None):
+    """How the step kernel and the adjoint's gather divide the grid, where they
+    cover it: dict(rows, chunks, chunk_planes, blocks, gather_rows,
+    gather_chunks); chunk_planes 0 stands for equal chunks without runs."""
+    p = (ctypes.c_int * 6)()
+    _host_check(_lib.load().dugks_config_plan(config_text.encode(), _b(base_dir), int(precision), p))
+    return dict(zip(("rows", "chunks", "chunk_planes", "blocks", "gather_rows", "gather_chunks"), list(p)))
+
+
 def initial_state(config_text, base_dir=None):
     dims, _ = derive(config_text, base_dir)
     nx, ny, nz = dims

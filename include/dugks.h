@@ -284,6 +284,12 @@ int dugks_config_derive(const char* config_text, const char* base_dir, int dims[
 /* Cell widths of one axis derived from a config text. */
 int dugks_config_spacing(const char* config_text, const char* base_dir, int axis,
                          double* widths);
+/* How the one-kernel step and the adjoint's z-marching gather divide the grid of a
+ * config text (where they cover it), precision DUGKS_PREC_*: plan[0] rows of the
+ * step's tiles, [1] z-chunks of each tile, [2] > 0: of that many planes, with runs
+ * over the planes behind them, [3] workgroups, [4] rows of the gather's tiles, [5]
+ * its z-chunks. */
+int dugks_config_plan(const char* config_text, const char* base_dir, int precision, int plan[6]);
 /* Initial f of the config's case in the dump layout (host part of init_dugks,
  * src/dugks.cu:221-281). */
 int dugks_config_initial_state(const char* config_text, const char* base_dir, double* host_f);

@@ -1,0 +1,26 @@
+"""Grids of the tests by the form that the plan gives them (test_plans.py checks
+that it does): the step's (reconstruction, tile rows, runs) and the rows of the
+gather's tiles.  The FP16 modes share FP32's tiles."""
+
+_fp32 = {
+    ("tri", 12, False): [(41, 21, 44), (96, 84, 40), (150, 97, 83)],   # overlaps in x and y, in x; large
+    ("tri", 12, True): [(102, 61, 41), (38, 54, 126)],
+    ("tri", 8, False): [(64, 64, 32), (64, 20, 37)],
+    ("tri", 4, False): [(20, 20, 20), (33, 25, 4)],
+}
+_fp64 = {
+    ("tri", 12, False): [(48, 40, 20), (90, 50, 121)],
+    ("tri", 12, True): [(82, 39, 41), (51, 50, 49)],
+    ("tri", 8, False): [(64, 64, 32), (64, 20, 37)],
+    ("tri", 4, False): [(20, 20, 20), (8, 64, 8)],
+}
+STEP_GRIDS = {form: {"fp64": _fp64[form], "fp32": _fp32[form], "fp16": _fp32[form], "fp16n": _fp32[form]}
+              for form in _fp32}
+
+# 12 rows: 40, 32 and 80 rows of cells leave an overlap, 48 and 96 none
+GATHER_GRIDS = {
+    12: {"fp64": [(32, 40, 26), (64, 80, 64), (96, 96, 30)],
+         "fp32": [(32, 32, 65), (64, 80, 64), (128, 40, 128), (96, 96, 64)],
+         "fp16": [(32, 32, 65), (96, 96, 64)]},
+    8: {"fp64": [(64, 64, 32)], "fp32": [(64, 64, 32)], "fp16": [(64, 64, 32)]},
+}

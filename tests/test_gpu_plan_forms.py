@@ -1,0 +1,120 @@
+"""Every form of the step's plan and of the adjoint's gather, in every storage mode,
+against the two-pass kernels, cell by cell (plan_grids.py names grids by form)."""
+import numpy as np
+import pytest
+
+from conftest import W, feq, moments, random_state
+from dugks_amd import (KERNEL_AUTO, KERNEL_TWOPASS, PREC_FP16N, PREC_FP16S, PREC_FP32, PREC_FP64, configs)
+from plan_grids import GATHER_GRIDS, STEP_GRIDS
+from test_gpu_adjoint import _flow_grad, _flow_J, _flow_problem
+from test_gpu_adjoint import _engine as _stream_engine
+from test_gpu_step import _engine
+
+torch = pytest.importorskip("torch")
+pytestmark = pytest.mark.gpu
+
+MODES = {"fp64": PREC_FP64, "fp32": PREC_FP32, "fp16": PREC_FP16S, "fp16n": PREC_FP16N}
+WALLS = {"periodic": {}, "walls_y": dict(periods_y=0, mesh_y="tanh:0.85", dt_rule="min"),
+         "walls_x": dict(periods_x=0, mesh_x="tanh:0.8", dt_rule="min"),
+         "walls_xy": dict(periods_x=0, periods_y=0)}
+
+
+def _text(n, walls, recon="tri"):
+    kw = {k: v for k, v in WALLS[walls].items() if recon == "tri" or not k.startswith(("mesh", "dt"))}
+    return configs.base(nx=n[0], ny=n[1], nz=n[2], xwidth=n[0] / 10, ywidth=n[1] / 10, zwidth=n[2] / 10, visc=0.02,
+                        CFL=0.5, recon=recon, ambient_fx=2e-4, ambient_fz=1e-4, **kw)
+
+
+STEP_CASES = [(form, mode, n, walls) for form in STEP_GRIDS for mode in MODES for n in STEP_GRIDS[form][mode]
+              for walls in WALLS if n[0] * n[1] * n[2] < 200000 or walls == "walls_y"]
+
+
+@pytest.mark.parametrize("form,mode,n,walls", STEP_CASES,
+                         ids=lambda v: "-".join(map(str, v)) if isinstance(v, tuple) else v)
+def test_step_forms_match_twopass(rng, form, mode, n, walls):
+    """With a force in every cell.  Both paths' distances from the oracle, as tested
+    on whole tiles: 1e-13 a step in FP64 (three steps here), 2e-6 in FP32
+    arithmetic, and for FP16 storage one rounding each."""
+    text = _text(n, walls, form[0])
+    f0 = random_state(n, rng)
+    G = 1e-4 * rng.standard_normal((3,) + f0.shape[:3])
+    got = []
+    for kernel in (KERNEL_AUTO, KERNEL_TWOPASS):
+        eng = _engine(text, precision=MODES[mode], kernel=kernel)
+        eng.set_f(f0)
+        eng.set_cell_force(*G)
+        eng.step(3 if mode == "fp64" else 1)
+        got.append(eng.get_f())
+    a, b = got
+    big = np.abs(b).max()
+    if mode == "fp64":
+        tol = 2 * 3e-13 * big
+    elif mode == "fp32":
+        tol = 2 * 2e-6 * big
+    elif mode == "fp16":
+        tol = 2 * (W * np.maximum(2.0 ** -11 * np.abs(b / W - eng.params["rho0"]), 2.0 ** -25) + 4e-6 * big)
+    else:
+        rho, j = moments(b)
+        tol = 2 * (2.0 ** -11 * np.abs(b - feq(rho, j / rho[..., None])) + 2.0 ** -25 * W / 1024 + 4e-6 * big)
+    assert np.all(np.abs(a - b) <= tol)
+
+
+GATHER_CASES = [(rows, mode, n, lam) for rows in GATHER_GRIDS for mode in GATHER_GRIDS[rows]
+                for n in GATHER_GRIDS[rows][mode] for lam in (("f64",) if mode == "fp64" else ("f64", "f32"))]
+
+
+@pytest.mark.parametrize("walls", ["periodic", "walls_y", "walls_x"])
+@pytest.mark.parametrize("rows,mode,n,lam", GATHER_CASES,
+                         ids=lambda v: "-".join(map(str, v)) if isinstance(v, tuple) else str(v))
+def test_gather_forms_match_twopass(rng, rows, mode, n, lam, walls):
+    """lam and the force gradient, added to what the array holds, against the FP64
+    two-pass adjoint about the same stored state: the bounds of one adjoint step
+    against the oracle, 1e-12 (FP64) and 2e-5 (FP32 arithmetic) of the largest
+    value.  A row of cells taken twice or not at all is off by that value."""
+    text = _text(n, walls)
+    nz, ny, nx = n[2], n[1], n[0]
+    lam0 = torch.randn((19, nz, ny, nx), dtype=torch.float32, device="cuda",
+                       generator=torch.Generator("cuda").manual_seed(3)).double()
+    G = 1e-4 * rng.standard_normal((3, nz, ny, nx))
+    eng = _stream_engine(text, precision=MODES[mode], kernel=KERNEL_AUTO)
+    eng.set_f(random_state(n, rng))
+    ref = _stream_engine(text, precision=PREC_FP64, kernel=KERNEL_TWOPASS)
+    ref.set_f(eng.get_f())
+    out = []
+    for e, dtype in ((eng, torch.float32 if lam == "f32" else torch.float64), (ref, torch.float64)):
+        e.set_cell_force(*G)
+        lp = torch.full((19, nz, ny, nx), float("nan"), dtype=dtype, device="cuda")
+        g = torch.full((3, nz, ny, nx), 0.5, dtype=torch.float64, device="cuda")
+        e.adjoint_step(lam0.to(dtype), lp, g)
+        torch.cuda.synchronize()
+        out.append((lp.double(), g - 0.5))
+    tol = 1e-12 if mode == "fp64" else 2e-5
+    for got, want in zip(*out):
+        assert float((got - want).abs().max()) <= tol * float(want.abs().max())
+
+
+def test_controller_sweep_on_12_row_gather(rng):
+    """The gather that adds the controller's term, on overlapping tiles of 12 rows:
+    FP64 against central differences (the bar of the 8-row sweep, 1e-7)."""
+    n = GATHER_GRIDS[12]["fp64"][0]
+    eng, f0, F0, G, T = _flow_problem(PREC_FP64, *n, T=8)
+    J, grad, dF0 = _flow_grad(eng, f0, F0, G, T)
+    for trial in range(3):
+        v = rng.standard_normal(G.shape) * 1e-6
+        fd = (_flow_J(eng, f0, F0, G + v, T) - _flow_J(eng, f0, F0, G - v, T)) / 2
+        an = float((grad * v).sum())
+        assert abs(fd - an) <= 1e-7 * abs(an), (trial, fd, an)
+
+
+@pytest.mark.parametrize("mode,tol", [("fp32", 1e-5), ("fp16", 2e-4)])
+def test_reduced_precision_controller_sweep_on_12_row_gather(mode, tol):
+    """Against the FP64 sweep, with the bars of the 8-row one."""
+    n = GATHER_GRIDS[12][mode][0]
+    got = []
+    for precision in (MODES[mode], PREC_FP64):
+        eng, f0, F0, G, T = _flow_problem(precision, *n, T=8)
+        got.append(_flow_grad(eng, f0, F0, G, T))
+    (Ja, ga, da), (Jb, gb, db) = got
+    assert abs(Ja - Jb) <= tol * abs(Jb)
+    assert np.abs(ga - gb).max() <= tol * np.abs(gb).max()
+    assert abs(da - db) <= tol * abs(db)
