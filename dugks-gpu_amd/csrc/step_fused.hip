@@ -634,8 +634,10 @@ int z_chunk(const Ctx& cx, int TX, int TY) {
 //    neighbouring tiles out of step, so that their halos miss L2: 263 us in
 //    FP64 and 137 in FP32.)  Only where the model gives 7 %: at 5 % a
 //    150x97x83 FP32 channel gained 2 % and a 90x50x121 FP64 duct lost 3.
-// Gradient reconstruction has only the first form (its kernel has no registers
-// left for the runs).
+// Gradient reconstruction takes the first two forms (its kernel has no registers
+// left for the runs).  Periodic, us a step with 12, 8 and 4 rows: 64x32x1 FP32
+// 12.4, 11.8 and 9.8; 64x64x32 FP32 21.6, 19.5 and 22.6, FP64 31.3, 26.6 and 31.8;
+// 96x96x16 FP32 22.9, 23.9 and 28.7.
 StepPlan step_plan(const Setup& s, int precision) {
   const int tx = precision == 0 ? 16 : 32, nz = s.n[2];
   const double start = 2.2;
@@ -650,8 +652,7 @@ StepPlan step_plan(const Setup& s, int precision) {
       best = {rows, nc, 0, tiles * nc};
       least = cost;
     }
-    if (s.recon != 0) return best;
-    if (rows != 12) continue;
+    if (rows != 12 || s.recon != 0) continue;
     const double chunks = 0.93 * least;
     for (int m = 1; m * tiles < 256; m++)
       for (int len = 1; m * len < nz && len + start < chunks; len++) {
@@ -670,7 +671,7 @@ StepPlan step_plan(const Setup& s, int precision) {
 
 namespace {
 
-template <class Real, class Store, int TX, int TY, bool GRAD, bool RUNS>
+template <class Real, class Store, int TX, int TY, bool GRAD, bool RUNS, bool FLAT>
 hipError_t run_step(Ctx& cx, const void* fin, void* fout, const StepPlan& plan) {
   using T = StepTile<Real, TX, TY, GRAD>;
   FlowLaw law{};
@@ -681,7 +682,7 @@ hipError_t run_step(Ctx& cx, const void* fin, void* fout, const StepPlan& plan) 
            s.width[0] * s.width[1] * s.width[2], s.flow_rate, s.flow_gain, s.dt};
   }
   if (cx.timing) hipEventRecord(cx.tev[0], cx.stream);
-  hipLaunchKernelGGL((k_step<Real, Store, TX, TY, GRAD, RUNS>), dim3((unsigned)plan.nblocks), dim3(T::NT), 0, cx.stream,
+  hipLaunchKernelGGL((k_step<Real, Store, TX, TY, GRAD, RUNS, FLAT>), dim3((unsigned)plan.nblocks), dim3(T::NT), 0, cx.stream,
                      cx.kp, static_cast<const Store*>(fin), static_cast<Store*>(fout), plan.nchunk, plan.len, law);
   if (cx.timing) hipEventRecord(cx.tev[1], cx.stream);
   cx.launches_per_step = 1;
@@ -766,15 +767,22 @@ bool step_covers(const Ctx& c) {
   return c.kernel != 1 /* DUGKS_KERNEL_FUSED */ && tiles_cover(c) && c.kp.N >= 512;
 }
 
+template <class Real, class Store, bool GRAD, bool FLAT>
+hipError_t run_step_rows(Ctx& c, const void* fin, void* fout) {
+  constexpr int TX = sizeof(Real) == 8 ? 16 : 32;
+  if (c.plan.rows == 12) return run_step<Real, Store, TX, 12, GRAD, false, FLAT>(c, fin, fout, c.plan);
+  if (c.plan.rows == 8) return run_step<Real, Store, TX, 8, GRAD, false, FLAT>(c, fin, fout, c.plan);
+  return run_step<Real, Store, TX, 4, GRAD, false, FLAT>(c, fin, fout, c.plan);
+}
+
 template <class Real, class Store>
 hipError_t launch_step_mode(Ctx& c, const void* fin, void* fout) {
   constexpr int TX = sizeof(Real) == 8 ? 16 : 32;
-  const StepPlan& plan = c.plan;
-  if (c.s.recon != 0) return run_step<Real, Store, TX, 12, true, false>(c, fin, fout, plan);
-  if (plan.len > 0) return run_step<Real, Store, TX, 12, false, true>(c, fin, fout, plan);
-  if (plan.rows == 12) return run_step<Real, Store, TX, 12, false, false>(c, fin, fout, plan);
-  if (plan.rows == 8) return run_step<Real, Store, TX, 8, false, false>(c, fin, fout, plan);
-  return run_step<Real, Store, TX, 4, false, false>(c, fin, fout, plan);
+  if (c.s.recon != 0)
+    return c.s.n[2] == 1 ? run_step_rows<Real, Store, true, true>(c, fin, fout)
+                         : run_step_rows<Real, Store, true, false>(c, fin, fout);
+  if (c.plan.len > 0) return run_step<Real, Store, TX, 12, false, true, false>(c, fin, fout, c.plan);
+  return run_step_rows<Real, Store, false, false>(c, fin, fout);
 }
 }  // namespace
 

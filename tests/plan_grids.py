@@ -7,12 +7,19 @@ _fp32 = {
     ("tri", 12, True): [(102, 61, 41), (38, 54, 126)],
     ("tri", 8, False): [(64, 64, 32), (64, 20, 37)],
     ("tri", 4, False): [(20, 20, 20), (33, 25, 4)],
+    # gradient reconstruction: grids of one plane (their own form) among them
+    ("grad", 12, False): [(41, 21, 44), (96, 84, 40), (256, 300, 1)],
+    ("grad", 8, False): [(64, 64, 32), (512, 96, 1)],
+    ("grad", 4, False): [(20, 20, 20), (33, 25, 4), (64, 32, 1), (200, 97, 1)],
 }
 _fp64 = {
     ("tri", 12, False): [(48, 40, 20), (90, 50, 121)],
     ("tri", 12, True): [(82, 39, 41), (51, 50, 49)],
     ("tri", 8, False): [(64, 64, 32), (64, 20, 37)],
     ("tri", 4, False): [(20, 20, 20), (8, 64, 8)],
+    ("grad", 12, False): [(48, 40, 20), (96, 84, 40), (256, 300, 1)],
+    ("grad", 8, False): [(64, 64, 32), (300, 97, 1)],
+    ("grad", 4, False): [(20, 20, 20), (64, 32, 1)],
 }
 STEP_GRIDS = {form: {"fp64": _fp64[form], "fp32": _fp32[form], "fp16": _fp32[form], "fp16n": _fp32[form]}
               for form in _fp32}
