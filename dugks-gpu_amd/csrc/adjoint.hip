@@ -376,7 +376,10 @@ struct GatherTile {
 // controller): lam' still lacks the bulk velocity's cotangent ubar (dV/V)
 // (c_ia - u_a)/rho of f(n+1), whose rho, j the previous pass left in the
 // other region; it is added as lam' is used.
-template <class Real, class Store, class Lam, int ROWS, bool FLOW = false>
+// FLAT: the grid has one plane, so planes p-1, p and p+1 are the same and the
+// first one taken completes it.  (FP32 with FP64 lam, us an adjoint step: 512x768x1
+// 98, with the same plane taken three times 144; 64x64x1 18 and 29.)
+template <class Real, class Store, class Lam, int ROWS, bool FLOW, bool FLAT>
 __global__ void __launch_bounds__(gather_lanes(sizeof(Real) == 8, ROWS), sizeof(Real) == 4 ? 2 : 1)
     k_adj_cells_z(KParams P, const Store* __restrict__ fin, const Lam* __restrict__ lam,
                   const Real* __restrict__ faces, Lam* __restrict__ lam_prev, double* __restrict__ grad, int nchunk,
@@ -594,7 +597,7 @@ __global__ void __launch_bounds__(gather_lanes(sizeof(Real) == 8, ROWS), sizeof(
   load_lam(I0{}, IQ{}, wrap(z0 - 1), true);
   load_recs(wrap(z0 - 1), true);
 
-  for (int p = z0 - 1; p <= zend; p++) {
+  for (int p = FLAT ? z0 : z0 - 1; p <= (FLAT ? z0 : zend); p++) {
     const int pos = here(pos0), Rg = here(Rg0), Cg = here(Cg0);  // (addresses formed anew each plane)
     // lam'(p), complete
     static_for<Q>([&](auto I) {
@@ -611,6 +614,8 @@ __global__ void __launch_bounds__(gather_lanes(sizeof(Real) == 8, ROWS), sizeof(
         lamC[ip] += fma_rn(Real(CX[ip]) * ax + Real(CY[ip]) * ay + Real(CZ[ip]) * az, sc, t0);
       });
     }
+    if constexpr (FLAT)
+      for (int ip = 0; ip < Q; ip++) lamP[ip] = lamC[ip];
     __syncthreads();  // the previous plane's gather is done with S
     static_for<Q>([&](auto I) {
       constexpr int ip = decltype(I)::value;
@@ -641,8 +646,8 @@ __global__ void __launch_bounds__(gather_lanes(sizeof(Real) == 8, ROWS), sizeof(
     }
     // The centre stage's inputs of plane p-1 first, then, in groups, what the
     // next plane needs
-    const bool centre = stored && p - 1 >= z0, more = p < zend;
-    const unsigned cell = centre ? (unsigned)(p - 1) * plane + column : 0u;
+    const bool centre = stored && (FLAT || p - 1 >= z0), more = !FLAT && p < zend;
+    const unsigned cell = centre ? (FLAT ? 0u : (unsigned)(p - 1) * plane) + column : 0u;
     const unsigned v8 = centre ? cell * 8u : kOutOfRange;
     Real m4[4] = {Real(1), Real(0), Real(0), Real(0)};
     RawCell<Real, Store> fraw;
@@ -711,6 +716,8 @@ __global__ void __launch_bounds__(gather_lanes(sizeof(Real) == 8, ROWS), sizeof(
         push(I, gq * hzr, gq * hz);
       });
     }
+    if constexpr (FLAT)
+      for (int ip = 0; ip < Q; ip++) accP[ip] += accC[ip] + accN[ip];
     // centre-stage adjoint of plane p-1 (as k_adj_cells)
     Real rho = m4[0], j[3] = {m4[1], m4[2], m4[3]};
     if constexpr (!kMoments) {
@@ -786,14 +793,28 @@ GatherPlan gather_plan(const Setup& s, bool fp64) {
 
 namespace {
 
-template <class Real, class Store, class Lam, int ROWS, bool FLOW>
+template <class Real, class Store, class Lam, int ROWS, bool FLOW, bool FLAT>
 void launch_gather(const Ctx& cx, const GatherPlan& g, const void* f, const Lam* lam_next, Lam* lam_prev,
                    double* grad, int mom, const double* ubar) {
   const double inv_vol = 1.0 / (cx.s.width[0] * cx.s.width[1] * cx.s.width[2]);
-  hipLaunchKernelGGL((k_adj_cells_z<Real, Store, Lam, ROWS, FLOW>), dim3((unsigned)g.nblocks),
+  hipLaunchKernelGGL((k_adj_cells_z<Real, Store, Lam, ROWS, FLOW, FLAT>), dim3((unsigned)g.nblocks),
                      dim3(GatherTile<Real, ROWS>::NT), 0, cx.stream, cx.kp, static_cast<const Store*>(f), lam_next,
                      static_cast<const Real*>(cx.adj_faces), lam_prev, grad, g.nchunk, mom, FLOW ? ubar : nullptr,
                      inv_vol);
+}
+template <class Real, class Store, class Lam, bool FLOW>
+void launch_gather(const Ctx& cx, const void* f, const Lam* lam_next, Lam* lam_prev, double* grad, int mom,
+                   const double* ubar) {
+  const GatherPlan g = gather_plan(cx.s, sizeof(Real) == 8);
+  const bool flat = cx.s.n[2] == 1;
+  if (g.rows == 12 && flat)
+    launch_gather<Real, Store, Lam, 12, FLOW, true>(cx, g, f, lam_next, lam_prev, grad, mom, ubar);
+  else if (g.rows == 12)
+    launch_gather<Real, Store, Lam, 12, FLOW, false>(cx, g, f, lam_next, lam_prev, grad, mom, ubar);
+  else if (flat)
+    launch_gather<Real, Store, Lam, 8, FLOW, true>(cx, g, f, lam_next, lam_prev, grad, mom, ubar);
+  else
+    launch_gather<Real, Store, Lam, 8, FLOW, false>(cx, g, f, lam_next, lam_prev, grad, mom, ubar);
 }
 
 // One adjoint step.  Lam = double: every configuration; Lam = float (FP32
@@ -830,19 +851,12 @@ hipError_t run_adjoint(Ctx& cx, const void* f, const Lam* lam_next, Lam* lam_pre
   if (fpart && !handled) return hipErrorNotSupported;
   {
     if (compact) {
-      const GatherPlan g = gather_plan(cx.s, sizeof(Real) == 8);
       bool flow = false;
       if constexpr (kFuse) {
         flow = ubar != nullptr;
-        if (flow && g.rows == 12)
-          launch_gather<Real, Store, Lam, 12, true>(cx, g, f, lam_next, lam_prev, grad, mom, ubar);
-        else if (flow)
-          launch_gather<Real, Store, Lam, 8, true>(cx, g, f, lam_next, lam_prev, grad, mom, ubar);
+        if (flow) launch_gather<Real, Store, Lam, true>(cx, f, lam_next, lam_prev, grad, mom, ubar);
       }
-      if (!flow && g.rows == 12)
-        launch_gather<Real, Store, Lam, 12, false>(cx, g, f, lam_next, lam_prev, grad, mom, ubar);
-      else if (!flow)
-        launch_gather<Real, Store, Lam, 8, false>(cx, g, f, lam_next, lam_prev, grad, mom, ubar);
+      if (!flow) launch_gather<Real, Store, Lam, false>(cx, f, lam_next, lam_prev, grad, mom, ubar);
       return hipGetLastError();
     }
   }

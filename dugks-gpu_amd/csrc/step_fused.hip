@@ -635,8 +635,8 @@ int z_chunk(const Ctx& cx, int TX, int TY) {
 //    FP64 and 137 in FP32.)  Only where the model gives 7 %: at 5 % a
 //    150x97x83 FP32 channel gained 2 % and a 90x50x121 FP64 duct lost 3.
 // Gradient reconstruction takes the first two forms (its kernel has no registers
-// left for the runs).  Periodic, us a step with 12, 8 and 4 rows: 64x32x1 FP32
-// 12.4, 11.8 and 9.8; 64x64x32 FP32 21.6, 19.5 and 22.6, FP64 31.3, 26.6 and 31.8;
+// left for the runs).  Periodic, us a step with 12, 8 and 4 rows: 64x32x2 FP32
+// 13.8, 12.5 and 10.4; 64x64x32 FP32 21.6, 19.5 and 22.6, FP64 31.3, 26.6 and 31.8;
 // 96x96x16 FP32 22.9, 23.9 and 28.7.
 StepPlan step_plan(const Setup& s, int precision) {
   const int tx = precision == 0 ? 16 : 32, nz = s.n[2];

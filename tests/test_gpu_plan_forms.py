@@ -1,5 +1,7 @@
 """Every form of the step's plan and of the adjoint's gather, in every storage mode,
 against the two-pass kernels, cell by cell (plan_grids.py names grids by form)."""
+import time
+
 import numpy as np
 import pytest
 
@@ -93,10 +95,11 @@ def test_gather_forms_match_twopass(rng, rows, mode, n, lam, walls):
         assert float((got - want).abs().max()) <= tol * float(want.abs().max())
 
 
-def test_controller_sweep_on_12_row_gather(rng):
-    """The gather that adds the controller's term, on overlapping tiles of 12 rows:
-    FP64 against central differences (the bar of the 8-row sweep, 1e-7)."""
-    n = GATHER_GRIDS[12]["fp64"][0]
+@pytest.mark.parametrize("n", [GATHER_GRIDS[12]["fp64"][0], (32, 16, 1)], ids=["rows12", "one_plane"])
+def test_controller_sweep_over_gather_forms(rng, n):
+    """The gather that adds the controller's term, on overlapping tiles of 12 rows
+    and on one plane: FP64 against central differences (the bar of the 8-row sweep,
+    1e-7)."""
     eng, f0, F0, G, T = _flow_problem(PREC_FP64, *n, T=8)
     J, grad, dF0 = _flow_grad(eng, f0, F0, G, T)
     for trial in range(3):
@@ -106,10 +109,10 @@ def test_controller_sweep_on_12_row_gather(rng):
         assert abs(fd - an) <= 1e-7 * abs(an), (trial, fd, an)
 
 
+@pytest.mark.parametrize("n", [GATHER_GRIDS[12]["fp32"][0], (32, 16, 1)], ids=["rows12", "one_plane"])
 @pytest.mark.parametrize("mode,tol", [("fp32", 1e-5), ("fp16", 2e-4)])
-def test_reduced_precision_controller_sweep_on_12_row_gather(mode, tol):
+def test_reduced_precision_controller_sweep_over_gather_forms(mode, tol, n):
     """Against the FP64 sweep, with the bars of the 8-row one."""
-    n = GATHER_GRIDS[12][mode][0]
     got = []
     for precision in (MODES[mode], PREC_FP64):
         eng, f0, F0, G, T = _flow_problem(precision, *n, T=8)
@@ -118,3 +121,24 @@ def test_reduced_precision_controller_sweep_on_12_row_gather(mode, tol):
     assert abs(Ja - Jb) <= tol * abs(Jb)
     assert np.abs(ga - gb).max() <= tol * np.abs(gb).max()
     assert abs(da - db) <= tol * abs(db)
+
+
+def test_one_plane_adjoint_takes_the_plane_once():
+    """On one plane the gather's three neighbouring planes are the same.  Taken once,
+    an adjoint step costs 0.6 of one on two planes, taken three times as much as
+    that one; the least time of many runs of each, in turn, must stay below 0.85."""
+    best = {}
+    runs = {}
+    for nz in (1, 2):
+        eng = _stream_engine(_text((64, 64, nz), "periodic"), precision=PREC_FP32)
+        lam = torch.randn((19, nz, 64, 64), dtype=torch.float64, device="cuda")
+        runs[nz] = (eng, lam, torch.empty_like(lam))
+    for _ in range(40):
+        for nz, (eng, lam, out) in runs.items():
+            torch.cuda.synchronize()
+            t = time.perf_counter()
+            for _ in range(20):
+                eng.adjoint_step(lam, out)
+            torch.cuda.synchronize()
+            best[nz] = min(best.get(nz, 1.0), time.perf_counter() - t)
+    assert best[1] <= 0.85 * best[2], best
