@@ -196,15 +196,7 @@ __device__ __forceinline__ double RawBuf::ld<double>(unsigned vb, unsigned sb) c
 // A byte offset no RawBuf of this code base reaches: loads through it read 0.
 constexpr unsigned kOutOfRange = 0x80000000u;
 
-// Decode / encode one population through a StateBuf (the Codec rules).
-template <class Real, class Store>
-__device__ __forceinline__ Real ld_state(const StateBuf<Store>& b, unsigned vb, unsigned sb, const KParams& P,
-                                         int ip) {
-  if constexpr (std::is_same<Store, __half>::value)
-    return (Real)((float)wgt(ip) * (P.rho0f + __half2float(b.raw(vb, sb))));
-  else
-    return (Real)b.raw(vb, sb);
-}
+// Encode one population through a StateBuf (the Codec rules).
 template <class Real, class Store>
 __device__ __forceinline__ void st_state(const StateBuf<Store>& b, unsigned vb, unsigned sb, Real v,
                                          const KParams& P, int ip) {
@@ -212,6 +204,24 @@ __device__ __forceinline__ void st_state(const StateBuf<Store>& b, unsigned vb, 
     b.put(__float2half((float)v * (float)(1.0 / wgt(ip)) - P.rho0f), vb, sb);
   else
     b.put((Store)v, vb, sb);
+}
+
+// Constant-flow-rate controller (one thread).  famb_dev layout:
+// [0..2] ambient force, [3] previous bulk velocity, [4] previous-valid flag.
+// The controlled quantity is the momentum bulk velocity U = <j/rho> (the
+// output velocity minus h F, which would respond to F instantly and make the
+// loop overshoot).  Per step U^{n+1} = U^n + dt (F^n - D) with D the wall
+// drag; D is estimated from the last step's change and the new force closes
+// a fraction `gain` of the gap: F^n = D + gain (U_target - U^n) / dt, so the
+// error obeys e^{n+1} = (1 - gain) e^n for a steady drag (stable 0 < gain < 2).
+__device__ __forceinline__ void flow_update(double* famb, int axis, double Ub, double target, double gain,
+                                            double dt) {
+  const double Fprev = famb[axis];
+  double drag = Fprev;
+  if (famb[4] != 0) drag = Fprev - (Ub - famb[3]) / dt;
+  famb[axis] = drag + gain * (target - Ub) / dt;
+  famb[3] = Ub;
+  famb[4] = 1;
 }
 
 // a * b + c rounded once

@@ -124,24 +124,7 @@ __global__ void __launch_bounds__(kRedThreads) k_reduce_final(const double* part
     for (int q = 0; q < NV; q++) out[q] = (accumulate ? out[q] : 0.0) + acc[q];
 }
 
-// Constant-flow-rate controller (single thread).  famb_dev layout:
-// [0..2] ambient force, [3] previous bulk velocity, [4] previous-valid flag.
-// The controlled quantity is the momentum bulk velocity U = <j/rho> (the
-// output velocity minus h F, which would respond to F instantly and make the
-// loop overshoot).  Per step U^{n+1} = U^n + dt (F^n - D) with D the wall
-// drag; D is estimated from the last step's change and the new force closes
-// a fraction `gain` of the gap: F^n = D + gain (U_target - U^n) / dt, so the
-// error obeys e^{n+1} = (1 - gain) e^n for a steady drag (stable 0 < gain < 2).
-__device__ __forceinline__ void flow_update(double* famb, int axis, double Ub, double target, double gain,
-                                            double dt) {
-  const double Fprev = famb[axis];
-  double drag = Fprev;
-  if (famb[4] != 0) drag = Fprev - (Ub - famb[3]) / dt;
-  famb[axis] = drag + gain * (target - Ub) / dt;
-  famb[3] = Ub;
-  famb[4] = 1;
-}
-
+// The controller after the two-pass step (single thread; flow_update).
 __global__ void k_flow_control(double* famb, const double* sums, int axis, double target, double gain,
                                double dt, double hdt) {
   // sums[4 + axis] / sums[7] is the bulk output velocity <j/rho + h F>

@@ -10,24 +10,13 @@ constexpr int step_nw(bool pair, int TX, int TY) {
 
 // The flow-rate controller: where the workgroups leave their parts of the sum
 // over cells of u dV of the new state (nullptr: no controller), and how many
-// have; the force and the controller's state (flow_law), and its constants.
+// have; the force and the controller's state (flow_update), and its constants.
 struct FlowLaw {
   double* partial;
   unsigned* arrived;
   double* famb;
   double volume, target, gain, dt;
 };
-// One step of the controller on bulk velocity Ub (the law of k_flow_control;
-// famb: the force, then the previous bulk velocity and whether there is one).
-__device__ __forceinline__ void flow_law(double* famb, int axis, double Ub, double target, double gain, double dt) {
-  const double Fprev = famb[axis];
-  double drag = Fprev;
-  if (famb[4] != 0) drag = Fprev - (Ub - famb[3]) / dt;
-  famb[axis] = drag + gain * (target - Ub) / dt;
-  famb[3] = Ub;
-  famb[4] = 1;
-}
-
 template <class Real, int TX, int TY, bool GRAD>
 struct StepTile {
   static constexpr bool PAIR = sizeof(Real) == 8;
@@ -431,11 +420,10 @@ __global__ void __launch_bounds__(step_nw(sizeof(Real) == 8, TX, TY) * 64, 2)
   // the top row of y-faces or the right column of x-faces, waves 0 and 1 one
   // unit each, which evens the SIMDs out (wave w runs on SIMD w % 4, so two
   // SIMDs hold two interior waves and two hold one).
-  constexpr int kHalo = T::NW - T::NWI;  // waves of halo columns
   constexpr int kMore = T::NWI >= 6 ? 2 : 1;
-  constexpr int kGive = kHalo >= 2 ? 2 * kMore : kMore;  // y units the halo waves take
-  static_assert(kHalo >= 1 && kGive <= T::NWI, "halo waves");
-  const bool top_wave = wave == T::NW - (kHalo >= 2 ? 2 : 1), right_wave = wave == T::NW - 1;
+  constexpr int kGive = 2 * kMore;  // y units the halo waves take
+  static_assert(T::NW - T::NWI == 2 && kGive <= T::NWI, "two waves of halo columns");
+  const bool top_wave = wave == T::NW - 2, right_wave = wave == T::NW - 1;
   const int ya = top_wave ? T::NWI - kMore : (right_wave ? T::NWI - 2 * kMore : (wave < T::NWI - kGive ? wave : 0));
   const int yb = top_wave ? T::NWI : (right_wave ? T::NWI - kMore : (wave < T::NWI - kGive ? wave + 1 : 0));
   const bool do_x = right_wave ? lane < th : interior;
@@ -695,7 +683,7 @@ __global__ void __launch_bounds__(step_nw(sizeof(Real) == 8, TX, TY) * 64, 2)
         sum[0] += __hip_atomic_load(&law.partial[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       block_reduce<1, T::NT>(sum, kSum);
       if (t == 0) {
-        flow_law(law.famb, as, sum[0] / law.volume, law.target, law.gain, law.dt);
+        flow_update(law.famb, as, sum[0] / law.volume, law.target, law.gain, law.dt);
         *law.arrived = 0;  // for the next launch
       }
     }
