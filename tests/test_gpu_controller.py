@@ -47,7 +47,19 @@ def test_force_follows_from_the_state(rng, precision, n, walls, axis, kernel):
     terms and a reciprocal: U to 2e-14 of the largest velocity (FP32 sums: about
     1e-8 a cell, 3e-12 and more of the mean over up to 1e7 terms); FP16 storage
     may move U by its rounding on top."""
-    kw = {f"periods_{walls}": 0, f"mesh_{walls}": "tanh:0.85", "dt_rule": "min"}
+    _force_follows(rng, precision, n, axis, kernel,
+                   {f"periods_{walls}": 0, f"mesh_{walls}": "tanh:0.85", "dt_rule": "min"})
+
+
+@pytest.mark.parametrize("n", [(16, 12, 1), (256, 300, 1), (45, 29, 11), (64, 64, 32), (41, 21, 44)], ids=str)
+@pytest.mark.parametrize("precision", [PREC_FP64, PREC_FP32, PREC_FP16S, PREC_FP16N],
+                         ids=["fp64", "fp32", "fp16", "fp16n"])
+def test_force_follows_from_the_state_with_gradient_reconstruction(rng, precision, n):
+    """The same on the gradient step's tiles and on one plane."""
+    _force_follows(rng, precision, n, 0, KERNEL_AUTO, {"periods_y": 0, "recon": "grad"})
+
+
+def _force_follows(rng, precision, n, axis, kernel, kw):
     text = configs.base(nx=n[0], ny=n[1], nz=n[2], xwidth=n[0] / 10, ywidth=n[1] / 10, zwidth=n[2] / 10, visc=0.02,
                         CFL=0.5, ambient_fx=2e-4, ambient_fz=1e-4, flow_rate=TARGET, flow_axis=axis, **kw)
     eng = _engine(text, precision=precision, kernel=kernel)
