@@ -389,8 +389,11 @@ struct LaneFace {
 // A position holds its slots side by side, STRIDE values apart from the next,
 // so that 16-byte accesses move four FP32 or two FP64 values and one address
 // register with immediate offsets reaches every neighbour.  STRIDE is an odd
-// number of 16-byte units: the eight lanes of one LDS pass then use each bank
-// once.  The order keeps the five slots with one sign of c_x or c_y, which
+// number of 16-byte units: the eight lanes of a 16-byte pass then start on
+// different banks.  (Conflicts remain, 1.1 cycles an LDS instruction in FP32 and
+// 2.9 in FP64; candidates are the groups that end in a single value, read 4 or 8
+// bytes wide at this stride, and the two halves that share a pass in FP64.)  The
+// order keeps the five slots with one sign of c_x or c_y, which
 // the reconstruction reads from an upwind neighbour, within two 16-byte
 // units (FP32: one unit and one value of the next).
 template <bool PAIR>

@@ -30,7 +30,8 @@
 // Other configurations use the two-pass kernels.
 //
 // What bounds it.  The step moves 38 values per cell (f in, f out; halos come
-// from L2) and does about 2300 operations per cell.  On 256x192x256 with one
+// from L2) and issues about 1450 VALU lane-instructions per cell in FP32 and 2360
+// in FP64.  On 256x192x256 with one
 // MI355X (a large copy runs at 4.9 TB/s) the traffic alone takes 0.39 ms in
 // FP32 and 0.78 ms in FP64, the arithmetic with the memory accesses taken out
 // 0.55 and 1.13 ms: the kernel is bound by issue.  Two waves per SIMD fit, so
@@ -617,7 +618,8 @@ int z_chunk(const Ctx& cx, int TX, int TY) {
 // A plane takes the same time whatever the grid, and the start of a tile or
 // chunk about 2.2 planes' time (f-bar+ of two planes and one face).  So a
 // round of 256 workgroups costs the planes of the longest one + 2.2, and the
-// plan is the cheapest of:
+// plan is the cheapest of these (times are those of a run of steps over their
+// number; event pairs around a launch read about 2.5 us more):
 //  - z-chunks of every tile (plan_z_chunks).  64x64x32 FP64 (24 tiles): 8
 //    chunks 30.5 us, 16 36.6, 32 39.4; 64x72x32 FP32 (12 tiles): 8 chunks
 //    28.0 us, 16 20.3, 32 24.3;
