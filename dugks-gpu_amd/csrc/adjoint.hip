@@ -350,16 +350,19 @@ __global__ void __launch_bounds__(256) k_adj_cells(KParams P, const Store* __res
 // with the state stored in the arithmetic type it reads them from the face pass
 // (16 or 32 bytes a cell) rather than the 19 values of f.
 //
-// What bounds it: HBM.  A cell reads lam' (19 values), three face records (4
-// each, in one 16-byte access with FP32) and rho, j, and writes lam; the records
-// held the ten crossing values as well (13 each) before, so that the two passes
-// moved 174 values a cell, now 120.  The next plane's loads go out during the
+// What bounds it: issue in FP32 (two waves per SIMD, VALU 61 % busy, 1795
+// lane-instructions a cell; 3.4 GB of HBM traffic on 256x192x256 at 3.7 TB/s, where
+// a large copy runs at 4.9) and latency in FP64 (a column's registers leave one
+// wave per SIMD, VALU 30 % busy).  A cell reads lam' (19 values), three face
+// records (4 each, in one 16-byte access with FP32) and rho, j, and writes lam; the
+// records held the ten crossing values as well (13 each) before, so that the two
+// passes moved 174 values a cell, now 120.  The next plane's loads go out during the
 // gather, a plane ahead of their use, without branches (accesses that are not
 // wanted go out of range), so that every wait counts exactly.  Ring lanes run
 // the gather and the centre stage on clamped positions and store nothing: they
-// share SIMDs with one wave of cells where the others hold two.
-// 256x192x256 FP32: 0.98 ms, before 1.23; the face pass 1.09, before 1.41 (0.86
-// since).
+// share SIMDs with one wave of cells where the others hold two.  The FP64 form
+// without FLOW and the 8-row FP16 form with FP64 lam spill two and seven registers.
+// 256x192x256 FP32: 0.94 ms, before 1.23 (the face pass beside it 0.84, before 1.41).
 // lanes of a workgroup, and LDS positions (the last ones idle)
 constexpr int gather_lanes(bool fp64, int rows) { return ((rows + 2) * (fp64 ? 18 : 34) + 63) / 64 * 64; }
 template <class Real, int ROWS>
