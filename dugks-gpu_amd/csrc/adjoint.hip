@@ -379,10 +379,14 @@ struct GatherTile {
 // controller): lam' still lacks the bulk velocity's cotangent ubar (dV/V)
 // (c_ia - u_a)/rho of f(n+1), whose rho, j the previous pass left in the
 // other region; it is added as lam' is used.
-// FLAT: the grid has one plane, so planes p-1, p and p+1 are the same and the
-// first one taken completes it.  (FP32 with FP64 lam, us an adjoint step: 512x768x1
-// 98, with the same plane taken three times 144; 64x64x1 18 and 29.)
-template <class Real, class Store, class Lam, int ROWS, bool FLOW, bool FLAT>
+// PLANES 1 or 2: the grid has that many planes, in one chunk, and each is taken
+// once: on one plane p-1, p and p+1 are the same, on two p-1 and p+1 are, so that
+// what a plane gives to either goes to the other one.  (PLANES 0 takes the two
+// planes beside a chunk too.  FP32 with FP64 lam, us an adjoint step: 512x768x1 98,
+// with the same plane taken three times 144; 64x64x1 18 and 29.  FP64, 192x288x2
+// with walls 90 and 105, 512x256x2 143 and 158.  With FP32 arithmetic the two-plane
+// form spills 34 to 96 registers and was slower, 100 and 89 us on 512x256x2.)
+template <class Real, class Store, class Lam, int ROWS, bool FLOW, int PLANES>
 __global__ void __launch_bounds__(gather_lanes(sizeof(Real) == 8, ROWS), sizeof(Real) == 4 ? 2 : 1)
     k_adj_cells_z(KParams P, const Store* __restrict__ fin, const Lam* __restrict__ lam,
                   const Real* __restrict__ faces, Lam* __restrict__ lam_prev, double* __restrict__ grad, int nchunk,
@@ -600,7 +604,7 @@ __global__ void __launch_bounds__(gather_lanes(sizeof(Real) == 8, ROWS), sizeof(
   load_lam(I0{}, IQ{}, wrap(z0 - 1), true);
   load_recs(wrap(z0 - 1), true);
 
-  for (int p = FLAT ? z0 : z0 - 1; p <= (FLAT ? z0 : zend); p++) {
+  for (int p = PLANES == 1 ? z0 : z0 - 1; p <= (PLANES == 1 ? z0 : zend); p++) {
     const int pos = here(pos0), Rg = here(Rg0), Cg = here(Cg0);  // (addresses formed anew each plane)
     // lam'(p), complete
     static_for<Q>([&](auto I) {
@@ -617,8 +621,16 @@ __global__ void __launch_bounds__(gather_lanes(sizeof(Real) == 8, ROWS), sizeof(
         lamC[ip] += fma_rn(Real(CX[ip]) * ax + Real(CY[ip]) * ay + Real(CZ[ip]) * az, sc, t0);
       });
     }
-    if constexpr (FLAT)
+    if constexpr (PLANES == 1)
       for (int ip = 0; ip < Q; ip++) lamP[ip] = lamC[ip];
+    // two planes: p = -1 gives lam' only, p = 2 takes plane 1 through the centre stage only
+    if (PLANES == 2 && p < z0) {
+      load_lam(I0{}, IQ{}, z0, true);
+      load_recs(z0, true);
+      continue;
+    }
+    const bool faces = PLANES != 2 || p < zend;
+    if (faces) {
     __syncthreads();  // the previous plane's gather is done with S
     static_for<Q>([&](auto I) {
       constexpr int ip = decltype(I)::value;
@@ -647,10 +659,12 @@ __global__ void __launch_bounds__(gather_lanes(sizeof(Real) == 8, ROWS), sizeof(
       });
       expand(std::integral_constant<int, 2>{}, pos, mu, p >= z0, false, false);
     }
+    }
     // The centre stage's inputs of plane p-1 first, then, in groups, what the
     // next plane needs
-    const bool centre = stored && (FLAT || p - 1 >= z0), more = !FLAT && p < zend;
-    const unsigned cell = centre ? (FLAT ? 0u : (unsigned)(p - 1) * plane) + column : 0u;
+    const bool centre = stored && (PLANES == 1 || p - 1 >= z0);
+    const bool more = PLANES == 0 ? p < zend : (PLANES == 2 && p + 1 < zend);
+    const unsigned cell = centre ? (PLANES == 1 ? 0u : (unsigned)(p - 1) * plane) + column : 0u;
     const unsigned v8 = centre ? cell * 8u : kOutOfRange;
     Real m4[4] = {Real(1), Real(0), Real(0), Real(0)};
     RawCell<Real, Store> fraw;
@@ -661,6 +675,7 @@ __global__ void __launch_bounds__(gather_lanes(sizeof(Real) == 8, ROWS), sizeof(
       fraw.load(bin, cell, (unsigned)P.N);
     for (int a = 0; a < 3; a++) fc[a] = fcb.ld<double>(v8, a * vec_pop);
     for (int a = 0; a < 3; a++) g0[a] = gradb.ld<double>(v8, a * vec_pop);
+    if (faces) {
     __syncthreads();
     // transposed reconstruction: a position's in-plane lerps through the
     // transposed z-lerps
@@ -719,8 +734,16 @@ __global__ void __launch_bounds__(gather_lanes(sizeof(Real) == 8, ROWS), sizeof(
         push(I, gq * hzr, gq * hz);
       });
     }
-    if constexpr (FLAT)
+    if constexpr (PLANES == 1)
       for (int ip = 0; ip < Q; ip++) accP[ip] += accC[ip] + accN[ip];
+    if constexpr (PLANES == 2) {
+      const bool low = p == z0;  // plane -1 is plane 1, plane 2 plane 0
+      for (int ip = 0; ip < Q; ip++) {
+        const Real v = accP[ip] + accN[ip];
+        if (low) accN[ip] = v; else accP[ip] = v;
+      }
+    }
+    }
     // centre-stage adjoint of plane p-1 (as k_adj_cells)
     Real rho = m4[0], j[3] = {m4[1], m4[2], m4[3]};
     if constexpr (!kMoments) {
@@ -796,11 +819,11 @@ GatherPlan gather_plan(const Setup& s, bool fp64) {
 
 namespace {
 
-template <class Real, class Store, class Lam, int ROWS, bool FLOW, bool FLAT>
+template <class Real, class Store, class Lam, int ROWS, bool FLOW, int PLANES>
 void launch_gather(const Ctx& cx, const GatherPlan& g, const void* f, const Lam* lam_next, Lam* lam_prev,
                    double* grad, int mom, const double* ubar) {
   const double inv_vol = 1.0 / (cx.s.width[0] * cx.s.width[1] * cx.s.width[2]);
-  hipLaunchKernelGGL((k_adj_cells_z<Real, Store, Lam, ROWS, FLOW, FLAT>), dim3((unsigned)g.nblocks),
+  hipLaunchKernelGGL((k_adj_cells_z<Real, Store, Lam, ROWS, FLOW, PLANES>), dim3((unsigned)g.nblocks),
                      dim3(GatherTile<Real, ROWS>::NT), 0, cx.stream, cx.kp, static_cast<const Store*>(f), lam_next,
                      static_cast<const Real*>(cx.adj_faces), lam_prev, grad, g.nchunk, mom, FLOW ? ubar : nullptr,
                      inv_vol);
@@ -809,15 +832,17 @@ template <class Real, class Store, class Lam, bool FLOW>
 void launch_gather(const Ctx& cx, const void* f, const Lam* lam_next, Lam* lam_prev, double* grad, int mom,
                    const double* ubar) {
   const GatherPlan g = gather_plan(cx.s, sizeof(Real) == 8);
-  const bool flat = cx.s.n[2] == 1;
-  if (g.rows == 12 && flat)
-    launch_gather<Real, Store, Lam, 12, FLOW, true>(cx, g, f, lam_next, lam_prev, grad, mom, ubar);
-  else if (g.rows == 12)
-    launch_gather<Real, Store, Lam, 12, FLOW, false>(cx, g, f, lam_next, lam_prev, grad, mom, ubar);
-  else if (flat)
-    launch_gather<Real, Store, Lam, 8, FLOW, true>(cx, g, f, lam_next, lam_prev, grad, mom, ubar);
-  else
-    launch_gather<Real, Store, Lam, 8, FLOW, false>(cx, g, f, lam_next, lam_prev, grad, mom, ubar);
+  const bool tall = g.rows == 12;
+  if (cx.s.n[2] == 1)
+    return tall ? launch_gather<Real, Store, Lam, 12, FLOW, 1>(cx, g, f, lam_next, lam_prev, grad, mom, ubar)
+                : launch_gather<Real, Store, Lam, 8, FLOW, 1>(cx, g, f, lam_next, lam_prev, grad, mom, ubar);
+  if constexpr (sizeof(Real) == 8) {
+    if (cx.s.n[2] == 2 && g.nchunk == 1)
+      return tall ? launch_gather<Real, Store, Lam, 12, FLOW, 2>(cx, g, f, lam_next, lam_prev, grad, mom, ubar)
+                  : launch_gather<Real, Store, Lam, 8, FLOW, 2>(cx, g, f, lam_next, lam_prev, grad, mom, ubar);
+  }
+  return tall ? launch_gather<Real, Store, Lam, 12, FLOW, 0>(cx, g, f, lam_next, lam_prev, grad, mom, ubar)
+              : launch_gather<Real, Store, Lam, 8, FLOW, 0>(cx, g, f, lam_next, lam_prev, grad, mom, ubar);
 }
 
 // One adjoint step.  Lam = double: every configuration; Lam = float (FP32

@@ -25,11 +25,11 @@ STEP_GRIDS = {form: {"fp64": _fp64[form], "fp32": _fp32[form], "fp16": _fp32[for
               for form in _fp32}
 
 # 12 rows: 96 rows of cells leave no overlap, the other grids do; grids of one
-# plane (their own form) among them
+# plane, and in FP64 of two in one chunk (forms of their own), among them
 GATHER_GRIDS = {
-    12: {"fp64": [(32, 40, 26), (64, 80, 64), (96, 96, 30), (512, 200, 1)],
+    12: {"fp64": [(32, 40, 26), (64, 80, 64), (96, 96, 30), (512, 200, 1), (512, 200, 2), (256, 192, 2)],
          "fp32": [(32, 32, 65), (64, 80, 64), (128, 40, 128), (96, 96, 64), (512, 400, 1)],
          "fp16": [(32, 32, 65), (96, 96, 64), (512, 400, 1)]},
-    8: {"fp64": [(64, 64, 32), (32, 8, 1), (96, 40, 1)], "fp32": [(64, 64, 32), (32, 8, 1), (96, 40, 1)],
+    8: {"fp64": [(64, 64, 32), (32, 8, 1), (96, 40, 1), (256, 200, 2)], "fp32": [(64, 64, 32), (32, 8, 1), (96, 40, 1)],
         "fp16": [(64, 64, 32), (32, 8, 1), (96, 40, 1)]},
 }

@@ -109,6 +109,29 @@ def test_controller_sweep_over_gather_forms(rng, n):
         assert abs(fd - an) <= 1e-7 * abs(an), (trial, fd, an)
 
 
+@pytest.mark.parametrize("n,images", [((32, 16, 1), 3), ((96, 40, 1), 4), ((256, 200, 2), 2), ((512, 200, 2), 2)],
+                         ids=str)
+def test_controller_sweep_on_periodic_images(rng, n, images):
+    """One and two planes in forms of their own against the general one: a state that
+    repeats along z has the same J per cell, so with `images` copies J and dJ/dF^0
+    are the same and the gradient in a cell is the 1/images part.  Eight FP64 steps
+    of 1e-13, forward and back, and sums of 1e5 terms: 1e-11."""
+    got = []
+    f0 = G = None
+    for m in (1, images):
+        text = configs.adjoint_channel(nx=n[0], ny=n[1], nz=n[2] * m, zwidth=0.13 * n[2] * m, xwidth=0.13 * n[0],
+                                       flow_rate=0.06, flow_axis=0)
+        eng = _stream_engine(text, precision=PREC_FP64)
+        if m == 1:
+            f0 = eng.get_f() * (1 + 1e-3 * rng.standard_normal(eng.fshape))
+            G = 1e-6 * rng.standard_normal((3,) + eng.fshape[:3])
+        got.append(_flow_grad(eng, np.tile(f0, (m, 1, 1, 1)), eng.ambient_force(), np.tile(G, (1, m, 1, 1)), 8))
+    (Ja, ga, da), (Jb, gb, db) = got
+    assert abs(Ja - Jb) <= 1e-11 * abs(Ja)
+    assert abs(da - db) <= 1e-11 * abs(da)
+    assert np.abs(np.tile(ga, (1, images, 1, 1)) - images * gb).max() <= 1e-11 * np.abs(ga).max()
+
+
 @pytest.mark.parametrize("n", [GATHER_GRIDS[12]["fp32"][0], (32, 16, 1)], ids=["rows12", "one_plane"])
 @pytest.mark.parametrize("mode,tol", [("fp32", 1e-5), ("fp16", 2e-4)])
 def test_reduced_precision_controller_sweep_over_gather_forms(mode, tol, n):
